@@ -89,8 +89,11 @@ int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h,
  *   absorb left  (flags bit0 = 1, keep_left_canonical=False):
  *       a_out = U[:, :k] S[:k],  b_out = V^H[:k, :]
  * The caller computes k = min(d*chi_l, d*chi_r, maxsvals) (core.py:1110-1130).
- * The SVD is a blocked one-sided Jacobi on the side that is not scaled by S,
- * so the scaled side never divides by a singular value. theta is formed in
+ * The SVD works on the side that is not scaled by S, so the scaled side never
+ * divides by a singular value: a blocked one-sided Jacobi on theta's rows up
+ * to 64 of them, above that the eigenvectors of the rows' Gram matrix, by a
+ * direct solver (tridiagonal form, divide and conquer) up to 1024 rows and
+ * by Jacobi rounds beyond. theta is formed in
  * complex FP32; by default the rotations are stored and applied in complex
  * FP64 (FP64 matrix cores), which keeps each truncated update as accurate
  * as a complex64 LAPACK SVD. With rotation_fp32 set they run in FP32
@@ -143,6 +146,8 @@ typedef struct {
     mpsx_plan plan;    /* library-owned, see mpsx_two_site_plan          */
 } mpsx_two_site_op;
 
+/* max_sweeps, check_every, inner_sweeps, tol and unconverged concern the
+ * problems that iterate; the direct solver does not. */
 typedef struct {
     int32_t block;      /* Jacobi block width b (pivot is 2b x 2b); 0 = auto  */
     int32_t max_sweeps; /* outer sweep limit; 0 = default (30)              */
@@ -172,7 +177,9 @@ typedef struct {
                            (max_sweeps bounds those). 0 (default) or < 0:
                            FP64 rounds only. The results agree with the FP64
                            rounds' to FP64 rounding of the converged rows. */
-    int32_t precondition;/* Householder QR before the FP64 Gram method (no
+    int32_t precondition;/* Householder QR before the FP64 Gram method's Jacobi
+                           rounds (a problem of the direct solver takes none;
+                           no
                            counterpart in the reference, whose SVD is
                            LAPACK's): X P = Q R with the columns ordered by
                            decreasing norm, then the same Jacobi on

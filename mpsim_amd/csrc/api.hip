@@ -181,6 +181,20 @@ int plan_method(const Resolved &r, int b, int nb) {
     return r.fp32_sweeps > 0 ? 2 : 1;
 }
 
+// Rows up to which the Gram problems of a call take the direct eigensolver.
+// Its largest group of workgroups has to be resident as a whole beside those
+// of up to three other streams, so a device (or partition) of fewer compute
+// units takes smaller problems only. k_eig_* launch problems as grid y.
+int direct_max(int count) {
+    int dev = 0, cus = 0;
+    if (count > 65535 || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    int n = EIG_MAX_N;
+    while (n > 128 && 4 * eig_group(n) > cus) n /= 2;
+    return 4 * eig_group(n) <= cus ? n : 0;
+}
+
 int *poll_buffer() {
     thread_local int *buf = nullptr;
     if (!buf) {
@@ -377,7 +391,7 @@ int mpsx_two_site_plan(mpsx_two_site_op *h, int count, const mpsx_svd_opts *opts
     if (count > 0 && !h) return fail(MPSX_EINVAL, "null descriptor table");
     const Resolved r = resolve(opts);
     if (int e = check_options(r)) return e;
-    int64_t off = kHeaderBytes, tiles = 0, pairs = 0, rows = 0, outs = 0;
+    int64_t off = kHeaderBytes, tiles = 0, pairs = 0, rows = 0, outs = 0, groups = 0;
     for (int i = 0; i < count; ++i) {
         mpsx_two_site_op &o = h[i];
         mpsx_plan p;
@@ -389,6 +403,7 @@ int mpsx_two_site_plan(mpsx_two_site_op *h, int count, const mpsx_svd_opts *opts
         p.out_base = outs;
         o.plan = p;
         off += problem_bytes(p);
+        if (eig_direct(p, EIG_MAX_N)) groups += eig_group(p.C);
         tiles += theta_tiles(o);
         pairs += p.nb / 2;
         rows += p.Cp;
@@ -396,8 +411,9 @@ int mpsx_two_site_plan(mpsx_two_site_op *h, int count, const mpsx_svd_opts *opts
     }
     if (tiles > kGridLimit || pairs > kGridLimit || rows > kGridLimit || outs > kGridLimit)
         return fail(MPSX_EINVAL, "batch too large for one launch");
-    // round workgroup -> problem table after the problems
-    off = align_up(off, 256) + align_up(4 * pairs, 256);
+    // round workgroup -> problem table after the problems, then the direct
+    // solver's workgroup table
+    off = align_up(off, 256) + align_up(4 * pairs, 256) + align_up(8 * groups, 256);
     if (bytes) *bytes = (size_t)off;
     g_err.clear();
     return MPSX_OK;
@@ -424,10 +440,16 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     // the table's plan: a table that was not planned, was planned for other
     // options, or was edited after planning is rejected.
     int64_t need = kHeaderBytes, tiles = 0, pairs = 0, rows = 0, outs = 0;
-    int rows_nb = 0, gram_nb = 0, gram_y = 0, gram_c = 0;
+    int rows_nb = 0, gram_nb = 0, round_nb = 0, gram_y = 0, gram_c = 0;
     bool has_d[THETA_GEN_DMAX + 1] = {};  // index 1: plain splits
     bool has_b[17] = {false};  // one-sided problems by block width
     bool has_gram = false, has_mixed = false;
+    bool has_rounds = false;  // some Gram problem runs Jacobi rounds
+    int max_n = -1;          // rows up to which the direct solver is taken, once a Gram problem asks
+    int64_t groups = 0;      // the direct solver's workgroup table (as planned)
+    int64_t eig_slots = 0;   // workgroups the direct solver launches
+    int eig_n = 0;           // its largest problem
+    bool eig_small = false, eig_large = false;
     int qr_c = 0, qr_r = 0, qr_rc = 0, qr_np = 0;  // QR-preconditioned problems: max C, R, R + C, panels
     bool qr_small = false, qr_large = false;  // some of at most 512 rows, some above
     for (int i = 0; i < count; ++i) {
@@ -457,11 +479,21 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         if (p.nb > 0 && p.method >= 1) {
             has_gram = true;
             has_mixed = has_mixed || p.method == 2;
-            gram_nb = std::max(gram_nb, p.nb);
-            gram_y = std::max(gram_y, p.nb / 4 + (p.Cp + 63) / 64);
+            if (max_n < 0) max_n = direct_max(count);
+            gram_nb = std::max(gram_nb, eig_direct(p, max_n) ? p.Cp / 16 : p.nb);
             gram_c = std::max(gram_c, (p.R + 31) / 32);
+            if (eig_direct(p, EIG_MAX_N)) groups += eig_group(p.C);
+            if (eig_direct(p, max_n)) {
+                eig_slots += eig_group(p.C);
+                eig_n = std::max(eig_n, (int)p.C);
+                (p.C <= 512 ? eig_small : eig_large) = true;
+            } else {
+                has_rounds = true;
+                round_nb = std::max(round_nb, p.nb);
+                gram_y = std::max(gram_y, p.nb / 4 + (p.Cp + 63) / 64);
+            }
         }
-        if (p.nb > 0 && p.method == 3) {
+        if (p.nb > 0 && p.method == 3 && !eig_direct(p, max_n)) {
             qr_c = std::max(qr_c, (int)p.C);
             qr_r = std::max(qr_r, (int)p.R);
             qr_rc = std::max(qr_rc, (int)(p.R + p.C));
@@ -469,10 +501,12 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
             (p.C <= 512 ? qr_small : qr_large) = true;
         }
     }
+    max_n = std::max(max_n, 0);
     if (tiles > kGridLimit || pairs > kGridLimit || rows > kGridLimit || outs > kGridLimit)
         return fail(MPSX_EINVAL, "batch too large for one launch");
     const int64_t owner_off = align_up(need, 256);
-    need = owner_off + align_up(4 * pairs, 256);
+    const int64_t map_off = owner_off + align_up(4 * pairs, 256);
+    need = map_off + align_up(8 * groups, 256);
     if (need_out) *need_out = (size_t)need;
     if ((int64_t)ws_bytes < need)
         return fail(MPSX_EWORKSPACE, "workspace %zu bytes < %lld needed", ws_bytes, (long long)need);
@@ -483,7 +517,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     const bool can_poll = may_poll && r.check_every > 0 && cap == hipStreamCaptureStatusNone;
 
     const bool f32 = r.fp32;
-    if (rows > 0) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows); }), "k_init_rows");
+    if (rows > 0) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n); }), "k_init_rows");
     for (int D = 1; D <= 4; ++D)
         if (has_d[D] && tiles > 0) HIP_TRY(timed("k_theta", stream, [&] { return launch_theta(stream, f32, D, d, count, ws, tiles); }), "k_theta");
     bool has_gen = false;
@@ -495,8 +529,8 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     }
     if (qr_c > 0) {
         // [X P | I] -> [R | Q^H] for the preconditioned problems, X0 saved
-        HIP_TRY(timed("k_qr_order", stream, [&] { return launch_qr_order(stream, d, count, ws, qr_c, qr_r); }), "k_qr_order");
-        HIP_TRY(timed("k_qr_permute", stream, [&] { return launch_qr_permute(stream, d, count, ws, rows); }),
+        HIP_TRY(timed("k_qr_order", stream, [&] { return launch_qr_order(stream, d, count, ws, qr_c, qr_r, max_n); }), "k_qr_order");
+        HIP_TRY(timed("k_qr_permute", stream, [&] { return launch_qr_permute(stream, d, count, ws, rows, max_n); }),
                 "k_qr_permute");
         for (int panel = -1; panel < qr_np; ++panel) {
             const int strips = panel < 0 ? 1 : (qr_rc - 16 * (panel + 1) + 15) / 16;
@@ -504,7 +538,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
                 HIP_TRY(timed("k_qr_step", stream,
                               [&] {
                                   return launch_qr_step(stream, d, count, ws, panel, strips, qr_c, qr_small,
-                                                        qr_large);
+                                                        qr_large, max_n);
                               }),
                         "k_qr_step");
         }
@@ -515,10 +549,22 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     if (pairs > 0)
         HIP_TRY(timed("k_owner", stream, [&] { return launch_owner(stream, d, count, owner); }), "k_owner");
     if (has_gram)
-        HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 0); }), "k_hgram");
+        HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 0, max_n); }), "k_hgram");
+    if (eig_slots > 0) {
+        HIP_TRY(timed("k_tridiag", stream,
+                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots); }),
+                "k_tridiag");
+        HIP_TRY(timed("k_eig_conquer", stream,
+                      [&] { return launch_eig_conquer(stream, d, count, ws, max_n, eig_n); }),
+                "k_eig_conquer");
+        HIP_TRY(timed("k_eig_back", stream,
+                      [&] { return launch_eig_back(stream, d, count, ws, max_n, eig_n, eig_small, eig_large); }),
+                "k_eig_back");
+    }
     // sweeps of both phases so far: indexes the header's active counters
     int sweep_idx = 0;
-    int *pin = (pairs > 0 && can_poll) ? poll_buffer() : nullptr;
+    const bool iterate = rows_nb > 0 || has_rounds;
+    int *pin = (iterate && can_poll) ? poll_buffer() : nullptr;
     auto poll_done = [&](int idx, bool *done) -> int {
         const TwoSiteHeader *hdr = reinterpret_cast<const TwoSiteHeader *>(ws);
         HIP_TRY(hipMemcpyAsync(pin, &hdr->active[idx & 63], sizeof(int), hipMemcpyDeviceToHost, stream),
@@ -536,19 +582,19 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         for (int s = 0; s < r.fp32_sweeps; ++s) {
             HIP_TRY(timed("k_hsolve32", stream,
                           [&] {
-                              return launch_hsolve(stream, true, d, owner, ws, pairs, 0, kGramTol32, ti,
+                              return launch_hsolve(stream, true, d, owner, ws, max_n, pairs, 0, kGramTol32, ti,
                                                    r.inner_sweeps, kGramAbsRel32);
                           }),
                     "k_hsolve32");
-            for (int round = 0; round < gram_nb - 2; ++round)
+            for (int round = 0; round < round_nb - 2; ++round)
                 HIP_TRY(timed("k_hround32", stream,
                               [&] {
-                                  return launch_hround(stream, true, d, owner, ws, pairs, gram_y, round,
+                                  return launch_hround(stream, true, d, owner, ws, max_n, pairs, gram_y, round,
                                                        kGramTol32, ti, r.inner_sweeps, kGramAbsRel32);
                               }),
                         "k_hround32");
             HIP_TRY(timed("k_hupdate32", stream,
-                          [&] { return launch_hupdate(stream, true, d, owner, ws, pairs, gram_y, gram_nb - 2, 0); }),
+                          [&] { return launch_hupdate(stream, true, d, owner, ws, max_n, pairs, gram_y, round_nb - 2, 0); }),
                     "k_hupdate32");
             HIP_TRY(timed("k_sweep_end", stream, [&] { return launch_sweep_end(stream, d, count, ws, sweep_idx, true); }), "k_sweep_end");
             ++sweep_idx;
@@ -558,10 +604,10 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
                 if (done) break;
             }
         }
-        HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 1, gram_nb); }), "k_hxgemm");
-        HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 1); }), "k_hgram");
+        HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 1, gram_nb, max_n); }), "k_hxgemm");
+        HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 1, max_n); }), "k_hgram");
     }
-    if (pairs > 0) {
+    if (iterate) {
         for (int s = 0; s < r.max_sweeps; ++s) {
             for (int round = 0; round < rows_nb - 1; ++round)
                 for (int b : {8, 16})
@@ -578,25 +624,25 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
             //   k_hsolve(0); then for r < R-1: k_hround(eigensolves of r+1,
             //   each after the tile holding its cross block, beside the rest
             //   of round r's update); finally k_hupdate(R-1, whole).
-            if (has_gram) {
+            if (has_rounds) {
                 const double ti = r.tol * 0.01;
                 HIP_TRY(timed("k_hsolve", stream,
                               [&] {
-                                  return launch_hsolve(stream, false, d, owner, ws, pairs, 0, r.tol, ti,
+                                  return launch_hsolve(stream, false, d, owner, ws, max_n, pairs, 0, r.tol, ti,
                                                        r.inner_sweeps, kGramAbsRel);
                               }),
                         "k_hsolve");
-                for (int round = 0; round < gram_nb - 2; ++round) {
+                for (int round = 0; round < round_nb - 2; ++round) {
                     HIP_TRY(timed("k_hround", stream,
                                   [&] {
-                                      return launch_hround(stream, false, d, owner, ws, pairs, gram_y, round, r.tol,
+                                      return launch_hround(stream, false, d, owner, ws, max_n, pairs, gram_y, round, r.tol,
                                                            ti, r.inner_sweeps, kGramAbsRel);
                                   }),
                             "k_hround");
                 }
                 HIP_TRY(timed("k_hupdate", stream,
                               [&] {
-                                  return launch_hupdate(stream, false, d, owner, ws, pairs, gram_y, gram_nb - 2, 0);
+                                  return launch_hupdate(stream, false, d, owner, ws, max_n, pairs, gram_y, round_nb - 2, 0);
                               }),
                         "k_hupdate");
             }
@@ -617,8 +663,8 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     }
 
     if (has_gram) {
-        HIP_TRY(timed("k_hxcopy", stream, [&] { return launch_hxcopy(stream, d, count, ws, rows); }), "k_hxcopy");
-        HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 0, gram_nb); }), "k_hxgemm");
+        HIP_TRY(timed("k_hxcopy", stream, [&] { return launch_hxcopy(stream, d, count, ws, rows, max_n); }), "k_hxcopy");
+        HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 0, gram_nb, max_n); }), "k_hxgemm");
     }
     if (rows > 0) {
         HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows); }), "k_rownorm");

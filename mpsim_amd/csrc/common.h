@@ -99,7 +99,8 @@ MPSX_DEV int find_record(const char *table, int count, size_t stride, size_t fie
 // Workspace header of a two-site batch (at ws + 0).
 struct TwoSiteHeader {
     int32_t active[64];  // active[s]: problems still unconverged after sweep s
-    int32_t pad[64];
+    int32_t ticket;      // workgroups of k_tridiag started so far
+    int32_t pad[63];
 };
 
 // Per-problem control block inside the workspace.
@@ -161,6 +162,25 @@ MPSX_HD int64_t qorder_off(const mpsx_plan &p) { return qt_off(p) + QR_RING * 16
 // Householder reflectors of the QR: one per column of X up to the last row.
 MPSX_HD int qr_reflectors(const mpsx_plan &p) { return p.C - 1 < p.R ? p.C - 1 : p.R; }
 MPSX_HD int qr_panels(const mpsx_plan &p) { return (qr_reflectors(p) + 15) / 16; }
+// Problems of the Gram method whose eigenvectors come from the direct solver
+// (csrc/eig.hip) instead of the Jacobi rounds: FP64 throughout (methods 1 and
+// 3; the mixed method 2 asks for its FP32 phase) and at most max_n rows (0:
+// none). The direct solver takes all C rows and no QR before it: on the
+// rank-deficient H of a tall problem it stops at the rank.
+constexpr int EIG_MAX_N = 1024;
+MPSX_HD bool eig_direct(const mpsx_plan &p, int max_n) {
+    return (p.method == 1 || p.method == 3) && p.C <= max_n;
+}
+// Workgroups that hold one problem's matrix in registers: 2, 4, 8 or 16
+// 64-column chunks a row leave room for 128, 64, 32 or 16 rows a workgroup.
+MPSX_HD int eig_class(int n) { return n <= 128 ? 0 : n <= 256 ? 1 : n <= 512 ? 2 : 3; }
+MPSX_HD int eig_group(int n) {
+    const int rows = 128 >> eig_class(n);
+    return (n + rows - 1) / rows;
+}
+// The value of an exchange slot that is not written yet (a NaN no arithmetic
+// produces, see k_tridiag).
+constexpr unsigned long long EIG_EMPTY = 0x7ff4dead5eedbeefULL;
 MPSX_HD int64_t problem_bytes(const mpsx_plan &p) {
     if (p.method == 0) return align_up(z_off(p) - p.ws_off + (int64_t)p.zbytes * p.Cp * p.LD, 256);
     if (p.method == 1) return align_up(qflag_off(p) - p.ws_off + 2 * 4LL * (p.nb / 2), 256);

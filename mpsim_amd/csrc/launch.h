@@ -16,8 +16,10 @@ bool gemm_rows_fit(const mpsx_gemm_op &o);
 hipError_t launch_gemm_rows(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gemm_op *d,
                             int count);
 
+// max_n: rows up to which the Gram problems take the direct eigensolver
+// (eig_direct; 0: none do).
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows);
+                            int64_t rows, int max_n);
 hipError_t launch_theta(hipStream_t s, bool f32, int D, const mpsx_two_site_op *d, int count, char *ws,
                         int64_t tiles);
 hipError_t launch_theta_gen(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
@@ -37,24 +39,34 @@ hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char
 hipError_t launch_gather(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
                          int64_t outs);
 hipError_t launch_hgram(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
-                        int64_t pairs, int max_nb, int stage);
+                        int64_t pairs, int max_nb, int stage, int max_n);
 hipError_t launch_hsolve(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int round, double tol, double tol_inner, int inner_sweeps,
+                         int max_n, int64_t pairs, int round, double tol, double tol_inner, int inner_sweeps,
                          double abs_rel);
 hipError_t launch_hupdate(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                          int64_t pairs, int ytiles, int round, int part);
+                          int max_n, int64_t pairs, int ytiles, int round, int part);
 hipError_t launch_hround(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int ytiles, int round, double tol, double tol_inner,
+                         int max_n, int64_t pairs, int ytiles, int round, double tol, double tol_inner,
                          int inner_sweeps, double abs_rel);
-hipError_t launch_hxcopy(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int64_t rows);
+hipError_t launch_hxcopy(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int64_t rows,
+                         int max_n);
 hipError_t launch_hxgemm(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int ctiles, int mode, int max_nb);
+                         int64_t pairs, int ctiles, int mode, int max_nb, int max_n);
 // QR preconditioning (plan.method 3): column order, X0 save and permute,
 // and step `panel` (-1 factors panel 0) over `strips` 16-column strips, for
 // the problems of at most 512 rows (`small`) and those above (`large`).
 hipError_t launch_qr_order(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_c,
-                           int max_r);
+                           int max_r, int max_n);
 hipError_t launch_qr_permute(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                             int64_t rows);
+                             int64_t rows, int max_n);
 hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int panel,
-                          int strips, int max_c, bool small, bool large);
+                          int strips, int max_c, bool small, bool large, int max_n);
+// Direct eigensolver (eig.hip) of the problems eig_direct selects: the
+// tridiagonal form (`map`: room for `slots` int2, the workgroups of all their
+// groups), the eigensystem of T, and Y. n: the largest C among them; `small`,
+// `large`: some of at most 512 rows, some above.
+hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
+                              int slots);
+hipError_t launch_eig_conquer(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
+hipError_t launch_eig_back(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n,
+                           bool small, bool large);

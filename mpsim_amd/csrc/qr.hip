@@ -262,9 +262,9 @@ MPSX_DEV double *qnorm_ptr(char *ws, const mpsx_plan &p) {
 // into part[y][column] (FP64), so that many workgroups share the problem's
 // read of X. part lies in the V ring, unused until the first panel is
 // factored.
-__global__ void __launch_bounds__(QR_NORM_COLS) k_qr_colnorm(const mpsx_two_site_op *ops, char *ws) {
+__global__ void __launch_bounds__(QR_NORM_COLS) k_qr_colnorm(const mpsx_two_site_op *ops, char *ws, int max_n) {
     const mpsx_plan p = ops[blockIdx.x].plan;
-    if (p.method != 3) return;
+    if (p.method != 3 || eig_direct(p, max_n)) return;
     const int C = p.C, R = p.R;
     const int r0 = (int)blockIdx.y * QR_NORM_ROWS, c = (int)blockIdx.z * QR_NORM_COLS + (int)threadIdx.x;
     if (r0 >= C || c >= R) return;
@@ -283,10 +283,10 @@ __global__ void __launch_bounds__(QR_NORM_COLS) k_qr_colnorm(const mpsx_two_site
 // (the parts summed in row order), then the rank of each column under (norm
 // descending, index ascending); order[rank] = column. A NaN norm ranks
 // last, so the order is a permutation whatever the data.
-__global__ void __launch_bounds__(1024) k_qr_order(const mpsx_two_site_op *ops, char *ws) {
+__global__ void __launch_bounds__(1024) k_qr_order(const mpsx_two_site_op *ops, char *ws, int max_n) {
     __shared__ double nrm[QR_MAX_R];
     const mpsx_plan p = ops[blockIdx.x].plan;
-    if (p.method != 3) return;
+    if (p.method != 3 || eig_direct(p, max_n)) return;
     const int R = p.R, parts = (p.C + QR_NORM_ROWS - 1) / QR_NORM_ROWS;
     const int tid = threadIdx.x;
     const double *part = qnorm_ptr(ws, p);
@@ -312,12 +312,12 @@ __global__ void __launch_bounds__(1024) k_qr_order(const mpsx_two_site_op *ops, 
 
 // One workgroup per padded row: X0[row] <- X[row] (zero for padded rows),
 // then X[row][j] <- X0[row][order[j]].
-__global__ void __launch_bounds__(256) k_qr_permute(const mpsx_two_site_op *ops, int count, char *ws) {
+__global__ void __launch_bounds__(256) k_qr_permute(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
     __shared__ double2 xs[QR_MAX_R];
     const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
                                OP_FIELD(plan.row_base), blockIdx.x);
     const mpsx_plan p = ops[pi].plan;
-    if (p.method != 3) return;
+    if (p.method != 3 || eig_direct(p, max_n)) return;
     const int row = (int)(blockIdx.x - p.row_base);
     if (row >= p.Cp) return;
     const int R = p.R;
@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(256) k_qr_permute(const mpsx_two_site_op *ops,
 // registers a[i][r] = (row 16 (w + 8 i) + 4 r + lq, column l16) of lane
 // (l16, lq), the matrix-core output layout.
 template <int CH>
-__global__ void __launch_bounds__(512) k_qr_step(const mpsx_two_site_op *ops, char *ws, int panel) {
+__global__ void __launch_bounds__(512) k_qr_step(const mpsx_two_site_op *ops, char *ws, int panel, int max_n) {
     // The update phase's arrays and, for panels of at most 512 rows, the
     // factorisation's LDS copy of the strip share one buffer.
     constexpr int kUpd = 11 * 16 * 17;
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__(512) k_qr_step(const mpsx_two_site_op *ops, ch
     __shared__ double2 vcol[8][CH == 4 ? 1 : 16 * CH];  // 1024-row panels: v, per wave for its rows
 
     const mpsx_plan p = ops[blockIdx.x].plan;
-    if (p.method != 3) return;
+    if (p.method != 3 || eig_direct(p, max_n)) return;
     // each problem always runs the same variant (4 chunks up to 512 rows, 8
     // above), so its result does not depend on what else is in the batch
     if ((CH == 4) != (p.C <= 512)) return;
@@ -637,30 +637,30 @@ __global__ void __launch_bounds__(512) k_qr_step(const mpsx_two_site_op *ops, ch
 }
 
 hipError_t launch_qr_order(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_c,
-                           int max_r) {
+                           int max_r, int max_n) {
     if (max_c > QR_MAX_CP || max_r > QR_MAX_R) return hipErrorInvalidValue;
     const dim3 parts((unsigned)count, (unsigned)((max_c + QR_NORM_ROWS - 1) / QR_NORM_ROWS),
                      (unsigned)((max_r + QR_NORM_COLS - 1) / QR_NORM_COLS));
-    k_qr_colnorm<<<parts, QR_NORM_COLS, 0, s>>>(d, ws);
+    k_qr_colnorm<<<parts, QR_NORM_COLS, 0, s>>>(d, ws, max_n);
     if (hipError_t e = hipGetLastError()) return e;
-    k_qr_order<<<count, 1024, 0, s>>>(d, ws);
+    k_qr_order<<<count, 1024, 0, s>>>(d, ws, max_n);
     return hipGetLastError();
 }
 
 hipError_t launch_qr_permute(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                             int64_t rows) {
-    k_qr_permute<<<(unsigned)rows, 256, 0, s>>>(d, count, ws);
+                             int64_t rows, int max_n) {
+    k_qr_permute<<<(unsigned)rows, 256, 0, s>>>(d, count, ws, max_n);
     return hipGetLastError();
 }
 
 hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int panel,
-                          int strips, int max_c, bool small, bool large) {
+                          int strips, int max_c, bool small, bool large, int max_n) {
     if (max_c > QR_MAX_CP) return hipErrorInvalidValue;
     const dim3 grid((unsigned)count, (unsigned)strips);
     if (small) {
-        k_qr_step<4><<<grid, 512, 0, s>>>(d, ws, panel);
+        k_qr_step<4><<<grid, 512, 0, s>>>(d, ws, panel, max_n);
         if (hipError_t e = hipGetLastError()) return e;
     }
-    if (large) k_qr_step<8><<<grid, 512, 0, s>>>(d, ws, panel);
+    if (large) k_qr_step<8><<<grid, 512, 0, s>>>(d, ws, panel, max_n);
     return hipGetLastError();
 }

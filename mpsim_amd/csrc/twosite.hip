@@ -70,10 +70,12 @@ MPSX_DEV double block_sum_256(double v, double *red) {
 // rows <- 0. Row 0 of each problem also resets its control block.
 template <class T>
 __global__ void __launch_bounds__(256)
-k_init_rows(const mpsx_two_site_op *ops, int count, char *ws) {
+k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
     using Z2 = typename Cx<T>::type;
-    if (blockIdx.x == 0 && threadIdx.x < 128)
-        reinterpret_cast<TwoSiteHeader *>(ws)->active[threadIdx.x & 63] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        reinterpret_cast<TwoSiteHeader *>(ws)->active[threadIdx.x] = 0;
+        if (threadIdx.x == 0) reinterpret_cast<TwoSiteHeader *>(ws)->ticket = 0;
+    }
     const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
                                OP_FIELD(plan.row_base), blockIdx.x);
     const mpsx_plan p = ops[pi].plan;
@@ -82,14 +84,22 @@ k_init_rows(const mpsx_two_site_op *ops, int count, char *ws) {
     Z2 *z = z_ptr<T>(ws, p) + (int64_t)row * p.LD;
     if (row >= p.C)
         for (int c = threadIdx.x; c < p.R; c += 256) z[c] = Cx<T>::make(0, 0);
-    for (int c = threadIdx.x; c < p.Cp; c += 256)
-        z[p.R + c] = Cx<T>::make(c == row ? 1 : 0, 0);
+    const bool direct = eig_direct(p, max_n);
+    if (!direct) {
+        for (int c = threadIdx.x; c < p.Cp; c += 256)
+            z[p.R + c] = Cx<T>::make(c == row ? 1 : 0, 0);
+    } else if (eig_group(p.C) > 1) {
+        // the direct solver writes Y itself; until then the rows are exchange
+        // slots, empty to begin with
+        unsigned long long *x = reinterpret_cast<unsigned long long *>(z + p.R);
+        for (int c = threadIdx.x; c < 2 * p.Cp; c += 256) x[c] = EIG_EMPTY;
+    }
     if (row == 0 && threadIdx.x == 0) {
         ProblemCtl *ctl = ctl_ptr(ws, p);
         ctl->fro2 = 0.0;
         ctl->null2 = 0.0;
         ctl->counter = 0;
-        ctl->conv = (p.C == 0 || p.R == 0) ? 1 : 0;
+        ctl->conv = (p.C == 0 || p.R == 0 || direct) ? 1 : 0;
         ctl->sweeps = 0;
     }
 }
@@ -979,15 +989,16 @@ MPSX_DEV double2 *t64_ptr(char *ws, const mpsx_plan &p) {
 // The copy of X (Cp x R, row stride R) that the end's X <- Y X reads: made
 // in the H region after the sweeps, or, QR-preconditioned, the X0 saved
 // before the QR.
-MPSX_DEV const double2 *xc_ptr(char *ws, const mpsx_plan &p) {
-    return p.method == 3 ? reinterpret_cast<const double2 *>(ws + qx0_off(p)) : h_ptr(ws, p);
+MPSX_DEV const double2 *xc_ptr(char *ws, const mpsx_plan &p, int max_n) {
+    return p.method == 3 && !eig_direct(p, max_n) ? reinterpret_cast<const double2 *>(ws + qx0_off(p)) : h_ptr(ws, p);
 }
 // Problems the Gram round kernels work on: in the FP32 phase (F32H) the
-// mixed ones (method 2), in the FP64 rounds every Gram problem (methods 1
-// and 2; a mixed problem there has passed its switch to FP64).
+// mixed ones (method 2), in the FP64 rounds every Gram problem that the
+// direct solver does not take (a mixed problem there has passed its switch to
+// FP64).
 template <bool F32H>
-MPSX_DEV bool gram_on(const mpsx_plan &p) {
-    return F32H ? p.method == 2 : p.method >= 1;
+MPSX_DEV bool gram_on(const mpsx_plan &p, int max_n) {
+    return F32H ? p.method == 2 : (p.method >= 1 && !eig_direct(p, max_n));
 }
 // Element access to H (Cp x Cp, row stride Cp) in the phase's precision;
 // values travel as double2 either way.
@@ -1029,8 +1040,11 @@ MPSX_DEV int rr_pivot(int item, int r, int n) {
 // The choice goes by the Jacobi's rows, 16 nb: for a tall QR-preconditioned
 // problem they are fewer than the working matrix's Cp rows, and the
 // launchers size their grids from nb too.
+// The direct solver works on all Cp rows (p.nb may count fewer blocks): its
+// tiles beyond the problem's nb / 2 slots are taken in further passes.
 constexpr int kTiledGemmRows = 512;
-MPSX_DEV bool tiled_gemm(const mpsx_plan &p) { return 16 * p.nb > kTiledGemmRows; }
+MPSX_DEV int gram_rows(const mpsx_plan &p, int max_n) { return eig_direct(p, max_n) ? p.Cp : 16 * p.nb; }
+MPSX_DEV bool tiled_gemm(const mpsx_plan &p, int max_n) { return gram_rows(p, max_n) > kTiledGemmRows; }
 
 // One workgroup per upper 16x16 block tile (bi <= bj) of H = X X^H. x: the
 // problem's pivot slot j (nb/2 per problem), y in [0, nb]; the tile is
@@ -1044,20 +1058,22 @@ MPSX_DEV bool tiled_gemm(const mpsx_plan &p) { return 16 * p.nb > kTiledGemmRows
 // the FP64 sweeps.
 template <int STAGE>
 __global__ void __launch_bounds__(256)
-k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws) {
+k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     __shared__ double2 part[4][16][17];
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if ((STAGE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p)) return;
+    if ((STAGE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p, max_n)) return;
     if (STAGE == 1 && blockIdx.x == p.pair_base && blockIdx.y == 0 && threadIdx.x == 0) {
         ProblemCtl *ctl = ctl_ptr(ws, p);
         ctl->conv = 0;
         ctl->counter = 0;
     }
-    const int nb = p.nb;
-    if ((int)blockIdx.y > nb) return;
-    int rem = (int)(blockIdx.x - p.pair_base) * (nb + 1) + (int)blockIdx.y;
-    int bi = 0;
+    if ((int)blockIdx.y > p.nb) return;
+    const bool direct = eig_direct(p, max_n);
+    const int nb = gram_rows(p, max_n) / 16;
+    for (int tile = (int)(blockIdx.x - p.pair_base) * (p.nb + 1) + (int)blockIdx.y; tile < nb * (nb + 1) / 2;
+         tile += p.nb / 2 * (p.nb + 1)) {
+    int rem = tile, bi = 0;
     while (rem >= nb - bi) {
         rem -= nb - bi;
         ++bi;
@@ -1074,7 +1090,7 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws) {
     // in the tile's second operand and add exact zeros, so they are skipped
     // (the sums are bitwise those of the full loop).
     int cs = wave * 16;
-    if (STAGE == 0 && p.method == 3 && 16 * bj >= cs + 16) cs += 64 * ((16 * bj - 16 - cs) / 64 + 1);
+    if (STAGE == 0 && p.method == 3 && !direct && 16 * bj >= cs + 16) cs += 64 * ((16 * bj - 16 - cs) / 64 + 1);
     for (int c0 = cs; c0 < R; c0 += 64) {
         const int cq = c0 + 4 * lq;
         double2 va[4], vb[4];
@@ -1104,6 +1120,13 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws) {
         h_store<true>(ws, p, idx, v);
     else
         h_ptr(ws, p)[idx] = v;
+    if (direct && bi != bj) {  // the direct solver reads whole rows: the mirrored tile too
+        const double2 e = part[0][j][i], f = part[1][j][i], g = part[2][j][i], h = part[3][j][i];
+        h_ptr(ws, p)[(int64_t)(bj * 16 + i) * p.Cp + bi * 16 + j] =
+            make_double2((e.x + g.x) + (f.x + h.x), -((e.y + g.y) + (f.y + h.y)));
+    }
+    __syncthreads();  // part is read before the next tile
+    }
 }
 
 // Workgroup size of the eigensolve kernel (eight waves measured slower than
@@ -1177,13 +1200,13 @@ MPSX_DEV void hsolve_core(const mpsx_plan &p, char *ws, int round, int pair, int
 // 32x32 block of H (all loads in flight together with the convergence flag:
 // the addresses are valid either way) and solves it.
 template <bool F32H>
-MPSX_DEV void hsolve_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int round,
+MPSX_DEV void hsolve_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round,
                           double tol, double tol_inner, int inner_sweeps, double abs_rel,
                           double2 (*H)[33], double2 (*Q)[33], double *prm_c, double2 *prm_s,
                           int &s_any) {
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if (!gram_on<F32H>(p) || round >= p.nb - 1) return;
+    if (!gram_on<F32H>(p, max_n) || round >= p.nb - 1) return;
     const int pair = (int)(blockIdx.x - p.pair_base);
     int I, J;
     rr_pair(pair, round, p.nb, &I, &J);
@@ -1196,14 +1219,14 @@ MPSX_DEV void hsolve_body(const mpsx_two_site_op *ops, const int *owner, char *w
 
 template <bool F32H>
 __global__ void __launch_bounds__(HSOLVE_THREADS)
-k_hsolve(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, double tol,
+k_hsolve(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round, double tol,
          double tol_inner, int inner_sweeps, double abs_rel) {
     __shared__ double2 H[32][33];
     __shared__ double2 Q[32][33];
     __shared__ double prm_c[16];
     __shared__ double2 prm_s[16];
     __shared__ int s_any;
-    hsolve_body<F32H>(ops, owner, ws, round, tol, tol_inner, inner_sweeps, abs_rel, H, Q, prm_c, prm_s,
+    hsolve_body<F32H>(ops, owner, ws, max_n, round, tol, tol_inner, inner_sweeps, abs_rel, H, Q, prm_c, prm_s,
                       s_any);
 }
 
@@ -1434,12 +1457,12 @@ MPSX_DEV const HTile32 *htile_update32(const mpsx_plan &p, char *ws, int round, 
 // 64 (y - n/2) .. +63 of the Y rows of P, Y <- Q_P^H Y (FP64 MFMAs, wave w
 // owns 16 columns of all 32 rows).
 template <bool F32H>
-MPSX_DEV void hupdate_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int round,
+MPSX_DEV void hupdate_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round,
                            int part, int y, double2 (*Ts)[33], double2 (*Ws)[33]) {
     constexpr int b = 16;
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if (!gram_on<F32H>(p) || round >= p.nb - 1) return;
+    if (!gram_on<F32H>(p, max_n) || round >= p.nb - 1) return;
     const int n = p.nb / 2, nt = n / 2, nb = p.nb;
     const int P = (int)(blockIdx.x - p.pair_base);
     int I, J;
@@ -1503,10 +1526,10 @@ MPSX_DEV void hupdate_body(const mpsx_two_site_op *ops, const int *owner, char *
 
 template <bool F32H>
 __global__ void __launch_bounds__(256, 4)
-k_hupdate(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, int part) {
+k_hupdate(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round, int part) {
     __shared__ double2 Ts[32][33];
     __shared__ double2 Ws[32][33];
-    hupdate_body<F32H>(ops, owner, ws, round, part, (int)blockIdx.y, Ts, Ws);
+    hupdate_body<F32H>(ops, owner, ws, max_n, round, part, (int)blockIdx.y, Ts, Ws);
 }
 
 // The eigensolve of pivot Pn of round + 1, preceded by the round `round`
@@ -1523,13 +1546,13 @@ k_hupdate(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, in
 // orientation part 0 uses (P2 = P + d mod n, 1 <= d <= n/2), so that its
 // arithmetic does not depend on which launch updates it.
 template <bool F32H>
-MPSX_DEV void hnext_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, double tol,
+MPSX_DEV void hnext_body(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round, double tol,
                          double tol_inner, int inner_sweeps, double abs_rel, double2 (*A)[33],
                          double2 (*B)[33], double *prm_c, double2 *prm_s, int &s_any) {
     constexpr int B2 = 32, b = 16;
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if (!gram_on<F32H>(p) || round >= p.nb - 1) return;
+    if (!gram_on<F32H>(p, max_n) || round >= p.nb - 1) return;
     const int nb = p.nb, n = nb / 2, nt = n / 2;
     const int Pn = (int)(blockIdx.x - p.pair_base);
     int In, Jn;
@@ -1594,7 +1617,7 @@ MPSX_DEV void hnext_body(const mpsx_two_site_op *ops, const int *owner, char *ws
 // workgroups per CU that the LDS allows.
 template <bool F32H>
 __global__ void __launch_bounds__(256, 4)
-k_hround(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, double tol,
+k_hround(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n, int round, double tol,
          double tol_inner, int inner_sweeps, double abs_rel) {
     __shared__ double2 A[32][33];
     __shared__ double2 B[32][33];
@@ -1602,20 +1625,20 @@ k_hround(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, dou
     __shared__ double2 prm_s[16];
     __shared__ int s_any;
     if (blockIdx.y == 0)
-        hnext_body<F32H>(ops, owner, ws, round, tol, tol_inner, inner_sweeps, abs_rel, A, B, prm_c, prm_s,
+        hnext_body<F32H>(ops, owner, ws, max_n, round, tol, tol_inner, inner_sweeps, abs_rel, A, B, prm_c, prm_s,
                          s_any);
     else
-        hupdate_body<F32H>(ops, owner, ws, round, 2, (int)blockIdx.y - 1, A, B);
+        hupdate_body<F32H>(ops, owner, ws, max_n, round, 2, (int)blockIdx.y - 1, A, B);
 }
 
 // End of the Gram method, 1: copy X (Cp x R) into the H region (row stride
 // R), one workgroup per padded row.
 __global__ void __launch_bounds__(256)
-k_hxcopy(const mpsx_two_site_op *ops, int count, char *ws) {
+k_hxcopy(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
     const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
                                OP_FIELD(plan.row_base), blockIdx.x);
     const mpsx_plan p = ops[pi].plan;
-    if (p.method < 1 || p.method == 3) return;  // method 3 kept X in X0
+    if (p.method < 1 || (p.method == 3 && !eig_direct(p, max_n))) return;  // the QR kept X in X0
     const int row = (int)(blockIdx.x - p.row_base);
     if (row >= p.Cp) return;
     const double2 *z = z_ptr<double>(ws, p) + (int64_t)row * p.LD;
@@ -1631,24 +1654,25 @@ k_hxcopy(const mpsx_two_site_op *ops, int count, char *ws) {
 // problem to FP64: X1 = Y X into region T (row stride R); X stays.
 template <int MODE>
 __global__ void __launch_bounds__(256)
-k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
+k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if ((MODE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p)) return;
+    if ((MODE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p, max_n)) return;
     const int R = p.R, LD = p.LD, Cp = p.Cp;
     const int col0 = (int)blockIdx.y * 32;
     if (col0 >= R) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, lq = lane >> 4;
     const int tm = wave >> 1, tn = wave & 1;
-    const int row0 = (int)(blockIdx.x - p.pair_base) * 32 + 16 * tm;
     const int col = col0 + 16 * tn + l16;
     const bool ok = col < R;
     double2 *Z = z_ptr<double>(ws, p);
-    const double2 *Xc = MODE == 0 ? xc_ptr(ws, p) : Z;  // B = X[k][col]
+    const double2 *Xc = MODE == 0 ? xc_ptr(ws, p, max_n) : Z;  // B = X[k][col]
     const int ldx = MODE == 0 ? R : LD;
     double2 *Out = MODE == 0 ? Z : t64_ptr(ws, p);
     const int ldo = MODE == 0 ? LD : R;
+    const int rows = gram_rows(p, max_n);
+    for (int row0 = (int)(blockIdx.x - p.pair_base) * 32 + 16 * tm; row0 < rows; row0 += 16 * p.nb) {
     const double2 *yrow = Z + (int64_t)(row0 + l16) * LD + R;  // A = Y[row0 + l16][k]
     mfma_d4 a1 = {0.0, 0.0, 0.0, 0.0}, a2 = a1, a3 = a1;
     for (int k0 = 0; k0 < Cp; k0 += 16) {
@@ -1672,6 +1696,7 @@ k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
             Out[(int64_t)(row0 + 4 * r + lq) * ldo + col] =
                 make_double2(a1[r] - a2[r], a3[r] - a1[r] - a2[r]);
     }
+    }
 }
 
 // The Gram method's products, one 64x64 output tile per workgroup, FP64
@@ -1690,14 +1715,14 @@ k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
 //   MODE 3: the switch of a mixed problem: X1 = Y X into region T.
 template <int MODE>
 __global__ void __launch_bounds__(256)
-k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
+k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     constexpr int TM = 64, TK = 16;
     __shared__ double2 As[TM][TK + 1];  // A[i][k]
     __shared__ double2 Bs[TK][TM + 1];  // B[k][j]
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
     const bool mixed_only = MODE == 1 || MODE == 3;
-    if ((mixed_only ? p.method != 2 : p.method < 1) || !tiled_gemm(p)) return;
+    if ((mixed_only ? p.method != 2 : p.method < 1) || !tiled_gemm(p, max_n)) return;
     if (MODE == 1 && blockIdx.x == p.pair_base && blockIdx.y == 0 && threadIdx.x == 0) {
         ProblemCtl *ctl = ctl_ptr(ws, p);
         ctl->conv = 0;
@@ -1705,19 +1730,21 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
     }
     const bool gram = MODE <= 1;
     const int Cp = p.Cp, R = p.R, LD = p.LD;
-    const int i0 = (int)(blockIdx.x - p.pair_base) * TM, j0 = (int)blockIdx.y * TM;
+    const int j0 = (int)blockIdx.y * TM;
     const int ncols = gram ? Cp : R, K = gram ? R : Cp;
-    if (i0 >= Cp || j0 >= ncols || (gram && j0 < i0)) return;
+    if (j0 >= ncols) return;
     double2 *Z = z_ptr<double>(ws, p);
     // row-major sources: A rows (length K), and for the Gram the rows of X
     // that form B = X^H; for MODES 2, 3 B = X[k][j]
     const double2 *Asrc = gram ? (MODE == 0 ? Z : t64_ptr(ws, p)) : Z + R;
     const int lda = gram ? (MODE == 0 ? LD : R) : LD;
-    const double2 *Bsrc = gram ? Asrc : (MODE == 2 ? xc_ptr(ws, p) : Z);
+    const double2 *Bsrc = gram ? Asrc : (MODE == 2 ? xc_ptr(ws, p, max_n) : Z);
     const int ldb = gram ? lda : (MODE == 2 ? R : LD);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, lq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
+    for (int i0 = (int)(blockIdx.x - p.pair_base) * TM; i0 < Cp; i0 += TM * (p.nb / 2)) {
+    if (gram && j0 < i0) break;
     mfma_d4 acc[2][2][3];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -1787,12 +1814,14 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws) {
                         h_store<true>(ws, p, idx, v);
                     else
                         h_ptr(ws, p)[idx] = v;
+                    if (j0 > i0 && eig_direct(p, max_n)) h_ptr(ws, p)[(int64_t)j * Cp + i] = zconj(v);
                 } else if (MODE == 2) {
                     Z[(int64_t)i * LD + j] = v;
                 } else {
                     t64_ptr(ws, p)[(int64_t)i * R + j] = v;
                 }
             }
+    }
 }
 
 // Round workgroup -> problem table (one workgroup per problem), so that the
@@ -1923,15 +1952,15 @@ k_gather(const mpsx_two_site_op *ops, int count, char *ws) {
 // ---------------------------------------------------------------- launchers
 template <class T>
 static void launch_init_rows_t(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                               int64_t rows) {
-    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws);
+                               int64_t rows, int max_n) {
+    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n);
 }
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows) {
+                            int64_t rows, int max_n) {
     if (f32)
-        launch_init_rows_t<float>(s, d, count, ws, rows);
+        launch_init_rows_t<float>(s, d, count, ws, rows, max_n);
     else
-        launch_init_rows_t<double>(s, d, count, ws, rows);
+        launch_init_rows_t<double>(s, d, count, ws, rows, max_n);
     return hipGetLastError();
 }
 
@@ -2029,73 +2058,73 @@ hipError_t launch_gather(hipStream_t s, bool f32, const mpsx_two_site_op *d, int
 }
 
 hipError_t launch_hgram(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
-                        int64_t pairs, int max_nb, int stage) {
+                        int64_t pairs, int max_nb, int stage, int max_n) {
     const dim3 small((unsigned)pairs, (unsigned)(max_nb + 1));
     const bool large = 16 * max_nb > kTiledGemmRows;
     const dim3 tiled((unsigned)pairs, (unsigned)((16 * max_nb + 63) / 64));  // 64-column tiles of Cp
     if (stage == 0) {
-        hipLaunchKernelGGL(k_hgram<0>, small, dim3(256), 0, s, d, owner, ws);
-        if (large) hipLaunchKernelGGL(k_hgemm<0>, tiled, dim3(256), 0, s, d, owner, ws);
+        hipLaunchKernelGGL(k_hgram<0>, small, dim3(256), 0, s, d, owner, ws, max_n);
+        if (large) hipLaunchKernelGGL(k_hgemm<0>, tiled, dim3(256), 0, s, d, owner, ws, max_n);
     } else {
-        hipLaunchKernelGGL(k_hgram<1>, small, dim3(256), 0, s, d, owner, ws);
-        if (large) hipLaunchKernelGGL(k_hgemm<1>, tiled, dim3(256), 0, s, d, owner, ws);
+        hipLaunchKernelGGL(k_hgram<1>, small, dim3(256), 0, s, d, owner, ws, max_n);
+        if (large) hipLaunchKernelGGL(k_hgemm<1>, tiled, dim3(256), 0, s, d, owner, ws, max_n);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_hsolve(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int round, double tol, double tol_inner, int inner_sweeps,
+                         int max_n, int64_t pairs, int round, double tol, double tol_inner, int inner_sweeps,
                          double abs_rel) {
     const dim3 g((unsigned)pairs), blk(HSOLVE_THREADS);
     if (f32h)
-        hipLaunchKernelGGL(k_hsolve<true>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner, inner_sweeps,
+        hipLaunchKernelGGL(k_hsolve<true>, g, blk, 0, s, d, owner, ws, max_n, round, tol, tol_inner, inner_sweeps,
                            abs_rel);
     else
-        hipLaunchKernelGGL(k_hsolve<false>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner, inner_sweeps,
+        hipLaunchKernelGGL(k_hsolve<false>, g, blk, 0, s, d, owner, ws, max_n, round, tol, tol_inner, inner_sweeps,
                            abs_rel);
     return hipGetLastError();
 }
 
 hipError_t launch_hround(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int ytiles, int round, double tol, double tol_inner,
+                         int max_n, int64_t pairs, int ytiles, int round, double tol, double tol_inner,
                          int inner_sweeps, double abs_rel) {
     static_assert(HSOLVE_THREADS == 256, "k_hround runs both roles with one workgroup size");
     const dim3 g((unsigned)pairs, (unsigned)(ytiles + 1)), blk(256);
     if (f32h)
-        hipLaunchKernelGGL(k_hround<true>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner, inner_sweeps,
+        hipLaunchKernelGGL(k_hround<true>, g, blk, 0, s, d, owner, ws, max_n, round, tol, tol_inner, inner_sweeps,
                            abs_rel);
     else
-        hipLaunchKernelGGL(k_hround<false>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner, inner_sweeps,
+        hipLaunchKernelGGL(k_hround<false>, g, blk, 0, s, d, owner, ws, max_n, round, tol, tol_inner, inner_sweeps,
                            abs_rel);
     return hipGetLastError();
 }
 
 hipError_t launch_hupdate(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
-                          int64_t pairs, int ytiles, int round, int part) {
+                          int max_n, int64_t pairs, int ytiles, int round, int part) {
     const dim3 g((unsigned)pairs, (unsigned)ytiles), blk(256);
     if (f32h)
-        hipLaunchKernelGGL(k_hupdate<true>, g, blk, 0, s, d, owner, ws, round, part);
+        hipLaunchKernelGGL(k_hupdate<true>, g, blk, 0, s, d, owner, ws, max_n, round, part);
     else
-        hipLaunchKernelGGL(k_hupdate<false>, g, blk, 0, s, d, owner, ws, round, part);
+        hipLaunchKernelGGL(k_hupdate<false>, g, blk, 0, s, d, owner, ws, max_n, round, part);
     return hipGetLastError();
 }
 
-hipError_t launch_hxcopy(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int64_t rows) {
-    hipLaunchKernelGGL(k_hxcopy, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws);
+hipError_t launch_hxcopy(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int64_t rows, int max_n) {
+    hipLaunchKernelGGL(k_hxcopy, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n);
     return hipGetLastError();
 }
 
 hipError_t launch_hxgemm(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
-                         int64_t pairs, int ctiles, int mode, int max_nb) {
+                         int64_t pairs, int ctiles, int mode, int max_nb, int max_n) {
     // ctiles counts 32-column tiles of R; k_hgemm takes 64 columns per workgroup
     const dim3 small((unsigned)pairs, (unsigned)ctiles), tiled((unsigned)pairs, (unsigned)((ctiles + 1) / 2));
     const bool large = 16 * max_nb > kTiledGemmRows;
     if (mode == 0) {
-        hipLaunchKernelGGL(k_hxgemm<0>, small, dim3(256), 0, s, d, owner, ws);
-        if (large) hipLaunchKernelGGL(k_hgemm<2>, tiled, dim3(256), 0, s, d, owner, ws);
+        hipLaunchKernelGGL(k_hxgemm<0>, small, dim3(256), 0, s, d, owner, ws, max_n);
+        if (large) hipLaunchKernelGGL(k_hgemm<2>, tiled, dim3(256), 0, s, d, owner, ws, max_n);
     } else {
-        hipLaunchKernelGGL(k_hxgemm<1>, small, dim3(256), 0, s, d, owner, ws);
-        if (large) hipLaunchKernelGGL(k_hgemm<3>, tiled, dim3(256), 0, s, d, owner, ws);
+        hipLaunchKernelGGL(k_hxgemm<1>, small, dim3(256), 0, s, d, owner, ws, max_n);
+        if (large) hipLaunchKernelGGL(k_hgemm<3>, tiled, dim3(256), 0, s, d, owner, ws, max_n);
     }
     return hipGetLastError();
 }

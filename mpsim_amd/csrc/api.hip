@@ -182,8 +182,8 @@ int plan_method(const Resolved &r, int b, int nb) {
 }
 
 // Rows up to which the Gram problems of a call take the direct eigensolver.
-// Its largest group of workgroups has to be resident as a whole beside those
-// of up to three other streams, so a device (or partition) of fewer compute
+// Its largest group of workgroups has to be resident as a whole, also beside
+// those of a few other streams (or it is given up, see k_tridiag), so a device (or partition) of fewer compute
 // units takes smaller problems only. k_eig_* launch problems as grid y.
 int direct_max(int count) {
     int dev = 0, cus = 0;
@@ -445,6 +445,9 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     bool has_b[17] = {false};  // one-sided problems by block width
     bool has_gram = false, has_mixed = false;
     bool has_rounds = false;  // some Gram problem runs Jacobi rounds
+    // up to 64 rows: one workgroup, unless the one-sided rounds are asked for
+    const int small = !r.fp32 && r.method == MPSX_SVD_AUTO ? 1 : 0;
+    bool has_small = false, other = false;
     int max_n = -1;          // rows up to which the direct solver is taken, once a Gram problem asks
     int64_t groups = 0;      // the direct solver's workgroup table (as planned)
     int64_t eig_slots = 0;   // workgroups the direct solver launches
@@ -472,9 +475,14 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         rows += p.Cp;
         outs += gather_units((int64_t)o.d * o.chi_l, o.k);
         has_d[o.d] = true;
-        if (p.nb > 0 && p.method == 0) {
-            has_b[p.b] = true;
-            rows_nb = std::max(rows_nb, p.nb);
+        if (small_route(p, small)) {
+            has_small = true;
+        } else {
+            other = true;
+            if (p.nb > 0 && p.method == 0) {
+                has_b[p.b] = true;
+                rows_nb = std::max(rows_nb, p.nb);
+            }
         }
         if (p.nb > 0 && p.method >= 1) {
             has_gram = true;
@@ -517,15 +525,20 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     const bool can_poll = may_poll && r.check_every > 0 && cap == hipStreamCaptureStatusNone;
 
     const bool f32 = r.fp32;
-    if (rows > 0) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n); }), "k_init_rows");
+    const bool rest = rows > 0 && other;  // some problem takes the launch sequence below
+    if (rest) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n, small); }), "k_init_rows");
     for (int D = 1; D <= 4; ++D)
         if (has_d[D] && tiles > 0) HIP_TRY(timed("k_theta", stream, [&] { return launch_theta(stream, f32, D, d, count, ws, tiles); }), "k_theta");
     bool has_gen = false;
     for (int D = 5; D <= THETA_GEN_DMAX; ++D) has_gen = has_gen || has_d[D];
     if (has_gen && tiles > 0) HIP_TRY(timed("k_theta", stream, [&] { return launch_theta_gen(stream, f32, d, count, ws, tiles); }), "k_theta");
-    if (rows > 0) {
-        HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows); }), "k_rownorm");
-        HIP_TRY(timed("k_fro", stream, [&] { return launch_fro(stream, d, count, ws, r.null_rel); }), "k_fro");
+    if (has_small)
+        HIP_TRY(timed("k_small", stream,
+                      [&] { return launch_small(stream, d, count, ws, r.tol, r.null_rel, r.unconverged); }),
+                "k_small");
+    if (rest) {
+        HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows, small); }), "k_rownorm");
+        HIP_TRY(timed("k_fro", stream, [&] { return launch_fro(stream, d, count, ws, r.null_rel, small); }), "k_fro");
     }
     if (qr_c > 0) {
         // [X P | I] -> [R | Q^H] for the preconditioned problems, X0 saved
@@ -546,13 +559,13 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
 
     int sweeps = 0;
     bool converged = false;
-    if (pairs > 0)
+    if (pairs > 0 && (has_gram || rows_nb > 0))
         HIP_TRY(timed("k_owner", stream, [&] { return launch_owner(stream, d, count, owner); }), "k_owner");
     if (has_gram)
         HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 0, max_n); }), "k_hgram");
     if (eig_slots > 0) {
         HIP_TRY(timed("k_tridiag", stream,
-                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots); }),
+                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128); }),
                 "k_tridiag");
         HIP_TRY(timed("k_eig_conquer", stream,
                       [&] { return launch_eig_conquer(stream, d, count, ws, max_n, eig_n); }),
@@ -596,7 +609,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
             HIP_TRY(timed("k_hupdate32", stream,
                           [&] { return launch_hupdate(stream, true, d, owner, ws, max_n, pairs, gram_y, round_nb - 2, 0); }),
                     "k_hupdate32");
-            HIP_TRY(timed("k_sweep_end", stream, [&] { return launch_sweep_end(stream, d, count, ws, sweep_idx, true); }), "k_sweep_end");
+            HIP_TRY(timed("k_sweep_end", stream, [&] { return launch_sweep_end(stream, d, count, ws, sweep_idx, true, small); }), "k_sweep_end");
             ++sweep_idx;
             if (pin && ((s + 1) % r.check_every == 0 || s + 1 == r.fp32_sweeps)) {
                 bool done = false;
@@ -616,7 +629,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
                                              : (f32 ? "k_jacobi_round32<32>" : "k_jacobi_round64<32>"),
                                       stream,
                                       [&] {
-                                          return launch_jacobi_round(stream, f32, b, d, owner, ws, pairs, round,
+                                          return launch_jacobi_round(stream, f32, b, d, owner, ws, small, pairs, round,
                                                                      r.tol, r.tol * 0.01, r.inner_sweeps);
                                       }),
                                 "k_jacobi_round");
@@ -646,7 +659,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
                               }),
                         "k_hupdate");
             }
-            HIP_TRY(timed("k_sweep_end", stream, [&] { return launch_sweep_end(stream, d, count, ws, sweep_idx, false); }), "k_sweep_end");
+            HIP_TRY(timed("k_sweep_end", stream, [&] { return launch_sweep_end(stream, d, count, ws, sweep_idx, false, small); }), "k_sweep_end");
             ++sweep_idx;
             ++sweeps;
             if (pin && ((s + 1) % r.check_every == 0 || s + 1 == r.max_sweeps)) {
@@ -666,11 +679,11 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         HIP_TRY(timed("k_hxcopy", stream, [&] { return launch_hxcopy(stream, d, count, ws, rows, max_n); }), "k_hxcopy");
         HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 0, gram_nb, max_n); }), "k_hxgemm");
     }
-    if (rows > 0) {
-        HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows); }), "k_rownorm");
-        HIP_TRY(timed("k_sort", stream, [&] { return launch_sort(stream, d, count, ws, r.unconverged); }), "k_sort");
+    if (rest) {
+        HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows, small); }), "k_rownorm");
+        HIP_TRY(timed("k_sort", stream, [&] { return launch_sort(stream, d, count, ws, r.unconverged, small); }), "k_sort");
+        if (outs > 0) HIP_TRY(timed("k_gather", stream, [&] { return launch_gather(stream, f32, d, count, ws, outs, small); }), "k_gather");
     }
-    if (outs > 0) HIP_TRY(timed("k_gather", stream, [&] { return launch_gather(stream, f32, d, count, ws, outs); }), "k_gather");
     if (sweeps_out) *sweeps_out = sweeps;
     if (can_poll && !converged)
         return fail(MPSX_ENOTCONV, "Jacobi SVD not converged after %d sweeps", sweeps);

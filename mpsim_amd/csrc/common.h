@@ -110,7 +110,7 @@ struct ProblemCtl {
     int32_t counter;  // pivot pairs rotated in the current sweep
     int32_t conv;     // 1 once a full sweep rotated nothing
     int32_t sweeps;   // sweeps that did work
-    int32_t pad;
+    int32_t group;    // direct solver: workgroups of this problem's group that have started, or given up
 };
 
 // Byte layout of one problem's region starting at plan.ws_off:
@@ -171,6 +171,14 @@ constexpr int EIG_MAX_N = 1024;
 MPSX_HD bool eig_direct(const mpsx_plan &p, int max_n) {
     return (p.method == 1 || p.method == 3) && p.C <= max_n;
 }
+// Problems that the one-workgroup kernel (csrc/small.hip) takes after theta:
+// FP64, at most 64 rows (the matrices it keeps in LDS) of at most 512 columns
+// (a longer row is more than one workgroup should read). on: 0 when the call
+// asks for the one-sided rounds.
+constexpr int SMALL_MAX_R = 512;
+MPSX_HD bool small_route(const mpsx_plan &p, int on) {
+    return on && p.method == 0 && p.zbytes == 16 && p.nb > 0 && p.C <= 64 && p.R <= SMALL_MAX_R;
+}
 // Workgroups that hold one problem's matrix in registers: 2, 4, 8 or 16
 // 64-column chunks a row leave room for 128, 64, 32 or 16 rows a workgroup.
 MPSX_HD int eig_class(int n) { return n <= 128 ? 0 : n <= 256 ? 1 : n <= 512 ? 2 : 3; }
@@ -187,6 +195,9 @@ MPSX_HD int64_t problem_bytes(const mpsx_plan &p) {
     if (p.method == 3) return align_up(qorder_off(p) - p.ws_off + 4LL * p.R, 256);
     return align_up(t_off(p) - p.ws_off + 16 * h_elems(p), 256);
 }
+
+// Sort key: NaN below everything, so that ranks are a permutation.
+MPSX_DEV double sort_key(double x) { return x == x ? x : -__builtin_huge_val(); }
 
 // Complex element of the working matrix: float2 (FP32 rotations) or
 // double2 (FP64 rotations).

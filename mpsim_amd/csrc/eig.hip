@@ -9,13 +9,8 @@
 //                symmetric tridiagonal (Golub & Van Loan, 4th ed., 8.3.1,
 //                in the one-pass form: the rank-2 update of step j and the
 //                product A v of step j + 1 share one pass over A);
-//   T = S L S^T  divide and conquer (Cuppen 1981) with the deflation of
-//                Dongarra & Sorensen (1987), the secular roots by rational
-//                interpolation at the two neighbouring poles (Bunch, Nielsen
-//                & Sorensen 1978) inside a bracket, and the eigenvectors of
-//                every rank-one update from the weights recomputed from the
-//                roots (Gu & Eisenstat 1994), which keeps S orthogonal to
-//                FP64 rounding without extended precision;
+//   T = S L S^T  divide and conquer (eig_dc.h), merges above 64 rows spread
+//                over the GPU;
 //   Y = (Q S)^H  the reflectors applied in blocks of 16 (compact WY), on the
 //                FP64 matrix cores.
 //
@@ -35,13 +30,10 @@
 #include <cstddef>
 
 #include "common.h"
+#include "eig_dc.h"
 #include "launch.h"
 
 namespace {
-
-constexpr double kEps = 2.220446049250313e-16;
-// Deflation threshold for T scaled to unit norm.
-constexpr double kDeflate = 8.0 * kEps;
 
 // Small vectors of a problem in its rotation region.
 struct EigVec {
@@ -97,67 +89,11 @@ MPSX_DEV int eig_levels(int n) {
     return l;
 }
 
-template <int CTRL>
-MPSX_DEV double dpp_f64(double x) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-// Sum over groups of L consecutive lanes, the same in every lane of the
-// group (quad permutes, then the half-row and row mirrors).
-template <int L>
-MPSX_DEV double group_sum(double x) {
-    if (L >= 2) x += dpp_f64<0xB1>(x);
-    if (L >= 4) x += dpp_f64<0x4E>(x);
-    if (L >= 8) x += dpp_f64<0x141>(x);
-    if (L >= 16) x += dpp_f64<0x140>(x);
-    return x;
-}
-template <int L>
-MPSX_DEV double group_prod(double x) {
-    if (L >= 2) x *= dpp_f64<0xB1>(x);
-    if (L >= 4) x *= dpp_f64<0x4E>(x);
-    if (L >= 8) x *= dpp_f64<0x141>(x);
-    if (L >= 16) x *= dpp_f64<0x140>(x);
-    return x;
-}
-MPSX_DEV double wave_sum64(double x) {
-    x = group_sum<16>(x);
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    return x;
-}
-// a' = [a.lower, b.lower], b' = [a.upper, b.upper] halves of the wave, added:
-// the lower half then holds a's pairwise sums, the upper half b's.
-MPSX_DEV double fold32(double a, double b) {
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-// The same on rows of 16 lanes: even rows hold a's sums, odd rows b's.
-MPSX_DEV double fold16(double a, double b) {
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-// Wave sums of four complex values at once: lanes 16 q .. 16 q + 15 receive
-// the sum of x[q]. Folding two values into one register halves the work of
-// every level (12 exchanges of 64-bit values instead of 48).
-MPSX_DEV double2 wave_sum4(const double2 (&x)[4]) {
-    const double re = fold16(fold32(x[0].x, x[2].x), fold32(x[1].x, x[3].x));
-    const double im = fold16(fold32(x[0].y, x[2].y), fold32(x[1].y, x[3].y));
-    return make_double2(group_sum<16>(re), group_sum<16>(im));
-}
-MPSX_DEV double uniform_f64(double x) {
-    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
-                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
-}
-MPSX_DEV double2 uniform_z(double2 v) { return make_double2(uniform_f64(v.x), uniform_f64(v.y)); }
-
 // ------------------------------------------------------- tridiagonal form
 // A group of G workgroups (eig_group: 128, 64, 32 or 16 rows each) holds one
-// problem's whole trailing matrix in registers: wave g of the group's 8 G owns
-// the rows g, g + 8 G, ..., lane l the columns l, l + 64, .... Step j
+// problem's whole trailing matrix in registers: the rows in blocks of eight,
+// dealt out to the workgroups in turn, a row of a block a wave; lane l the
+// columns l, l + 64, .... Step j
 //   1. takes p = A v (of the previous reflector v) and column j of A, both
 //      as they were before the pending rank-2 update;
 //   2. w = tau p - (tau/2)(tau p)^H v) v; column j brought up to date; its
@@ -166,21 +102,25 @@ MPSX_DEV double2 uniform_z(double2 v) { return make_double2(uniform_f64(v.x), un
 // Step 2 is repeated by every workgroup of the group (n-vectors only), so
 // the only exchange between workgroups is p' and column j + 1: 2 (n - j)
 // complex values a step, published by the owner of each row and awaited by
-// all.
+// all. In a workgroup the vectors of up to 256 elements are the work of its
+// first four waves: a SIMD issues for one of them as fast as for two.
 //
 // The exchange carries no flags: every slot is used once, starts as a NaN
 // of one fixed bit pattern (EIG_EMPTY, written by k_init_rows) and is written
 // by one 64-bit store at device scope; a reader polls until the pattern is
-// gone (a published NaN is given other bits). Slots of step J: p_i and c_i
-// for i = J .. n-1. Steps J and n - J share two Y rows of Cp complex values.
+// gone (a published NaN is given other bits). Slots of step J: four arrays of n
+// - J doubles (p re, p im, c re, c im). Steps J and n - J share two Y rows.
 //
-// Workgroups take their place by a ticket in the order they start, so a
-// workgroup waits only for others that have the tickets next to its own:
-// all groups but the last started one are whole and run to their end
-// whatever else holds the GPU, and four launches at once leave fewer than
-// 4 (64 - 1) workgroups waiting on the 256 compute units. A wait that is not
-// served within kSpin polls (seconds) gives up for good and the problem's
-// results become NaN.
+// Workgroups take their place by a ticket in the order they start, and a
+// group starts its work only when all its workgroups have: from then on it
+// holds its compute units and waits for nothing but itself. Before that a
+// workgroup may hold a compute unit that a missing member needs (each XCD
+// is dealt a fixed share of a launch, and several launches, each with an
+// incomplete group, can fill one), so that wait has an end: after
+// kFormTicks, spread over the launches so that they do not all give up
+// at once, the group is given up for good, its workgroups leave, and
+// k_tridiag_one does the problem. The flag and the count are one word (ctl->group), so a
+// group is either whole or given up for all its members.
 //
 // The iteration stops where the trailing matrix is zero to working precision
 // (its trace, what the diagonal has left of tr H, is at most 64 eps tr H; H is
@@ -188,9 +128,33 @@ MPSX_DEV double2 uniform_z(double2 v) { return make_double2(uniform_f64(v.x), un
 // is after about r steps, whatever n. Tall theta and the zero singular
 // values that gates of low Schmidt rank leave make such H.
 //
-// Bound: the step's latency, an exchange (about 2 us) and four barriers;
-// the arithmetic of step 3 is under a microsecond.
-constexpr int kSpin = 1 << 21;
+// Bound: the step's latency: an exchange (about 2 us), three barriers, and
+// instruction issue; 4.6 us a step at n = 512, 4.1 at 128. The whole update
+// of 512 x 512 takes 3.6 ms, with the Jacobi rounds (300 launches of 37 us,
+// behind a QR of 1.6 ms) it took 13.2. k_tridiag_one: 28 ms at 512, 0.3 s at
+// 1024.
+constexpr int kSpin = 1 << 21;  // polls of a slot of a whole group (seconds): never reached
+constexpr long long kFormTicks = 4000000;  // 40 ms at 100 MHz
+constexpr int kGroupLost = 1 << 30;
+
+// Whether the group is whole; one thread of each of its workgroups asks.
+MPSX_DEV bool form_group(int *state, int G, int spread) {
+    if (G == 1) return true;
+    int s = __hip_atomic_fetch_add(state, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    const long long start = wall_clock64(), limit = kFormTicks * (1 + (spread & 3));
+    while (true) {
+        if (s & kGroupLost) return false;
+        if (s >= G) return true;
+        if (wall_clock64() - start > limit) {
+            if (__hip_atomic_compare_exchange_strong(state, &s, s | kGroupLost, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT))
+                return false;
+            continue;  // s is the newer value
+        }
+        __builtin_amdgcn_s_sleep(4);
+        s = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
 
 MPSX_DEV void publish(double *at, double v) {
     unsigned long long b = (unsigned long long)__double_as_longlong(v);
@@ -202,43 +166,56 @@ MPSX_DEV unsigned long long peek(const double *at) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// NX: rows a one-workgroup group may have.
+template <int NX>
 struct TriShared {
     double2 v[2][EIG_MAX_N];  // reflectors of the previous and this step
     double2 w[EIG_MAX_N];
-    double2 p[128], c[128];   // the exchange of a one-workgroup group
+    double2 p[NX], c[NX];     // the exchange of a one-workgroup group
     double2 red1[8];
     double red2[8];
     double2 xj, al;
     double dj;
-    int fail;
+    int fail, stop, whole;
     int slot;
 };
 
-// Slot of (step J, row i): four doubles (p re, p im, c re, c im).
-MPSX_DEV double *xslot(double *y, int64_t ld2, int Cp, int n, int J, int i) {
+// The slots of step J in the Y rows: doubles first .. of a stretch that starts in
+// row `row` and goes on in the next at Cp complex values.
+struct Slots {
+    double *y;
+    int64_t ld2;
+    int first, split, m;
+};
+MPSX_DEV Slots slots_of(double *y, int64_t ld2, int Cp, int n, int J) {
     const bool late = J > n - J;
     const int q = late ? n - J : J;
-    int pos = 2 * (i - J) + (late ? 2 * (n - q) : 0);
-    int row = 2 * q - 2;
-    if (pos >= Cp) {
-        pos -= Cp;
-        ++row;
-    }
-    return y + row * ld2 + 2 * pos;
+    Slots s;
+    s.y = y + (int64_t)(2 * q - 2) * ld2;
+    s.ld2 = ld2;
+    s.first = late ? 4 * (n - q) : 0;
+    s.split = 2 * Cp;
+    s.m = n - J;
+    return s;
+}
+MPSX_DEV double *slot_at(const Slots &s, int array, int i) {
+    const int pos = s.first + array * s.m + i;
+    return s.y + (pos >= s.split ? s.ld2 + (pos - s.split) : (int64_t)pos);
 }
 
-// Step 3 on NL live rows (the last of the four rows at r0): update, product
-// and the publication of column J.
-template <int CH, int RW, int NL, int NG>
-MPSX_DEV void tri_rows(double2 (&a)[RW][CH], int r0, const double2 *v, const double2 *w, const double2 *vn,
+// Step 3 on NL live rows (the last of the NG at r0), and the publication of
+// their entries of column J. MEM: the rows are in memory (A, row stride lda)
+// instead of registers.
+template <int CH, int RW, int NL, int NG, bool MEM, class SM>
+MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, const double2 *v, const double2 *w, const double2 *vn,
                        int lane, const int (&row)[4], double2 (&acc)[4], int t0, int J, int n, bool alone,
-                       TriShared &sm, double *y, int64_t ld2, int Cp) {
+                       SM &sm, const Slots &sl) {
     double2 vi[4], wi[4];
 #pragma unroll
     for (int q = NG - NL; q < NG; ++q) {
-        const int r = row[q] < n ? row[q] : n;  // entry n and above are zero
-        vi[q] = uniform_z(v[r < EIG_MAX_N ? r : 0]);
-        wi[q] = uniform_z(w[r < EIG_MAX_N ? r : 0]);
+        const int r = row[q] < n ? row[q] : 0;  // entry 0 is zero from the second step on, a row beyond n always
+        vi[q] = uniform_z(v[r]);
+        wi[q] = uniform_z(w[r]);
     }
     const int tc = J >> 6, lc = J & 63;
 #pragma unroll
@@ -248,231 +225,266 @@ MPSX_DEV void tri_rows(double2 (&a)[RW][CH], int r0, const double2 *v, const dou
         const double2 vk = v[k], wk = w[k], nk = vn[k];
 #pragma unroll
         for (int q = NG - NL; q < NG; ++q) {
-            double2 x = a[r0 + q][t];
+            double2 x;
+            if constexpr (MEM)
+                x = (row[q] < n && k < n) ? A[row[q] * lda + k] : make_double2(0.0, 0.0);
+            else
+                x = a[r0 + q][t];
             x.x = fma(-vi[q].x, wk.x, fma(-vi[q].y, wk.y, fma(-wi[q].x, vk.x, fma(-wi[q].y, vk.y, x.x))));
             x.y = fma(-vi[q].y, wk.x, fma(vi[q].x, wk.y, fma(-wi[q].y, vk.x, fma(wi[q].x, vk.y, x.y))));
             acc[q].x = fma(x.x, nk.x, fma(-x.y, nk.y, acc[q].x));
             acc[q].y = fma(x.x, nk.y, fma(x.y, nk.x, acc[q].y));
-            a[r0 + q][t] = x;
+            if constexpr (MEM) {
+                if (row[q] < n && k < n) A[row[q] * lda + k] = x;
+            } else {
+                a[r0 + q][t] = x;
+            }
         }
         if (t == tc && lane == lc) {
 #pragma unroll
             for (int q = NG - NL; q < NG; ++q) {
                 if (row[q] >= n) continue;
-                const double2 x = a[r0 + q][t];
+                double2 x;
+                if constexpr (MEM)
+                    x = A[row[q] * lda + k];
+                else
+                    x = a[r0 + q][t];
                 if (alone) {
                     sm.c[row[q]] = x;
                 } else {
-                    double *s = xslot(y, ld2, Cp, n, J, row[q]);
-                    publish(s + 2, x.x);
-                    publish(s + 3, x.y);
+                    publish(slot_at(sl, 2, row[q] - J), x.x);
+                    publish(slot_at(sl, 3, row[q] - J), x.y);
                 }
             }
         }
     }
 }
 
-template <int CH, int RW>
-MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, TriShared &sm) {
-    constexpr int EPT = CH > 8 ? 2 : 1;  // vector elements per thread
-    constexpr int NG = RW < 4 ? RW : 4;  // rows per reduction
+// MEM: one workgroup, the matrix copied to the Y rows (which hold no slots
+// then); every sum is formed in the same order as by a group.
+template <int CH, int RW, bool MEM, class SM>
+MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
+    constexpr int VW = CH > 4 ? 8 : 4;        // waves that hold the vectors
+    constexpr int EPT = CH > VW ? CH / VW : 1;  // vector elements per thread of theirs
+    constexpr int NG = RW < 4 ? RW : 4;       // rows per reduction
     const int n = p.C, Cp = p.Cp;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int gw = member * 8 + wave, NW = 8 * G;
-    const bool alone = G == 1;
+    const int tid = threadIdx.x;
+    int wave = tid >> 6;
+    const bool alone = G == 1, vec = VW == 8 || wave < VW;
     double2 *H = eig_h(ws, p);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
     const EigVec ev = eig_vec(ws, p);
 
-    double2 a[RW][CH];
+    double2 a[RW][CH], vown[EPT];
+    double2 *A = reinterpret_cast<double2 *>(y);
+    double rem;  // trace of the trailing matrix
+    {
+        const int lane = tid & 63;
+        if constexpr (MEM) {
+            for (int row = wave; row < n; row += 8)
+                for (int k = lane; k < n; k += 64) A[(int64_t)row * p.LD + k] = H[(int64_t)row * Cp + k];
+        } else {
 #pragma unroll
-    for (int r = 0; r < RW; ++r)
+            for (int r = 0; r < RW; ++r)
 #pragma unroll
-        for (int t = 0; t < CH; ++t) {
-            const int row = gw + NW * r, k = lane + 64 * t;
-            a[r][t] = (row < n && k < n) ? H[(int64_t)row * Cp + k] : make_double2(0.0, 0.0);
+                for (int t = 0; t < CH; ++t) {
+                    const int row = 8 * (member + G * r) + wave, k = lane + 64 * t;
+                    a[r][t] = (row < n && k < n) ? H[(int64_t)row * Cp + k] : make_double2(0.0, 0.0);
+                }
         }
-    double2 c0[EPT], vown[EPT];
 #pragma unroll
-    for (int s = 0; s < EPT; ++s) {
-        const int i = tid + 512 * s;
-        c0[s] = i < n ? H[(int64_t)i * Cp] : make_double2(0.0, 0.0);
-        vown[s] = make_double2(0.0, 0.0);
+        for (int s = 0; s < EPT; ++s) vown[s] = make_double2(0.0, 0.0);
+        for (int i = tid; i < EIG_MAX_N; i += 512) {
+            sm.v[0][i] = make_double2(0.0, 0.0);
+            sm.v[1][i] = make_double2(0.0, 0.0);
+            sm.w[i] = make_double2(0.0, 0.0);
+        }
+        rem = 0.0;
+        if (vec)
+            for (int i = lane; i < n; i += 64) rem += H[(int64_t)i * Cp + i].x;
+        rem = wave_sum64(rem);  // the same in each of these waves
     }
-    for (int i = tid; i < EIG_MAX_N; i += 512) {
-        sm.v[0][i] = make_double2(0.0, 0.0);
-        sm.v[1][i] = make_double2(0.0, 0.0);
-        sm.w[i] = make_double2(0.0, 0.0);
-    }
-    double trace = 0.0;
-    for (int i = lane; i < n; i += 64) trace += H[(int64_t)i * Cp + i].x;
-    double rem = wave_sum64(trace);  // trace of the trailing matrix; the same in every wave
     const double floor_tr = 64.0 * kEps * rem;
-    int nref = n - 1;
     if (tid == 0) {
         sm.fail = 0;
         sm.xj = make_double2(0.0, 0.0);
         sm.al = make_double2(0.0, 0.0);
+        sm.dj = 0.0;
     }
     __syncthreads();
     double2 tau = make_double2(0.0, 0.0);
-    int cur = 0;
+    int cur = 0, nref = n - 1;
     for (int j = 0; j < n; ++j) {
-        // ---- 1. p and column j
-        double2 x[EPT], c[EPT], dot = make_double2(0.0, 0.0);
-        const bool failed = sm.fail != 0;
+        // the lane and the wave through an empty asm statement: addresses are
+        // formed in the step rather than held (and spilled) across it
+        int lane = tid & 63;
+        asm volatile("" : "+v"(lane), "+v"(wave));
+        const int ti = 64 * wave + lane;  // this thread's first vector element
+        double2 x[EPT], c[EPT];
+        if (vec) {
+            // ---- 1. p and column j
+            double2 dot = make_double2(0.0, 0.0);
+            const bool failed = sm.fail != 0;
+            const Slots sl = slots_of(y, ld2, Cp, n, j);
 #pragma unroll
-        for (int s = 0; s < EPT; ++s) {
-            const int i = tid + 512 * s;
-            double2 pv = make_double2(0.0, 0.0);
-            c[s] = make_double2(0.0, 0.0);
-            if (i >= j && i < n) {
-                if (j == 0) {
-                    c[s] = c0[s];
-                } else if (alone) {
-                    pv = sm.p[i];
-                    c[s] = sm.c[i];
-                } else {
-                    const double *at = xslot(y, ld2, Cp, n, j, i);
-                    unsigned long long b0, b1, b2, b3;
-                    int spin = failed ? kSpin : 0;
-                    while (true) {
-                        b0 = peek(at);
-                        b1 = peek(at + 1);
-                        b2 = peek(at + 2);
-                        b3 = peek(at + 3);
-                        if (b0 != EIG_EMPTY && b1 != EIG_EMPTY && b2 != EIG_EMPTY && b3 != EIG_EMPTY) break;
-                        if (++spin > kSpin) {
-                            sm.fail = 1;
-                            break;
+            for (int s = 0; s < EPT; ++s) {
+                const int i = ti + 64 * VW * s;
+                double2 pv = make_double2(0.0, 0.0);
+                c[s] = make_double2(0.0, 0.0);
+                if (i >= j && i < n) {
+                    if (j == 0) {
+                        c[s] = H[(int64_t)i * Cp];
+                    } else if (alone) {
+                        pv = sm.p[i];
+                        c[s] = sm.c[i];
+                    } else {
+                        const double *a0 = slot_at(sl, 0, i - j), *a1 = slot_at(sl, 1, i - j),
+                                     *a2 = slot_at(sl, 2, i - j), *a3 = slot_at(sl, 3, i - j);
+                        unsigned long long b0, b1, b2, b3;
+                        int spin = failed ? kSpin : 0;
+                        while (true) {
+                            b0 = peek(a0);
+                            b1 = peek(a1);
+                            b2 = peek(a2);
+                            b3 = peek(a3);
+                            if (b0 != EIG_EMPTY && b1 != EIG_EMPTY && b2 != EIG_EMPTY && b3 != EIG_EMPTY) break;
+                            if (++spin > kSpin) {
+                                sm.fail = 1;
+                                break;
+                            }
                         }
+                        pv = make_double2(__longlong_as_double((long long)b0), __longlong_as_double((long long)b1));
+                        c[s] = make_double2(__longlong_as_double((long long)b2), __longlong_as_double((long long)b3));
                     }
-                    pv = make_double2(__longlong_as_double((long long)b0), __longlong_as_double((long long)b1));
-                    c[s] = make_double2(__longlong_as_double((long long)b2), __longlong_as_double((long long)b3));
                 }
+                x[s] = zmul(tau, pv);
+                // conj(x) v
+                dot.x = fma(x[s].x, vown[s].x, fma(x[s].y, vown[s].y, dot.x));
+                dot.y = fma(x[s].x, vown[s].y, fma(-x[s].y, vown[s].x, dot.y));
+                if (i == j) sm.xj = x[s];
             }
-            x[s] = zmul(tau, pv);
-            // conj(x) v
-            dot.x = fma(x[s].x, vown[s].x, fma(x[s].y, vown[s].y, dot.x));
-            dot.y = fma(x[s].x, vown[s].y, fma(-x[s].y, vown[s].x, dot.y));
-            if (i == j) sm.xj = x[s];
+            double f = fold32(dot.x, dot.y);  // the two halves of the wave
+            f = group_sum<16>(fold16(f, f));
+            if (lane == 0) sm.red1[wave].x = f;
+            if (lane == 32) sm.red1[wave].y = f;
+            if (ti == 0) sm.stop = rem <= floor_tr;
         }
-        dot = make_double2(wave_sum64(dot.x), wave_sum64(dot.y));
-        if (lane == 0) sm.red1[wave] = dot;
         __syncthreads();
-        // ---- 2. w, column j, its reflector
-        dot = make_double2(0.0, 0.0);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) dot = zadd(dot, sm.red1[u]);
-        const double2 alpha = zscale(zmul(tau, dot), -0.5);
-        const double2 wj = zadd(sm.xj, alpha);  // v_j = 1 for j > 0; zero otherwise
+        const bool stop = sm.stop != 0;
         double2 col[EPT];
-        double nrm = 0.0;
-        const bool writer = j > 0 && member == j % G;
-        const bool stop = rem <= floor_tr;
+        if (vec) {
+            // ---- 2. w, column j, its reflector
+            double2 dot = zadd(zadd(sm.red1[0], sm.red1[1]), zadd(sm.red1[2], sm.red1[3]));
+            if (VW == 8)
+                dot = zadd(dot, zadd(zadd(sm.red1[4], sm.red1[5]), zadd(sm.red1[6], sm.red1[7])));
+            const double2 alpha = zscale(zmul(tau, dot), -0.5);
+            const double2 wj = zadd(sm.xj, alpha);  // v_j = 1 for j > 0; zero otherwise
+            double nrm = 0.0;
+            const bool writer = j > 0 && member == j % G;
 #pragma unroll
-        for (int s = 0; s < EPT; ++s) {
-            const int i = tid + 512 * s;
-            const double2 v = vown[s];
-            const double2 w = zadd(x[s], zmul(alpha, v));
-            // c - v conj(w_j) - w conj(v_j), v_j = 1
-            col[s].x = c[s].x - (v.x * wj.x + v.y * wj.y) - (j > 0 ? w.x : 0.0);
-            col[s].y = c[s].y - (v.y * wj.x - v.x * wj.y) - (j > 0 ? w.y : 0.0);
-            if (i < EIG_MAX_N) sm.w[i] = (i > j && i < n) ? w : make_double2(0.0, 0.0);
-            if (i > j + 1 && i < n) nrm = fma(col[s].x, col[s].x, fma(col[s].y, col[s].y, nrm));
-            if (i == j + 1) sm.al = col[s];
-            if (i == j) sm.dj = col[s].x;
-            if (member == 0 && i == j && !stop) ev.d[j] = col[s].x;
-            // reflector j - 1 to its panel (every workgroup has read H by now)
-            if (writer && i < n && i >= ((j - 1) & ~15))
-                H[(int64_t)((j - 1) >> 4) * 16 * Cp + (int64_t)i * 16 + ((j - 1) & 15)] = v;
+            for (int s = 0; s < EPT; ++s) {
+                const int i = ti + 64 * VW * s;
+                const double2 v = vown[s];
+                const double2 w = zadd(x[s], zmul(alpha, v));
+                // c - v conj(w_j) - w conj(v_j), v_j = 1
+                col[s].x = c[s].x - (v.x * wj.x + v.y * wj.y) - (j > 0 ? w.x : 0.0);
+                col[s].y = c[s].y - (v.y * wj.x - v.x * wj.y) - (j > 0 ? w.y : 0.0);
+                sm.w[i] = (i > j && i < n) ? w : make_double2(0.0, 0.0);
+                if (i > j + 1 && i < n) nrm = fma(col[s].x, col[s].x, fma(col[s].y, col[s].y, nrm));
+                if (i == j + 1) sm.al = col[s];
+                if (i == j) sm.dj = col[s].x;
+                if (member == 0 && i == j && !stop) ev.d[j] = col[s].x;
+                // reflector j - 1 to its panel (every workgroup has read H by now)
+                if (writer && i < n && i >= ((j - 1) & ~15))
+                    H[(int64_t)((j - 1) >> 4) * 16 * Cp + (int64_t)i * 16 + ((j - 1) & 15)] = v;
+            }
+            nrm = wave_sum64(nrm);
+            if (lane == 0) sm.red2[wave] = nrm;
         }
-        if (stop) {
-            nref = j;
-            if (member == 0)
-                for (int i = j + tid; i < n; i += 512) {
-                    ev.d[i] = 0.0;
-                    ev.e[i] = 0.0;
-                }
-            break;
-        }
-        nrm = wave_sum64(nrm);
-        if (lane == 0) sm.red2[wave] = nrm;
         __syncthreads();
-        if (j == n - 1) break;
-        rem -= sm.dj;
-        nrm = ((sm.red2[0] + sm.red2[1]) + (sm.red2[2] + sm.red2[3])) +
-              ((sm.red2[4] + sm.red2[5]) + (sm.red2[6] + sm.red2[7]));
-        const double2 al = sm.al;
-        double beta = al.x;
-        double2 sc = make_double2(0.0, 0.0);
-        tau = make_double2(0.0, 0.0);
-        if (!(nrm == 0.0 && al.y == 0.0)) {
-            beta = -copysign(sqrt(fma(al.x, al.x, fma(al.y, al.y, nrm))), al.x);
-            const double ib = 1.0 / beta;
-            tau = make_double2((beta - al.x) * ib, -al.y * ib);
-            const double2 df = make_double2(al.x - beta, al.y);
-            const double id = 1.0 / fma(df.x, df.x, df.y * df.y);
-            sc = make_double2(df.x * id, -df.y * id);
-        }
-        if (member == 0 && tid == 0) {
-            ev.e[j] = beta;
-            ev.tau[j] = tau;
-        }
+        // one exit only: with two, the registers' array is kept twice
+        nref = stop ? j : n - 1;
+        if (stop || j == n - 1) break;
         double2 *vn = sm.v[cur ^ 1];
+        if (vec) {
+            rem -= sm.dj;
+            double nrm = (sm.red2[0] + sm.red2[1]) + (sm.red2[2] + sm.red2[3]);
+            if (VW == 8) nrm += (sm.red2[4] + sm.red2[5]) + (sm.red2[6] + sm.red2[7]);
+            const double2 al = sm.al;
+            double beta = al.x;
+            double2 sc = make_double2(0.0, 0.0);
+            tau = make_double2(0.0, 0.0);
+            if (!(fma(al.y, al.y, nrm) <= kTiny)) {
+                beta = -copysign(sqrt(fma(al.x, al.x, fma(al.y, al.y, nrm))), al.x);
+                const double ib = recip(beta);
+                tau = make_double2((beta - al.x) * ib, -al.y * ib);
+                const double2 df = make_double2(al.x - beta, al.y);
+                const double id = recip(fma(df.x, df.x, df.y * df.y));
+                sc = make_double2(df.x * id, -df.y * id);
+            }
+            if (member == 0 && ti == 0) {
+                ev.e[j] = beta;
+                ev.tau[j] = tau;
+            }
 #pragma unroll
-        for (int s = 0; s < EPT; ++s) {
-            const int i = tid + 512 * s;
-            vown[s] = i == j + 1 ? make_double2(1.0, 0.0)
-                                 : ((i > j + 1 && i < n) ? zmul(col[s], sc) : make_double2(0.0, 0.0));
-            if (i < EIG_MAX_N) vn[i] = vown[s];
+            for (int s = 0; s < EPT; ++s) {
+                const int i = ti + 64 * VW * s;
+                vown[s] = i == j + 1 ? make_double2(1.0, 0.0)
+                                     : ((i > j + 1 && i < n) ? zmul(col[s], sc) : make_double2(0.0, 0.0));
+                vn[i] = vown[s];
+            }
         }
         __syncthreads();
         // ---- 3. A -= v w^H + w v^H, p' = A v'; publish p' and column j + 1
         const double2 *v = sm.v[cur];
         const int J = j + 1, t0 = J >> 6;
-#pragma unroll
-        for (int g = 0; g < RW / NG; ++g) {
+        const Slots sl = slots_of(y, ld2, Cp, n, J);
+        auto rows = [&](int g) {
             int row[4] = {n, n, n, n};
 #pragma unroll
-            for (int q = 0; q < NG; ++q) row[q] = gw + NW * (g * NG + q);
+            for (int q = 0; q < NG; ++q) row[q] = 8 * (member + G * (g * NG + q)) + wave;
             double2 acc[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) acc[q] = make_double2(0.0, 0.0);
             int live = 0;  // rows of index >= J: the last ones
 #pragma unroll
             for (int q = 0; q < NG; ++q) live += row[q] >= J;
-            if (live == 0) continue;
+            if (live == 0) return;
             if (live == 1)
-                tri_rows<CH, RW, 1, NG>(a, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, y, ld2, Cp);
+                tri_rows<CH, RW, 1, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
             else if (live == 2)
-                tri_rows<CH, RW, 2, NG>(a, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, y, ld2, Cp);
+                tri_rows<CH, RW, 2, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
             else if (live == 3)
-                tri_rows<CH, RW, (NG < 3 ? NG : 3), NG>(a, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm,
-                                                        y, ld2, Cp);
+                tri_rows<CH, RW, (NG < 3 ? NG : 3), NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
             else
-                tri_rows<CH, RW, NG, NG>(a, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, y, ld2, Cp);
-            const double2 s = wave_sum4(acc);
-            const int q = lane >> 4;
-            int rq = row[0];
-            if (q == 1) rq = row[1];
-            if (q == 2) rq = row[2];
-            if (q == 3) rq = row[3];
-            if ((lane & 15) == 0 && q < NG && rq >= J && rq < n) {
-                if (alone) {
-                    sm.p[rq] = s;
-                } else {
-                    double *at = xslot(y, ld2, Cp, n, J, rq);
-                    publish(at, s.x);
-                    publish(at + 1, s.y);
-                }
+                tri_rows<CH, RW, NG, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
+            const double s = wave_sum4(acc);
+            const int q = lane >> 4, im = (lane >> 3) & 1;
+            const int rq = 8 * (member + G * (g * NG + q)) + wave;
+            if ((lane & 7) == 0 && q < NG && rq >= J && rq < n) {
+                if (alone)
+                    (im ? sm.p[rq].y : sm.p[rq].x) = s;
+                else
+                    publish(slot_at(sl, im, rq - J), s);
             }
+        };
+        if constexpr (MEM) {
+            for (int g = 0; g < (n + 8 * NG - 1) / (8 * NG); ++g) rows(g);
+        } else {
+#pragma unroll
+            for (int g = 0; g < RW / NG; ++g) rows(g);
         }
         cur ^= 1;
         if (alone) __syncthreads();
     }
-    if (member == 0 && tid == 0) *ev.nref = nref;
+    if (member != 0) return;
+    if (tid == 0) *ev.nref = nref;
+    if (nref < n - 1 || sm.stop)
+        for (int i = nref + tid; i < n; i += 512) {
+            ev.d[i] = 0.0;
+            ev.e[i] = 0.0;
+        }
 }
 
 }  // namespace
@@ -483,7 +495,7 @@ __global__ void __launch_bounds__(256)
 k_eig_map(const mpsx_two_site_op *ops, int count, int2 *map, int max_n) {
     __shared__ int wsum[4];
     __shared__ int total;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     if (tid == 0) total = 0;
     __syncthreads();
     for (int cls = 3; cls >= 0; --cls)
@@ -512,7 +524,7 @@ k_eig_map(const mpsx_two_site_op *ops, int count, int2 *map, int max_n) {
 
 __global__ void __launch_bounds__(512, 2)
 k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
-    __shared__ TriShared sm;
+    __shared__ TriShared<128> sm;
     if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
     __syncthreads();
     const int slot = sm.slot;
@@ -520,11 +532,32 @@ k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
     const int2 m = map[slot];
     const mpsx_plan p = ops[m.x].plan;
     const int member = m.y >> 8, G = m.y & 255;
+    if (threadIdx.x == 0)
+        sm.whole = form_group(&reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->group, G,
+                              (int)(reinterpret_cast<uintptr_t>(ws) >> 12));
+    __syncthreads();
+    if (!sm.whole) return;
     switch (eig_class(p.C)) {
-        case 0: tridiag<2, 16>(p, ws, member, G, sm); break;
-        case 1: tridiag<4, 8>(p, ws, member, G, sm); break;
-        case 2: tridiag<8, 4>(p, ws, member, G, sm); break;
-        default: tridiag<16, 2>(p, ws, member, G, sm); break;
+        case 0: tridiag<2, 16, false>(p, ws, member, G, sm); break;
+        case 1: tridiag<4, 8, false>(p, ws, member, G, sm); break;
+        case 2: tridiag<8, 4, false>(p, ws, member, G, sm); break;
+        default: tridiag<16, 2, false>(p, ws, member, G, sm); break;
+    }
+}
+
+// The problems whose group was given up, one workgroup each, the matrix in
+// memory: it waits for no other workgroup. The results have the same bits.
+__global__ void __launch_bounds__(512, 2)
+k_tridiag_one(const mpsx_two_site_op *ops, char *ws, int max_n) {
+    __shared__ TriShared<EIG_MAX_N> sm;
+    const mpsx_plan p = ops[blockIdx.x].plan;
+    if (!eig_direct(p, max_n)) return;
+    if (!(reinterpret_cast<const ProblemCtl *>(ws + p.ws_off)->group & kGroupLost)) return;
+    switch (eig_class(p.C)) {
+        case 0: break;  // a group of one
+        case 1: tridiag<4, 8, true>(p, ws, 0, 1, sm); break;
+        case 2: tridiag<8, 4, true>(p, ws, 0, 1, sm); break;
+        default: tridiag<16, 2, true>(p, ws, 0, 1, sm); break;
     }
 }
 
@@ -542,7 +575,7 @@ k_eig_t(const mpsx_two_site_op *ops, char *ws, int max_n) {
     const int nref = *ev.nref;
     if (16 * q >= nref) return;
     const int ncols = min(16, nref - 16 * q);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), l16 = lane & 15, lq = lane >> 4;
     const double2 *V = eig_h(ws, p) + (int64_t)q * 16 * Cp;
     mfma_d4 m1 = {0.0, 0.0, 0.0, 0.0}, m2 = m1, m3 = m1, m4 = m1;
     for (int r0 = 16 * q + 4 * wave; r0 < n; r0 += 16) {
@@ -580,188 +613,14 @@ k_eig_t(const mpsx_two_site_op *ops, char *ws, int max_n) {
 }
 
 // ---------------------------------------------------- divide and conquer
-namespace {
-
-// Rank-one update diag(d) + rho z z^T of a merge, poles in ascending order
-// (ds, zs, id): deflates the entries with negligible weight and, of poles
-// closer than the weights resolve, one of each pair after a rotation. K
-// poles stay (dl, zl, src[0 .. K-1]); the deflated ones fill dd and src from
-// the end. rot_i, rot_c: the rotations (row a, row b, c, s) in order. Serial.
-MPSX_DEV int deflate(int m, double rho, const double *ds, const double *zs, const int *id, double *dl,
-                     double *zl, int *src, double *dd, int2 *rot_i, double2 *rot_c, int *nrot) {
-    int K = 0, e = m, nr = 0, pj = -1;
-    double pd = 0.0, pz = 0.0;
-    int in = id[0];
-    double dn = ds[0], zn = zs[0];
-    for (int r = 0; r < m; ++r) {
-        const int i = in;
-        const double dr = dn, zr = zn;
-        if (r + 1 < m) {
-            in = id[r + 1];
-            dn = ds[r + 1];
-            zn = zs[r + 1];
-        }
-        if (rho * fabs(zr) <= kDeflate) {
-            --e;
-            src[e] = i;
-            dd[e] = dr;
-            continue;
-        }
-        if (pj >= 0) {
-            const double n2 = fma(pz, pz, zr * zr);
-            if (fabs((dr - pd) * pz * zr) <= kDeflate * n2) {
-                const double t = sqrt(n2), c = zr / t, s = -pz / t;
-                rot_i[nr] = make_int2(pj, i);
-                rot_c[nr] = make_double2(c, s);
-                ++nr;
-                --e;
-                src[e] = pj;
-                dd[e] = pd * c * c + dr * s * s;
-                pd = pd * s * s + dr * c * c;
-                pz = t;
-                pj = i;
-                continue;
-            }
-            dl[K] = pd;
-            zl[K] = pz;
-            src[K] = pj;
-            ++K;
-        }
-        pj = i;
-        pd = dr;
-        pz = zr;
-    }
-    if (pj >= 0) {
-        dl[K] = pd;
-        zl[K] = pz;
-        src[K] = pj;
-        ++K;
-    }
-    *nrot = nr;
-    return K;
-}
-
-MPSX_DEV double recip(double x) {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(r, fma(-x, r, 1.0), r);
-    return fma(r, fma(-x, r, 1.0), r);
-}
-
-// Root j of 1 + rho sum_i z_i^2 / (d_i - lambda), 0 <= j < K, by L lanes (sub
-// = lane in the group): lambda = dl[base] + tau with base the nearer of the
-// two poles around it, so that every difference d_i - lambda is accurate.
-template <int L>
-MPSX_DEV void secular_root(int K, const double *dl, const double *zl, double rho, int j, int sub, int *base,
-                           double *root) {
-    const bool last = j == K - 1;
-    const double dj = dl[j];
-    int org = j;
-    double lo, hi, t;
-    if (last) {
-        double s = 0.0;
-        for (int i = sub; i < K; i += L) s = fma(zl[i], zl[i], s);
-        s = group_sum<L>(s);
-        lo = 0.0;
-        hi = rho * s * (1.0 + 4.0 * kEps);
-        t = K == 1 ? rho * s : 0.5 * hi;
-    } else {
-        const double gap = dl[j + 1] - dj, mid = 0.5 * gap;
-        double c0 = 0.0;
-        for (int i = sub; i < K; i += L) {
-            if (i == j || i == j + 1) continue;
-            c0 = fma(zl[i] * zl[i], recip((dl[i] - dj) - mid), c0);
-        }
-        c0 = group_sum<L>(c0);
-        const double s = rho * zl[j] * zl[j], v = rho * zl[j + 1] * zl[j + 1], c = fma(rho, c0, 1.0);
-        const bool left = c + (v - s) / mid >= 0.0;
-        org = left ? j : j + 1;
-        lo = left ? 0.0 : -mid;
-        hi = left ? mid : 0.0;
-        // c + s / (p1 - t) + v / (p2 - t) = 0 with the poles at 0 and +-gap
-        const double A = left ? fma(c, gap, s + v) : fma(-c, gap, s + v);
-        const double B = left ? s * gap : -v * gap;
-        const double sq = sqrt(fmax(fma(A, A, -4.0 * c * B), 0.0));
-        t = A > 0.0 ? 2.0 * B / (A + sq) : (A - sq) / (2.0 * c);
-    }
-    if (K > 1) {
-        if (!(t > lo && t < hi)) t = 0.5 * (lo + hi);
-        const double dorg = dl[org], p1 = dj - dorg, p2 = last ? 0.0 : dl[j + 1] - dorg;
-        for (int it = 0; it < 64; ++it) {
-            double psi = 0.0, dpsi = 0.0, phi = 0.0, dphi = 0.0;
-            for (int i = sub; i < K; i += L) {
-                const double r = recip((dl[i] - dorg) - t), q = zl[i] * zl[i] * r, dq = q * r;
-                if (i <= j) {
-                    psi += q;
-                    dpsi += dq;
-                } else {
-                    phi += q;
-                    dphi += dq;
-                }
-            }
-            psi = rho * group_sum<L>(psi);
-            phi = rho * group_sum<L>(phi);
-            dpsi = rho * group_sum<L>(dpsi);
-            dphi = rho * group_sum<L>(dphi);
-            const double g = 1.0 + psi + phi;
-            if (fabs(g) <= kEps * (8.0 * (1.0 + fabs(psi) + fabs(phi)) + fabs(t) * (dpsi + dphi))) break;
-            if (g < 0.0)
-                lo = t;
-            else
-                hi = t;
-            double tn;
-            if (last) {
-                // c - s / t = 0 through the pole at the origin
-                tn = dpsi * t * t / fma(dpsi, t, g);
-            } else {
-                const double D1 = p1 - t, D2 = p2 - t;
-                const double s = dpsi * D1 * D1, v = dphi * D2 * D2, c = g - dpsi * D1 - dphi * D2;
-                const double A = fma(c, D1 + D2, s + v), B = D1 * D2 * g;
-                const double sq = sqrt(fmax(fma(A, A, -4.0 * c * B), 0.0));
-                const double q = 0.5 * (A + copysign(sq, A));
-                double eta = B / q;  // of the two roots, the one between the poles
-                if (!(eta > D1 && eta < D2)) eta = q / c;
-                tn = t + eta;
-            }
-            if (!(tn > lo && tn < hi)) tn = 0.5 * (lo + hi);
-            if (tn == t || hi - lo <= 2.0 * kEps * fmax(fabs(lo), fabs(hi))) break;
-            t = tn;
-        }
-    }
-    *base = org;
-    *root = t;
-}
-
-// |z_i| for which the computed roots are the exact ones (Gu & Eisenstat), by
-// L lanes.
-template <int L>
-MPSX_DEV double zhat(int K, const double *dl, const int *base, const double *rt, int i, int sub) {
-    const double di = dl[i];
-    double pr = 1.0;
-    for (int j = sub; j < K; j += L) {
-        const double num = (dl[base[j]] - di) + rt[j];
-        const double den = j < i ? dl[j] - di : (j < K - 1 ? dl[j + 1] - di : 1.0);
-        pr *= num / den;
-    }
-    return sqrt(fmax(group_prod<L>(pr), 0.0));
-}
-
-// Sort key: NaN below everything, so that ranks are a permutation.
-MPSX_DEV double sort_key(double x) { return x == x ? x : -__builtin_huge_val(); }
-
-}  // namespace
-
 // Leaves: the eigensystem of every 64 x 64 diagonal block of T, torn at each
 // entry, by six levels of merges in LDS. x: block, y: problem. Also scales T to
 // unit norm (es, d) for the merges above.
 __global__ void __launch_bounds__(256)
 k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
-    constexpr int M = 64;
-    __shared__ double S[2][M][M + 1];
-    __shared__ double U[M][M + 1];
-    __shared__ double d[M], z[M], ds[M], zs[M], dl[M], zl[M], dd[M], zh[M], rt[M];
-    __shared__ int id[M], src[M], base[M], kn[M], nrot[M];
-    __shared__ int2 rot_i[M];
-    __shared__ double2 rot_c[M];
+    constexpr int M = LEAF;
+    __shared__ double S[M][M + 1], U[M][M + 1];
+    __shared__ LeafShared L;
     __shared__ double red[4];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
@@ -784,104 +643,11 @@ k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
         const int i = b0 + tid;
         // d stays unscaled in memory (other leaves read it): this leaf's
         // eigenvalues go to rt, where the first merge takes them
-        d[tid] = i < n ? ev.d[i] * scale - fabs(off(i - 1)) - fabs(off(i)) : 0.0;
+        L.d[tid] = i < n ? ev.d[i] * scale - fabs(off(i - 1)) - fabs(off(i)) : 0.0;
+        L.e[tid] = off(i);
         if (i < n) ev.es[i] = off(i);
     }
-    for (int e = tid; e < M * M; e += 256) {
-        S[0][e >> 6][e & 63] = (e >> 6) == (e & 63) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    int cur = 0;
-    for (int s = 1; s < m; s <<= 1) {
-        const int h = 2 * s;
-        const int ni = tid < M ? tid : (tid >> 2);  // index this thread serves in the 1-per-index steps
-        const int lo = ni & ~(h - 1), mid = lo + s, hi = min(lo + h, m), sz = hi - lo;
-        const bool merge = mid < hi;
-        const double ee = (lo < m && merge) ? off(b0 + mid - 1) : 0.0;
-        if (tid < m) {
-            z[tid] = merge ? S[cur][tid][tid < mid ? mid - 1 : mid] *
-                                 (tid >= mid && ee < 0.0 ? -0.7071067811865476 : 0.7071067811865476)
-                           : 0.0;
-        }
-        __syncthreads();
-        if (tid < m) {
-            const double key = sort_key(d[tid]);
-            int rank = 0;
-            for (int o = lo; o < hi; ++o) {
-                const double ko = sort_key(d[o]);
-                rank += (ko < key) || (ko == key && o < tid);
-            }
-            ds[lo + rank] = d[tid];
-            zs[lo + rank] = z[tid];
-            id[lo + rank] = tid;
-        }
-        __syncthreads();
-        if (tid < m && tid == lo) {
-            kn[lo] = deflate(sz, merge ? 2.0 * fabs(ee) : 0.0, ds + lo, zs + lo, id + lo, dl + lo, zl + lo, src + lo,
-                             dd + lo, rot_i + lo, rot_c + lo, &nrot[lo]);
-        }
-        __syncthreads();
-        if (tid < m) {  // component tid of the node's rows
-            for (int r = 0; r < nrot[lo]; ++r) {
-                const int2 ab = rot_i[lo + r];
-                const double2 cs = rot_c[lo + r];
-                const double xa = S[cur][ab.x][tid], xb = S[cur][ab.y][tid];
-                S[cur][ab.x][tid] = cs.x * xa + cs.y * xb;
-                S[cur][ab.y][tid] = cs.x * xb - cs.y * xa;
-            }
-        }
-        __syncthreads();
-        // four lanes per root from here on
-        const int g = tid >> 2, sub = tid & 3;
-        const int glo = g & ~(h - 1), gmid = glo + s;
-        const int K = g < m ? kn[glo] : 0, gj = g - glo;
-        const double grho = (g < m && gmid < min(glo + h, m)) ? 2.0 * fabs(off(b0 + gmid - 1)) : 0.0;
-        if (gj < K) {
-            int bs;
-            double root;
-            secular_root<4>(K, dl + glo, zl + glo, grho, gj, sub, &bs, &root);
-            if (sub == 0) {
-                base[g] = bs;
-                rt[g] = root;
-            }
-        }
-        __syncthreads();
-        if (gj < K) {
-            const double v = zhat<4>(K, dl + glo, base + glo, rt + glo, gj, sub);
-            if (sub == 0) zh[g] = copysign(v, zl[g]);
-        }
-        __syncthreads();
-        if (gj < K) {
-            const double db = dl[glo + base[g]], tj = rt[g];
-            double nn = 0.0;
-            for (int i = sub; i < K; i += 4) {
-                const double u = zh[glo + i] / ((dl[glo + i] - db) - tj);
-                U[g][i] = u;
-                nn = fma(u, u, nn);
-            }
-            nn = group_sum<4>(nn);
-            const double f = 1.0 / sqrt(nn);
-            for (int i = sub; i < K; i += 4) U[g][i] *= f;
-        }
-        __syncthreads();
-        for (int e = tid; e < M * M; e += 256) {
-            const int j = e >> 6, r = e & 63;
-            const int jlo = j & ~(h - 1);
-            double v = 0.0;
-            if (j < m && r >= jlo && r < min(jlo + h, m)) {
-                const int Kj = kn[jlo];
-                if (j - jlo < Kj) {
-                    for (int i = 0; i < Kj; ++i) v = fma(U[j][i], S[cur][src[jlo + i]][r], v);
-                } else {
-                    v = S[cur][src[j]][r];
-                }
-            }
-            S[cur ^ 1][j][r] = v;
-        }
-        if (tid < m) d[tid] = (tid - lo) < kn[lo] ? dl[lo + base[tid]] + rt[tid] : dd[tid];
-        __syncthreads();
-        cur ^= 1;
-    }
+    leaf_conquer<256>(m, S, U, L);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
     // both buffers of S^T: zero outside the block (the merges write their
@@ -889,9 +655,9 @@ k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
     for (int j = tid >> 6; j < m; j += 4)
         for (int r = tid & 63; r < 2 * p.Cp; r += 64) {
             const int rr = r - b0;
-            y[(int64_t)(b0 + j) * ld2 + r] = (rr >= 0 && rr < m) ? S[cur][j][rr] : 0.0;
+            y[(int64_t)(b0 + j) * ld2 + r] = (rr >= 0 && rr < m) ? S[j][rr] : 0.0;
         }
-    if (tid < m) ev.rt[b0 + tid] = d[tid];
+    if (tid < m) ev.rt[b0 + tid] = L.d[tid];
 }
 
 // Merge of the blocks [lo, lo + s) and [lo + s, lo + 2 s): z, sorting,
@@ -1054,7 +820,7 @@ k_eig_vectors(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf) 
     const double *in = eig_y(ws, p) + (int64_t)buf * p.Cp + lo;
     double *out = eig_y(ws, p) + (int64_t)(buf ^ 1) * p.Cp + lo;
     const int K = ev.kn[lo];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), l16 = lane & 15, lq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
     if (j0 < K) {
         // thread: row j of the tile, 4 of the 16 poles of a stage
@@ -1138,7 +904,7 @@ k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
     if (!eig_direct(p, max_n) || (CH == 4) != (p.C <= 512)) return;
     const int n = p.C, Cp = p.Cp, i0 = 16 * (int)blockIdx.x;
     if (i0 >= n) return;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, lq = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = wave_id(), l16 = lane & 15, lq = lane >> 4;
     const EigVec ev = eig_vec(ws, p);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
@@ -1230,10 +996,12 @@ k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
 
 // ---------------------------------------------------------------- launchers
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots) {
+                              int slots, bool grouped) {
     hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, static_cast<int2 *>(map), max_n);
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)slots), dim3(512), 0, s, d, static_cast<const int2 *>(map), ws,
                        slots);
+    if (grouped)
+        hipLaunchKernelGGL(k_tridiag_one, dim3((unsigned)count), dim3(512), 0, s, d, ws, max_n);
     return hipGetLastError();
 }
 

@@ -17,27 +17,31 @@ hipError_t launch_gemm_rows(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gem
                             int count);
 
 // max_n: rows up to which the Gram problems take the direct eigensolver
-// (eig_direct; 0: none do).
+// (eig_direct; 0: none do). small: 1 when the one-workgroup kernel takes the
+// problems small_route selects; the others of these launches pass them by.
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows, int max_n);
+                            int64_t rows, int max_n, int small);
 hipError_t launch_theta(hipStream_t s, bool f32, int D, const mpsx_two_site_op *d, int count, char *ws,
                         int64_t tiles);
 hipError_t launch_theta_gen(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
                             int64_t tiles);
 hipError_t launch_rownorm(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                          int64_t rows);
+                          int64_t rows, int small);
 hipError_t launch_fro(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                      double null_rel);
+                      double null_rel, int small);
 hipError_t launch_owner(hipStream_t s, const mpsx_two_site_op *d, int count, int *owner);
 hipError_t launch_jacobi_round(hipStream_t s, bool f32, int b, const mpsx_two_site_op *d, const int *owner,
-                               char *ws, int64_t pairs, int round, double tol, double tol_inner,
+                               char *ws, int small, int64_t pairs, int round, double tol, double tol_inner,
                                int inner_sweeps);
 hipError_t launch_sweep_end(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                            int sweep, bool fp32_phase);
+                            int sweep, bool fp32_phase, int small);
 hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                       int *unconverged);
+                       int *unconverged, int small);
 hipError_t launch_gather(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                         int64_t outs);
+                         int64_t outs, int small);
+// The one-workgroup kernel (small.hip), from theta to the factors.
+hipError_t launch_small(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, double tol, double null_rel,
+                        int *unconverged);
 hipError_t launch_hgram(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
                         int64_t pairs, int max_nb, int stage, int max_n);
 hipError_t launch_hsolve(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
@@ -63,10 +67,10 @@ hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, c
                           int strips, int max_c, bool small, bool large, int max_n);
 // Direct eigensolver (eig.hip) of the problems eig_direct selects: the
 // tridiagonal form (`map`: room for `slots` int2, the workgroups of all their
-// groups), the eigensystem of T, and Y. n: the largest C among them; `small`,
+// groups; `grouped`: some group has more than one), the eigensystem of T, and Y. n: the largest C among them; `small`,
 // `large`: some of at most 512 rows, some above.
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots);
+                              int slots, bool grouped);
 hipError_t launch_eig_conquer(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
 hipError_t launch_eig_back(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n,
                            bool small, bool large);

@@ -70,7 +70,7 @@ MPSX_DEV double block_sum_256(double v, double *red) {
 // rows <- 0. Row 0 of each problem also resets its control block.
 template <class T>
 __global__ void __launch_bounds__(256)
-k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
+k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n, int small) {
     using Z2 = typename Cx<T>::type;
     if (blockIdx.x == 0 && threadIdx.x < 64) {
         reinterpret_cast<TwoSiteHeader *>(ws)->active[threadIdx.x] = 0;
@@ -80,7 +80,7 @@ k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
                                OP_FIELD(plan.row_base), blockIdx.x);
     const mpsx_plan p = ops[pi].plan;
     const int row = (int)(blockIdx.x - p.row_base);
-    if (row >= p.Cp) return;
+    if (row >= p.Cp || small_route(p, small)) return;
     Z2 *z = z_ptr<T>(ws, p) + (int64_t)row * p.LD;
     if (row >= p.C)
         for (int c = threadIdx.x; c < p.R; c += 256) z[c] = Cx<T>::make(0, 0);
@@ -101,6 +101,7 @@ k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n) {
         ctl->counter = 0;
         ctl->conv = (p.C == 0 || p.R == 0 || direct) ? 1 : 0;
         ctl->sweeps = 0;
+        ctl->group = 0;
     }
 }
 
@@ -297,13 +298,13 @@ k_load(const mpsx_two_site_op *ops, int count, char *ws) {
 // One workgroup per padded row: sig2[row] = sum_c |X[row, c]|^2 (FP64).
 template <class T>
 __global__ void __launch_bounds__(256)
-k_rownorm(const mpsx_two_site_op *ops, int count, char *ws) {
+k_rownorm(const mpsx_two_site_op *ops, int count, char *ws, int small) {
     __shared__ double red[4];
     const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
                                OP_FIELD(plan.row_base), blockIdx.x);
     const mpsx_plan p = ops[pi].plan;
     const int row = (int)(blockIdx.x - p.row_base);
-    if (row >= p.Cp) return;
+    if (row >= p.Cp || small_route(p, small)) return;
     const typename Cx<T>::type *z = z_ptr<T>(ws, p) + (int64_t)row * p.LD;
     double s = 0.0;
     if (row < p.C)
@@ -317,11 +318,12 @@ k_rownorm(const mpsx_two_site_op *ops, int count, char *ws) {
 
 // One workgroup per problem: Frobenius norm and the null-row threshold.
 __global__ void __launch_bounds__(256)
-k_fro(const mpsx_two_site_op *ops, int count, char *ws, double null_rel) {
+k_fro(const mpsx_two_site_op *ops, int count, char *ws, double null_rel, int small) {
     __shared__ double red[4];
     const int pi = blockIdx.x;
     if (pi >= count) return;
     const mpsx_plan p = ops[pi].plan;
+    if (small_route(p, small)) return;
     const double *sig = sig_ptr(ws, p);
     double s = 0.0;
     for (int i = threadIdx.x; i < p.C; i += 256) s += sig[i];
@@ -733,7 +735,7 @@ k_jacobi_round32(const mpsx_two_site_op *ops, const int *owner, char *ws, int ro
 
 template <int B2>
 __global__ void __launch_bounds__(256)
-k_jacobi_round64(const mpsx_two_site_op *ops, const int *owner, char *ws, int round, double tol,
+k_jacobi_round64(const mpsx_two_site_op *ops, const int *owner, char *ws, int small, int round, double tol,
                  double tol_inner, int inner_sweeps) {
     constexpr int b = B2 / 2;
     constexpr int RG = B2 / 16;         // 16-row groups of complex pivot rows
@@ -754,7 +756,7 @@ k_jacobi_round64(const mpsx_two_site_op *ops, const int *owner, char *ws, int ro
 
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if (p.b != b || p.method != 0) return;
+    if (p.b != b || p.method != 0 || small_route(p, small)) return;
     if (round >= p.nb - 1) return;
     ProblemCtl *ctl = ctl_ptr(ws, p);
     if (ctl->conv) return;
@@ -1838,12 +1840,12 @@ __global__ void k_owner(const mpsx_two_site_op *ops, int count, int *owner) {
 // header's active counters, reused modulo 64: the next one is cleared
 // here). In the FP32 phase (fp32_phase) only the mixed Gram problems swept.
 __global__ void k_sweep_end(const mpsx_two_site_op *ops, int count, char *ws, int sweep,
-                            int fp32_phase) {
+                            int fp32_phase, int small) {
     const int pi = blockIdx.x * blockDim.x + threadIdx.x;
     if (pi == 0) reinterpret_cast<TwoSiteHeader *>(ws)->active[(sweep + 1) & 63] = 0;
     if (pi >= count) return;
     const mpsx_plan p = ops[pi].plan;
-    if (fp32_phase && p.method != 2) return;
+    if ((fp32_phase && p.method != 2) || small_route(p, small)) return;
     ProblemCtl *ctl = ctl_ptr(ws, p);
     if (ctl->conv) return;
     if (ctl->counter == 0) {
@@ -1861,30 +1863,31 @@ __global__ void k_sweep_end(const mpsx_two_site_op *ops, int count, char *ws, in
 // a count of problems left unconverged (when `unconverged` is not null).
 constexpr int SORT_LDS = 4096;
 __global__ void __launch_bounds__(256)
-k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged) {
+k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int small) {
     __shared__ double sg[SORT_LDS];
     __shared__ double red[4];
     const int pi = blockIdx.x;
     if (pi >= count) return;
     const mpsx_two_site_op &op = ops[pi];
     const mpsx_plan p = op.plan;
+    if (small_route(p, small)) return;
     const int C = p.C, k = op.k;
     const double *sig = sig_ptr(ws, p);
     int *perm = perm_ptr(ws, p);
     const bool in_lds = C <= SORT_LDS;
     if (in_lds)
-        for (int i = threadIdx.x; i < C; i += 256) sg[i] = sig[i];
+        for (int i = threadIdx.x; i < C; i += 256) sg[i] = sort_key(sig[i]);
     __syncthreads();
     double disc = 0.0;
     for (int i = threadIdx.x; i < C; i += 256) {
-        const double si = in_lds ? sg[i] : sig[i];
+        const double si = in_lds ? sg[i] : sort_key(sig[i]);
         int rank = 0;
         for (int j = 0; j < C; ++j) {
-            const double sj = in_lds ? sg[j] : sig[j];
+            const double sj = in_lds ? sg[j] : sort_key(sig[j]);
             rank += (sj > si) || (sj == si && j < i);
         }
         perm[rank] = i;
-        if (rank >= k) disc += si;
+        if (rank >= k) disc += sig[i];
     }
     disc = block_sum_256(disc, red);
     __syncthreads();
@@ -1893,8 +1896,7 @@ k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged) {
         atomicAdd(unconverged, 1);
     if (op.s_out)
         for (int j = threadIdx.x; j < k; j += 256) {
-            const double s2 = in_lds ? sg[perm[j]] : sig[perm[j]];
-            op.s_out[j] = (float)sqrt(s2);
+            op.s_out[j] = (float)sqrt(sig[perm[j]]);
         }
 }
 
@@ -1908,13 +1910,14 @@ k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged) {
 //   absorb left:  a_out[m][j] = X[perm[j]][m],        b_out[j][n] = conj(Y[perm[j]][n])
 template <class T>
 __global__ void __launch_bounds__(256)
-k_gather(const mpsx_two_site_op *ops, int count, char *ws) {
+k_gather(const mpsx_two_site_op *ops, int count, char *ws, int small) {
     using Z2 = typename Cx<T>::type;
     __shared__ Z2 tile[32][33];
     const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
                                OP_FIELD(plan.out_base), blockIdx.x);
     const mpsx_two_site_op &op = ops[pi];
     const mpsx_plan p = op.plan;
+    if (small_route(p, small)) return;
     const int M = op.d * op.chi_l, N = op.d * op.chi_r, k = op.k;
     const int64_t u = (int64_t)blockIdx.x - p.out_base;
     if (u >= gather_units(M, k)) return;
@@ -1952,15 +1955,15 @@ k_gather(const mpsx_two_site_op *ops, int count, char *ws) {
 // ---------------------------------------------------------------- launchers
 template <class T>
 static void launch_init_rows_t(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                               int64_t rows, int max_n) {
-    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n);
+                               int64_t rows, int max_n, int small) {
+    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n, small);
 }
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows, int max_n) {
+                            int64_t rows, int max_n, int small) {
     if (f32)
-        launch_init_rows_t<float>(s, d, count, ws, rows, max_n);
+        launch_init_rows_t<float>(s, d, count, ws, rows, max_n, small);
     else
-        launch_init_rows_t<double>(s, d, count, ws, rows, max_n);
+        launch_init_rows_t<double>(s, d, count, ws, rows, max_n, small);
     return hipGetLastError();
 }
 
@@ -1994,16 +1997,16 @@ hipError_t launch_theta_gen(hipStream_t s, bool f32, const mpsx_two_site_op *d, 
 }
 
 hipError_t launch_rownorm(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                          int64_t rows) {
+                          int64_t rows, int small) {
     if (f32)
-        hipLaunchKernelGGL(k_rownorm<float>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws);
+        hipLaunchKernelGGL(k_rownorm<float>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, small);
     else
-        hipLaunchKernelGGL(k_rownorm<double>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws);
+        hipLaunchKernelGGL(k_rownorm<double>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, small);
     return hipGetLastError();
 }
 
-hipError_t launch_fro(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, double null_rel) {
-    hipLaunchKernelGGL(k_fro, dim3((unsigned)count), dim3(256), 0, s, d, count, ws, null_rel);
+hipError_t launch_fro(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, double null_rel, int small) {
+    hipLaunchKernelGGL(k_fro, dim3((unsigned)count), dim3(256), 0, s, d, count, ws, null_rel, small);
     return hipGetLastError();
 }
 
@@ -2013,7 +2016,7 @@ hipError_t launch_owner(hipStream_t s, const mpsx_two_site_op *d, int count, int
 }
 
 hipError_t launch_jacobi_round(hipStream_t s, bool f32, int b, const mpsx_two_site_op *d,
-                               const int *owner, char *ws, int64_t pairs, int round, double tol,
+                               const int *owner, char *ws, int small, int64_t pairs, int round, double tol,
                                double tol_inner, int inner_sweeps) {
     const dim3 g((unsigned)pairs), blk(256);
     if (b != 8 && b != 16) return hipErrorInvalidValue;
@@ -2026,34 +2029,34 @@ hipError_t launch_jacobi_round(hipStream_t s, bool f32, int b, const mpsx_two_si
                                inner_sweeps);
     } else {
         if (b == 8)
-            hipLaunchKernelGGL(k_jacobi_round64<16>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner,
+            hipLaunchKernelGGL(k_jacobi_round64<16>, g, blk, 0, s, d, owner, ws, small, round, tol, tol_inner,
                                inner_sweeps);
         else
-            hipLaunchKernelGGL(k_jacobi_round64<32>, g, blk, 0, s, d, owner, ws, round, tol, tol_inner,
+            hipLaunchKernelGGL(k_jacobi_round64<32>, g, blk, 0, s, d, owner, ws, small, round, tol, tol_inner,
                                inner_sweeps);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_sweep_end(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int sweep,
-                            bool fp32_phase) {
+                            bool fp32_phase, int small) {
     hipLaunchKernelGGL(k_sweep_end, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, d, count, ws,
-                       sweep, fp32_phase ? 1 : 0);
+                       sweep, fp32_phase ? 1 : 0, small);
     return hipGetLastError();
 }
 
 hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                       int *unconverged) {
-    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(256), 0, s, d, count, ws, unconverged);
+                       int *unconverged, int small) {
+    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(256), 0, s, d, count, ws, unconverged, small);
     return hipGetLastError();
 }
 
 hipError_t launch_gather(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                         int64_t outs) {
+                         int64_t outs, int small) {
     if (f32)
-        hipLaunchKernelGGL(k_gather<float>, dim3((unsigned)outs), dim3(256), 0, s, d, count, ws);
+        hipLaunchKernelGGL(k_gather<float>, dim3((unsigned)outs), dim3(256), 0, s, d, count, ws, small);
     else
-        hipLaunchKernelGGL(k_gather<double>, dim3((unsigned)outs), dim3(256), 0, s, d, count, ws);
+        hipLaunchKernelGGL(k_gather<double>, dim3((unsigned)outs), dim3(256), 0, s, d, count, ws, small);
     return hipGetLastError();
 }
 

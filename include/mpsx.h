@@ -56,6 +56,18 @@ int mpsx_device_info(int device, char *arch, int arch_len, int *num_cus);
 size_t mpsx_sizeof(int which);
 
 /* ------------------------------------------------------------------------
+ * Copies a small host table (at most MPSX_PUT_MAX bytes, a multiple of 4) to
+ * the device buffer `dst` on `stream`: the bytes travel in the arguments of
+ * kernel launches, so `src` may be changed on return and neither the host
+ * nor the stream waits for the other. For the descriptor tables of the calls
+ * below. Refused on a stream being captured (the bytes would be frozen into
+ * the graph).
+ * ---------------------------------------------------------------------- */
+#define MPSX_PUT_MAX ((size_t)16384)
+
+int mpsx_put(mpsx_stream stream, void *dst, const void *src, size_t bytes);
+
+/* ------------------------------------------------------------------------
  * One-site gate.
  * Replaces MPS.apply_one_qudit_gate (mpsim/core.py:753-826): gate edge 1
  * contracts the site's physical leg, gate edge 0 becomes the new leg,

@@ -27,7 +27,7 @@ from typing import List, Optional, Sequence, Tuple, Union
 import numpy as np
 
 from . import _native as nat
-from .engine import Engine, SplitItem, TwoSiteItem
+from .engine import Engine, GemmChain, SplitItem, TwoSiteItem
 from .gates import (Edge, Node, as_tensor, cnot, haar_random_unitary, hgate, is_unitary, rgate,
                     swap, xgate)
 
@@ -279,13 +279,15 @@ class MPS:
         d = self._qudit_dimension
         t0 = self._tensors[0]
         psi = t0.reshape(d, t0.shape[2])
+        chain = GemmChain(self._engine)
         for t in self._tensors[1:]:
             cl, _, cr = t.shape
             rows = psi.shape[0]
             out = torch.empty((rows, d * cr), dtype=torch.complex64, device=self._engine.dev)
-            self._engine.gemm([dict(A=psi, B=t, C=out, m=rows, n=d * cr, k=cl, lda=psi.shape[1],
-                                    ldb=d * cr, ldc=d * cr)])
+            chain.gemm([dict(A=psi, B=t, C=out, m=rows, n=d * cr, k=cl, lda=psi.shape[1],
+                             ldb=d * cr, ldc=d * cr)])
             psi = out.reshape(rows * d, cr)
+        chain.flush()
         return psi.reshape(d ** self._nqudits)
 
     def dagger(self) -> None:
@@ -311,18 +313,20 @@ class MPS:
         dev = self._engine.dev
         d = self._qudit_dimension
         env = torch.ones((1, 1), dtype=torch.complex64, device=dev)
+        chain = GemmChain(self._engine)
         for a, b in zip(self._tensors, other._tensors):
             xl, _, xr = a.shape
             yl, _, yr = b.shape
             f = torch.empty((yl, d * xr), dtype=torch.complex64, device=dev)
             e2 = torch.empty((yr, xr), dtype=torch.complex64, device=dev)
             # F[y, (p, x')] = sum_x E[y, x] a[x, p, x']
-            self._engine.gemm([dict(A=env, B=a, C=f, m=yl, n=d * xr, k=xl, lda=xl, ldb=d * xr,
-                                    ldc=d * xr)])
+            chain.gemm([dict(A=env, B=a, C=f, m=yl, n=d * xr, k=xl, lda=xl, ldb=d * xr,
+                             ldc=d * xr)])
             # E'[y', x'] = sum_{y,p} conj(b[y, p, y']) F[y, p, x']
-            self._engine.gemm([dict(A=b, B=f, C=e2, m=yr, n=xr, k=yl * d, lda=yr, ldb=xr,
-                                    ldc=xr, flags=nat.GEMM_CONJ_A)])
+            chain.gemm([dict(A=b, B=f, C=e2, m=yr, n=xr, k=yl * d, lda=yr, ldb=xr,
+                             ldc=xr, flags=nat.GEMM_CONJ_A)])
             env = e2
+        chain.flush()
         return env[0, 0]
 
     def norm(self) -> float:
@@ -380,28 +384,30 @@ class MPS:
         dev, eng, d = self._engine.dev, self._engine, self._qudit_dimension
         keep = set(kept)
         env = torch.ones((1, 1, 1, 1), dtype=torch.complex64, device=dev)
+        chain = GemmChain(eng)
         kb = ka = 1
         for i, a in enumerate(self._tensors):
             xl, _, xr = a.shape
             f = torch.empty((kb, xl, ka, d * xr), dtype=torch.complex64, device=dev)
-            eng.gemm([dict(A=env, B=a, C=f, m=kb * xl * ka, n=d * xr, k=xl, lda=xl,
-                           ldb=d * xr, ldc=d * xr)])
+            chain.gemm([dict(A=env, B=a, C=f, m=kb * xl * ka, n=d * xr, k=xl, lda=xl,
+                             ldb=d * xr, ldc=d * xr)])
             row_f = ka * d * xr
             if i in keep:
                 nxt = torch.empty((kb, d, xr, ka, d, xr), dtype=torch.complex64, device=dev)
-                eng.gemm([dict(A=a, B=(f, b * xl * row_f), C=(nxt, b * d * xr * ka * d * xr),
-                               m=d * xr, n=row_f, k=xl, lda=d * xr, ldb=row_f, ldc=row_f,
-                               flags=nat.GEMM_CONJ_A) for b in range(kb)])
+                chain.gemm([dict(A=a, B=(f, b * xl * row_f), C=(nxt, b * d * xr * ka * d * xr),
+                                 m=d * xr, n=row_f, k=xl, lda=d * xr, ldb=row_f, ldc=row_f,
+                                 flags=nat.GEMM_CONJ_A) for b in range(kb)])
                 kb, ka = kb * d, ka * d
             else:
                 nxt = torch.empty((kb, xr, ka, xr), dtype=torch.complex64, device=dev)
                 for s in range(d):
-                    eng.gemm([dict(A=(a, s * xr), B=(f, b * xl * row_f + c * d * xr + s * xr),
-                                   C=(nxt, b * xr * ka * xr + c * xr), m=xr, n=xr, k=xl,
-                                   lda=d * xr, ldb=row_f, ldc=ka * xr,
-                                   flags=nat.GEMM_CONJ_A | (nat.GEMM_ACCUM if s else 0))
-                              for b in range(kb) for c in range(ka)])
+                    chain.gemm([dict(A=(a, s * xr), B=(f, b * xl * row_f + c * d * xr + s * xr),
+                                     C=(nxt, b * xr * ka * xr + c * xr), m=xr, n=xr, k=xl,
+                                     lda=d * xr, ldb=row_f, ldc=ka * xr,
+                                     flags=nat.GEMM_CONJ_A | (nat.GEMM_ACCUM if s else 0))
+                                for b in range(kb) for c in range(ka)])
             env = nxt
+        chain.flush()
         return env.reshape(kb, ka).transpose(0, 1)
 
     def _marginals_device(self):
@@ -419,38 +425,40 @@ class MPS:
         torch = self._engine.torch
         dev, eng, d, n = self._engine.dev, self._engine, self._qudit_dimension, self._nqudits
         c64 = torch.complex64
+        chain = GemmChain(eng)
         q = [None] * (n + 1)
         q[n] = torch.ones((1, 1), dtype=c64, device=dev)
         for i in range(n - 1, 0, -1):
             a = self._tensors[i]
             xl, _, xr = a.shape
             g = torch.empty((xl * d, xr), dtype=c64, device=dev)
-            eng.gemm([dict(A=a, B=q[i + 1], C=g, m=xl * d, n=xr, k=xr, lda=xr, ldb=xr, ldc=xr,
-                           flags=nat.GEMM_CONJ_B)])
+            chain.gemm([dict(A=a, B=q[i + 1], C=g, m=xl * d, n=xr, k=xr, lda=xr, ldb=xr, ldc=xr,
+                             flags=nat.GEMM_CONJ_B)])
             q[i] = torch.empty((xl, xl), dtype=c64, device=dev)
-            eng.gemm([dict(A=a, B=g, C=q[i], m=xl, n=xl, k=d * xr, lda=d * xr, ldb=d * xr,
-                           ldc=xl, flags=nat.GEMM_CONJ_B)])
+            chain.gemm([dict(A=a, B=g, C=q[i], m=xl, n=xl, k=d * xr, lda=d * xr, ldb=d * xr,
+                             ldc=xl, flags=nat.GEMM_CONJ_B)])
         env = torch.ones((1, 1), dtype=c64, device=dev)
         dsv = []
         for i, a in enumerate(self._tensors):
             xl, _, xr = a.shape
             f = torch.empty((xl, d * xr), dtype=c64, device=dev)
-            eng.gemm([dict(A=env, B=a, C=f, m=xl, n=d * xr, k=xl, lda=xl, ldb=d * xr,
-                           ldc=d * xr)])
+            chain.gemm([dict(A=env, B=a, C=f, m=xl, n=d * xr, k=xl, lda=xl, ldb=d * xr,
+                             ldc=d * xr)])
             ds = torch.empty((d, xr, xr), dtype=c64, device=dev)
-            eng.gemm([dict(A=(a, s * xr), B=(f, s * xr), C=(ds, s * xr * xr), m=xr, n=xr,
-                           k=xl, lda=d * xr, ldb=d * xr, ldc=xr, flags=nat.GEMM_CONJ_A)
-                      for s in range(d)])
+            chain.gemm([dict(A=(a, s * xr), B=(f, s * xr), C=(ds, s * xr * xr), m=xr, n=xr,
+                             k=xl, lda=d * xr, ldb=d * xr, ldc=xr, flags=nat.GEMM_CONJ_A)
+                        for s in range(d)])
             dsv.append(ds)
             if i + 1 < n:
                 env = torch.empty((xr, xr), dtype=c64, device=dev)
-                eng.gemm([dict(A=a, B=f, C=env, m=xr, n=xr, k=xl * d, lda=xr, ldb=xr, ldc=xr,
-                               flags=nat.GEMM_CONJ_A)])
+                chain.gemm([dict(A=a, B=f, C=env, m=xr, n=xr, k=xl * d, lda=xr, ldb=xr, ldc=xr,
+                                 flags=nat.GEMM_CONJ_A)])
         p = torch.empty((n, d), dtype=c64, device=dev)
         # p[i, s] = conj(Q_{i+1})^T . vec(D_s): a 1 x 1 product over xr^2 terms
-        eng.gemm([dict(A=q[i + 1], B=(dsv[i], s * q[i + 1].numel()), C=(p, i * d + s), m=1, n=1,
-                       k=q[i + 1].numel(), lda=1, ldb=1, ldc=1, flags=nat.GEMM_CONJ_A)
-                  for i in range(n) for s in range(d)])
+        chain.gemm([dict(A=q[i + 1], B=(dsv[i], s * q[i + 1].numel()), C=(p, i * d + s), m=1, n=1,
+                         k=q[i + 1].numel(), lda=1, ldb=1, ldc=1, flags=nat.GEMM_CONJ_A)
+                    for i in range(n) for s in range(d)])
+        chain.flush()
         return p.real
 
     def _sample(self, as_string: bool = False, marginals: Optional[np.ndarray] = None):

@@ -236,6 +236,20 @@ int mpsx_device_info(int device, char *arch, int arch_len, int *num_cus) {
     return MPSX_OK;
 }
 
+// ---------------------------------------------------------------- tables
+int mpsx_put(mpsx_stream stream, void *dst, const void *src, size_t bytes) {
+    if (bytes == 0) return MPSX_OK;
+    if (!dst || !src) return fail(MPSX_EINVAL, "null pointer");
+    if (bytes > MPSX_PUT_MAX || bytes % 4 || reinterpret_cast<uintptr_t>(dst) % 4)
+        return fail(MPSX_EINVAL, "%zu bytes: not a multiple of 4 up to %zu at a 4-byte boundary", bytes,
+                    (size_t)MPSX_PUT_MAX);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap), "hipStreamIsCapturing");
+    if (cap != hipStreamCaptureStatusNone) return fail(MPSX_EINVAL, "mpsx_put on a stream being captured");
+    HIP_TRY(timed("k_put", (hipStream_t)stream, [&] { return launch_put((hipStream_t)stream, dst, src, bytes); }), "k_put");
+    return MPSX_OK;
+}
+
 // ---------------------------------------------------------------- one-site
 int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h, const mpsx_site_op *d,
                         int count) {

@@ -211,6 +211,10 @@ template <> struct Cx<double> {
     static MPSX_DEV double2 make(double x, double y) { return make_double2(x, y); }
 };
 
+// Bytes of a table that one launch of k_put carries in its arguments (below
+// the 4 KB a launch takes), and the largest table mpsx_put takes.
+constexpr int PUT_CHUNK = 3840;
+
 // Workgroups of the final gather of one problem: 32x32 tiles of the
 // M x k unscaled-by-column factor (read as a transpose of rows of Z), then
 // one per row of the k x N factor.

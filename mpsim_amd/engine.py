@@ -18,19 +18,48 @@ from . import _native as nat
 MAX_OPS = 65535  # descriptors per grouped launch (grid y / x limits of the kernels)
 
 
-def _matrix_addr(x, rows: int, cols: int, ld: int, what: str) -> int:
+def _tensor_info(t, what: str) -> Tuple[int, int]:
+    """(device address, elements) of a contiguous complex64 tensor."""
+    n = t.numel()
+    if n and t.element_size() != 8:
+        raise ValueError(f"gemm operand {what} must be complex64")
+    return nat.ptr(t), n
+
+
+def _matrix_addr(x, rows: int, cols: int, ld: int, what: str, seen: dict) -> int:
     """Device address of a rows x cols matrix with row stride `ld` stored in
     a contiguous complex64 tensor at an element offset (x = tensor or
-    (tensor, offset)); raises if any element would fall outside it."""
-    t, off = x if isinstance(x, tuple) else (x, 0)
-    if rows == 0 or cols == 0:
-        return nat.ptr(t) + 8 * off if t.numel() else 0
-    if cols > ld or off < 0 or off + (rows - 1) * ld + cols > t.numel():
+    (tensor, offset)); raises if any element would fall outside it. seen: the
+    _tensor_info of the call's tensors so far (many products share one)."""
+    t, off = x if type(x) is tuple else (x, 0)
+    info = seen.get(id(t))
+    if info is None:
+        if rows == 0 or cols == 0:
+            return nat.ptr(t) + 8 * off if t.numel() else 0
+        info = seen[id(t)] = _tensor_info(t, what)
+    p, n = info
+    if rows and cols and (cols > ld or off < 0 or off + (rows - 1) * ld + cols > n):
         raise ValueError(f"gemm operand {what}: {rows}x{cols} (ld {ld}) at offset {off} "
-                         f"exceeds a tensor of {t.numel()} elements")
-    if t.element_size() != 8:
-        raise ValueError(f"gemm operand {what} must be complex64")
-    return nat.ptr(t) + 8 * off
+                         f"exceeds a tensor of {n} elements")
+    return p + 8 * off if n else 0
+
+
+def _gemm_rows(ops: Sequence[dict]) -> List[tuple]:
+    """Descriptor rows of a grouped product, every matrix checked to lie
+    inside its tensor."""
+    rows, seen = [], {}
+    for o in ops:
+        m, n, k, fl = int(o["m"]), int(o["n"]), int(o["k"]), int(o.get("flags", 0))
+        lda, ldb, ldc = o["lda"], o["ldb"], o["ldc"]
+        # stored shapes: op(A) = A^H means A is stored k x m, else m x k
+        ra, ca = (k, m) if fl & nat.GEMM_CONJ_A else (m, k)
+        rb, cb = (n, k) if fl & nat.GEMM_CONJ_B else (k, n)
+        pa = _matrix_addr(o["A"], ra, ca, lda, "A", seen)
+        pb = _matrix_addr(o["B"], rb, cb, ldb, "B", seen)
+        pc = _matrix_addr(o["C"], m, n, ldc, "C", seen)
+        al = complex(o.get("alpha", 1.0))
+        rows.append((pa, pb, pc, m, n, k, lda, ldb, ldc, al.real, al.imag, fl, 0))
+    return rows
 
 
 SPLIT_ROWS = 128  # default split_rows: rows from which a problem counts toward splitting a call
@@ -196,8 +225,9 @@ class Engine:
         if not rows:
             return
         tab = np.array(rows, dtype=nat.SITE_OP)
-        dtab = nat.to_device_table(tab, self.dev)
-        nat.check(self.lib.mpsx_apply_one_site(self.stream, tab.ctypes.data, dtab.data_ptr(),
+        stream = self.stream
+        dtab = nat.put_table(tab, self.dev, stream)
+        nat.check(self.lib.mpsx_apply_one_site(stream, tab.ctypes.data, dtab.data_ptr(),
                                                len(rows)))
         del dtab
 
@@ -264,7 +294,7 @@ class Engine:
         nat.check(self.lib.mpsx_two_site_plan(tab.ctypes.data, n, ctypes.byref(cfg),
                                               ctypes.byref(nbytes)))
         ws = self.workspace(nbytes.value, slot) if workspace else None
-        dtab = nat.to_device_table(tab, self.dev)
+        dtab = nat.put_table(tab, self.dev, self.stream)
         return outs, tab, dtab, ws
 
     def _run_two_site(self, tab, dtab, ws, cfg, stream: int) -> int:
@@ -362,20 +392,9 @@ class Engine:
             for s in range(0, len(ops), MAX_OPS):
                 self.gemm(ops[s:s + MAX_OPS])
             return
-        tab = np.zeros(len(ops), dtype=nat.GEMM_OP)
-        for i, o in enumerate(ops):
-            m, n, k, fl = int(o["m"]), int(o["n"]), int(o["k"]), int(o.get("flags", 0))
-            # stored shapes: op(A) = A^H means A is stored k x m, else m x k
-            ra, ca = (k, m) if fl & nat.GEMM_CONJ_A else (m, k)
-            rb, cb = (n, k) if fl & nat.GEMM_CONJ_B else (k, n)
-            pa = _matrix_addr(o["A"], ra, ca, o["lda"], "A")
-            pb = _matrix_addr(o["B"], rb, cb, o["ldb"], "B")
-            pc = _matrix_addr(o["C"], m, n, o["ldc"], "C")
-            al = complex(o.get("alpha", 1.0))
-            tab[i] = (pa, pb, pc, m, n, k, o["lda"], o["ldb"], o["ldc"], al.real, al.imag, fl, 0)
-        dtab = nat.to_device_table(tab, self.dev)
-        nat.check(self.lib.mpsx_gemm(self.stream, tab.ctypes.data, dtab.data_ptr(), len(ops)))
-        self._last_gemm_table = dtab
+        chain = GemmChain(self)
+        chain.gemm(ops)
+        chain.flush()
 
     # ------------------------------------------------------------ scale
     def scale(self, tensors: Sequence[object], factor: complex, conj: bool = False) -> None:
@@ -385,6 +404,57 @@ class Engine:
         f = complex(factor)
         for i, t in enumerate(tensors):
             tab[i] = (nat.ptr(t), t.numel(), f.real, f.imag, 1 if conj else 0, 0)
-        dtab = nat.to_device_table(tab, self.dev)
-        nat.check(self.lib.mpsx_scale(self.stream, tab.ctypes.data, dtab.data_ptr(), len(tensors)))
+        stream = self.stream
+        dtab = nat.put_table(tab, self.dev, stream)
+        nat.check(self.lib.mpsx_scale(stream, tab.ctypes.data, dtab.data_ptr(), len(tensors)))
         self._last_scale_table = dtab
+
+
+class GemmChain:
+    """Grouped products that depend on one another (the sweeps of the read-outs), in
+    the order they are added: their descriptors travel together, one table for many
+    launches, up to what one launch of mpsx_put carries. The operands of products
+    not yet launched are kept alive, up to KEEP_BYTES of results. flush() launches
+    the rest."""
+
+    TABLE_ROWS = 40         # 3840 bytes of descriptors
+    KEEP_BYTES = 64 << 20
+
+    def __init__(self, eng: Engine):
+        self.eng = eng
+        self._rows: List[tuple] = []
+        self._counts: List[int] = []
+        self._ops: list = []
+        self._bytes = 0
+
+    def gemm(self, ops: Sequence[dict]) -> None:
+        if not ops:
+            return
+        if len(ops) > MAX_OPS:
+            for s in range(0, len(ops), MAX_OPS):
+                self.gemm(ops[s:s + MAX_OPS])
+            return
+        if self._rows and len(self._rows) + len(ops) > self.TABLE_ROWS:
+            self.flush()
+        rows = _gemm_rows(ops)
+        self._rows += rows
+        self._counts.append(len(rows))
+        self._ops.append(ops)
+        self._bytes += 8 * sum(r[3] * r[4] for r in rows)
+        if self._bytes > self.KEEP_BYTES:
+            self.flush()
+
+    def flush(self) -> None:
+        if not self._rows:
+            return
+        eng = self.eng
+        tab = np.array(self._rows, dtype=nat.GEMM_OP)
+        stream = eng.stream
+        dtab = nat.put_table(tab, eng.dev, stream)
+        h, d = tab.ctypes.data, dtab.data_ptr()
+        for c in self._counts:
+            nat.check(eng.lib.mpsx_gemm(stream, h, d, c))
+            h += c * tab.itemsize
+            d += c * tab.itemsize
+        eng._last_gemm_table = dtab
+        self._rows, self._counts, self._ops, self._bytes = [], [], [], 0

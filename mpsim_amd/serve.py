@@ -269,6 +269,9 @@ class MPSServer:
         torch = eng.torch
         stream = torch.cuda.current_stream(eng.dev)
         active: List[Tuple[DeviceCircuit, Served, int]] = []
+        # Two ticks are in flight at most: the calls of a tick do not wait for
+        # the GPU, and a request that arrives joins the next tick enqueued.
+        ended: deque = deque()
 
         def now() -> float:
             return time.perf_counter() - t0
@@ -298,6 +301,10 @@ class MPSServer:
                 eng.split_ways = shared.ways(i)
             tick(eng, [a[0] for a in active], self.svd)
             stats["ticks"] += 1
+            ended.append(torch.cuda.Event())
+            ended[-1].record(stream)
+            if len(ended) > 1:
+                ended.popleft().synchronize()
             finished = [a for a in active if a[0].done]
             if finished:
                 stream.synchronize()

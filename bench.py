@@ -165,8 +165,9 @@ def run_hbm(args, eng, svd):
     kk = nat.profile_read(reset=True)
     ms = sum(kk.get(k, (0.0, 0))[0] for k in ("k_gemm", "k_gemm_rows"))
     nl = sum(kk.get(k, (0.0, 0))[1] for k in ("k_gemm", "k_gemm_rows"))
-    # two-sided roofline per product: max(bytes / HBM peak, flops / FP32 vector
-    # peak without packed FP32, 78.6 TFLOP/s)
+    # two-sided roofline per product: max(bytes / HBM peak, flops / FP32 peak of
+    # the units it runs on: k_gemm the matrix cores, 157.3 TFLOP/s; k_gemm_rows
+    # (k <= 32) the vector units without packed FP32, 78.6)
     by, fl, bound, rows = 0, 0, 0.0, 2
     for i in range(1, nq):
         cl, cr = bonds[i], bonds[i + 1]
@@ -174,7 +175,7 @@ def run_hbm(args, eng, svd):
         f_i = 8 * rows * cl * 2 * cr
         by += b_i
         fl += f_i
-        bound += max(b_i / (PEAK_HBM * 1e9), f_i / 78.6e12)
+        bound += max(b_i / (PEAK_HBM * 1e9), f_i / (78.6e12 if cl <= 32 and 2 * cr <= 256 else 157.3e12))
         rows *= 2
     t = ms / reps * 1e-3
     out["k_gemm_wavefunction"] = {
@@ -183,8 +184,8 @@ def run_hbm(args, eng, svd):
         "tflops": round(fl / t / 1e12, 2),
         "roofline_ms": round(bound * 1e3, 3), "frac_of_roofline": round(bound / t, 3),
         "by_kernel_ms_per_call": {k: round(v[0] / reps, 3) for k, v in kk.items()},
-        "roofline_basis": "sum over the chain's products of max(bytes / 8 TB/s, flops / 78.6 "
-                          "TFLOP/s FP32 vector)"}
+        "roofline_basis": "sum over the chain's products of max(bytes / 8 TB/s, flops / FP32 peak: "
+                          "157.3 TFLOP/s matrix for k_gemm, 78.6 vector for k_gemm_rows)"}
     del mps
 
     # theta and gather of 31 chi=256 updates, as one group (a split call would

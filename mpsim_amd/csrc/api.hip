@@ -321,7 +321,7 @@ int mpsx_gemm(mpsx_stream stream, const mpsx_gemm_op *h, const mpsx_gemm_op *d, 
     }
     if (((max_m + 31) / 32) * ((max_n + 31) / 32) > 2147483647LL)
         return fail(MPSX_EINVAL, "m x n too large for one launch");
-    HIP_TRY(timed("k_gemm", (hipStream_t)stream, [&] { return launch_gemm((hipStream_t)stream, d, count, max_m, max_n); }), "k_gemm");
+    HIP_TRY(timed("k_gemm", (hipStream_t)stream, [&] { return launch_gemm((hipStream_t)stream, h, d, count, max_m, max_n); }), "k_gemm");
     return MPSX_OK;
 }
 

@@ -46,6 +46,29 @@ MPSX_DEV mfma_d4 mfma16d(double a, double b, mfma_d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// The FP32 one: lane l holds A[l % 16][l / 16] and B[l / 16][l % 16];
+// register r of lane l holds D[4 (l / 16) + r][l % 16].
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+MPSX_DEV mfma_f4 mfma16(float a, float b, mfma_f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Loads and stores through a pointer that was itself read from memory (a
+// descriptor's), as global ones: from such a pointer the compiler makes
+// flat accesses, which may be LDS's and are only ever waited for all together.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+#define MPSX_GLOBAL __attribute__((address_space(1)))
+MPSX_DEV float2 gload2(const float2 *p) {
+    const f32x2 v = *(const MPSX_GLOBAL f32x2 *)p;
+    return make_float2(v.x, v.y);
+}
+MPSX_DEV float4 gload4(const float2 *p) {
+    const f32x4 v = *(const MPSX_GLOBAL f32x4 *)p;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+MPSX_DEV void gstore2(float2 *p, float2 v) { *(MPSX_GLOBAL f32x2 *)p = f32x2{v.x, v.y}; }
+
 // Round-robin ("circle method") pairing of n (even) items: in round r
 // (0 <= r < n-1) slot p (0 <= p < n/2) pairs item lo with item hi; every
 // item appears once per round and every unordered pair meets exactly once

@@ -10,7 +10,7 @@ hipError_t launch_one_site(hipStream_t s, const mpsx_site_op *d, int count, int6
                            uint32_t dmask);
 hipError_t launch_put(hipStream_t s, void *dst, const void *src, size_t bytes);
 hipError_t launch_scale(hipStream_t s, const mpsx_scale_op *d, int count, int64_t max_n);
-hipError_t launch_gemm(hipStream_t s, const mpsx_gemm_op *d, int count, int64_t max_m,
+hipError_t launch_gemm(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gemm_op *d, int count, int64_t max_m,
                        int64_t max_n);
 // The tall-narrow variant: every op without conjugation, k <= 32, n <= 256.
 bool gemm_rows_fit(const mpsx_gemm_op &o);

@@ -343,13 +343,7 @@ k_fro(const mpsx_two_site_op *ops, int count, char *ws, double null_rel, int sma
 //   Gram:   G = S S^T,  H = (G11 + G22) + i (G21 - G12)
 //   apply:  [Re Zp'; Im Zp'] = T [Re Zp; Im Zp],  T = [[Ar, -Ai], [Ai, Ar]],
 //           A = Q^H
-// MFMA 16x16x4 operand layout (wave64): lane l holds A[l%16][l/16],
-// B[l/16][l%16]; result register r of lane l is D[4*(l/16)+r][l%16].
-typedef float mfma_f4 __attribute__((ext_vector_type(4)));
-
-MPSX_DEV mfma_f4 mfma16(float a, float b, mfma_f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
+// (mfma16, common.h)
 
 // Rotation parameters of the pivot eigensolve. They sit on the serial path
 // of every step, and the correctly rounded FP64 sqrt, division and rsqrt are

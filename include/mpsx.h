@@ -106,8 +106,8 @@ int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h,
  * to 64 of them, above that the eigenvectors of the rows' Gram matrix, by a
  * direct solver (tridiagonal form, divide and conquer) up to 1024 rows and
  * by Jacobi rounds beyond. theta is formed in
- * complex FP32; by default the rotations are stored and applied in complex
- * FP64 (FP64 matrix cores), which keeps each truncated update as accurate
+ * complex FP64 for d = 2 and 3 (FP32 for other d and with rotation_fp32); by
+ * default the rotations are stored and applied in complex FP64 (FP64 matrix cores), which keeps each truncated update as accurate
  * as a complex64 LAPACK SVD. With rotation_fp32 set they run in FP32
  * (faster, about 1e-6 relative error per update).
  *

@@ -18,8 +18,8 @@
 // divided by a singular value, and the unscaled factor W is exactly unitary
 // also for the zero singular values the reference keeps.
 //
-// Precision: theta is formed in complex FP32 (from the complex64 site
-// tensors). The working matrix Z is complex FP64 by default: Gram matrices
+// Precision: theta is formed from the complex64 site tensors, in FP64 for d = 2
+// and 3 (k_theta64), in FP32 otherwise. The working matrix Z is complex FP64 by default: Gram matrices
 // and rotations run on the FP64 matrix cores, and each update is then as
 // accurate as a complex64 LAPACK SVD. Over the ~10 sweeps of an update
 // every row is rewritten a few hundred times, and an FP32 Z accumulates
@@ -106,6 +106,7 @@ k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n, int sma
 }
 
 // ---------------------------------------------------------------- theta
+// For the FP32 working matrix and D = 4 (FP32 sums on the vector units).
 // One workgroup per 32x32 (l, r) tile; thread (ty, tx) owns l in
 // {ty, ty+16}, r in {tx, tx+16} and all D*D (p1, p2) partial products.
 template <int D, class T>
@@ -211,6 +212,138 @@ k_theta(const mpsx_two_site_op *ops, int count, char *ws) {
                     else
                         Z[col * LD + row] = Cx<T>::make(v.x, v.y);
                 }
+        }
+    }
+}
+
+// theta for D = 2 and 3 and an FP64 working matrix, on the FP64 matrix cores:
+// the complex64 inputs are exact in FP64, so theta carries no rounding of its own (an
+// FP32 sum leaves 1e-7 of it, also in the rows that the gate's rank makes
+// zero, which the solvers then have to resolve). A wave takes 16 l and 16 r of the
+// 32 x 32 tile and all D * D (p1, p2), 16 x 16 products each, so the gate
+// applies in its registers. Fragments come from global memory, PD blocks of 16 m
+// ahead, lane l with m = 4 (l / 16) .. + 3 of a block in its four matrix
+// instructions (the order of m is free): from a 32 bytes a lane, from b 16 lanes a
+// 128-byte line. D = 4 would need 256 accumulator registers.
+// Bound: the matrix instructions of one tile, 27 us at chi_m = 256, D = 2. One
+// update of chi 256 takes 44 us (the FP32 kernel above: 85), 28 of them 250
+// (237), 31 of chi 64 18 (26); a whole update's error against FP64 halves.
+template <int D>
+__global__ void __launch_bounds__(256, D == 2 ? 2 : 1)
+k_theta64(const mpsx_two_site_op *ops, int count, char *ws) {
+    constexpr int PD = D == 2 ? 2 : 1;
+    __shared__ float2 Gs[D * D * D * D];
+    const int pi = find_record(reinterpret_cast<const char *>(ops), count, sizeof(mpsx_two_site_op),
+                               OP_FIELD(plan.tile_base), blockIdx.x);
+    const mpsx_two_site_op &op = ops[pi];
+    if (op.d != D || op.gate == nullptr) return;
+    const int chi_l = op.chi_l, chi_m = op.chi_m, chi_r = op.chi_r;
+    const mpsx_plan p = op.plan;
+    const int tiles_r = (chi_r + THETA_TR - 1) / THETA_TR;
+    const int t = (int)(blockIdx.x - p.tile_base);
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l0 = (t / tiles_r) * THETA_TL + 16 * (wave >> 1), r0 = (t % tiles_r) * THETA_TR + 16 * (wave & 1);
+    for (int i = tid; i < D * D * D * D; i += 256) Gs[i] = gload2(reinterpret_cast<const float2 *>(op.gate) + i);
+    __syncthreads();
+    if (l0 >= chi_l || r0 >= chi_r) return;
+    // l and r beyond the tensors repeat the last (never stored)
+    const float2 *A = reinterpret_cast<const float2 *>(op.a) + (int64_t)min(l0 + l16, chi_l - 1) * D * chi_m;
+    const float2 *B = reinterpret_cast<const float2 *>(op.b) + min(r0 + l16, chi_r - 1);
+    const bool vec = (chi_m & 1) == 0 && (reinterpret_cast<uintptr_t>(op.a) & 15) == 0;
+
+    mfma_d4 re[D][D], im[D][D];
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+        for (int j = 0; j < D; ++j) re[i][j] = im[i][j] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+    float2 fa[PD][D][4], fb[PD][D][4];
+    auto load = [&](int blk, float2 (&x)[D][4], float2 (&y)[D][4]) {
+        const int m = 16 * blk + 4 * q;
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            const float2 *a = A + (int64_t)i * chi_m + m;
+            if (vec) {
+                const float4 u = gload4(a), v = gload4(a + 2);
+                x[i][0] = make_float2(u.x, u.y);
+                x[i][1] = make_float2(u.z, u.w);
+                x[i][2] = make_float2(v.x, v.y);
+                x[i][3] = make_float2(v.z, v.w);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[i][u] = gload2(a + u);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) y[i][u] = gload2(B + ((int64_t)(m + u) * D + i) * chi_r);
+        }
+    };
+    auto multiply = [&](const float2 (&x)[D][4], const float2 (&y)[D][4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < D; ++i)
+#pragma unroll
+                for (int j = 0; j < D; ++j) {
+                    const double ar = x[i][u].x, ai = x[i][u].y, br = y[j][u].x, bi = y[j][u].y;
+                    re[i][j] = mfma16d(ar, br, re[i][j]);
+                    im[i][j] = mfma16d(ar, bi, im[i][j]);
+                    re[i][j] = mfma16d(-ai, bi, re[i][j]);
+                    im[i][j] = mfma16d(ai, br, im[i][j]);
+                }
+    };
+    // whole blocks; a load past the last one repeats that
+    const int blocks = chi_m / 16;
+    if (blocks > 0) {
+#pragma unroll
+        for (int u = 0; u < PD; ++u) load(min(u, blocks - 1), fa[u], fb[u]);
+        int s = 0;
+        for (; s + PD <= blocks; s += PD) {
+#pragma unroll
+            for (int u = 0; u < PD; ++u) {
+                multiply(fa[u], fb[u]);
+                load(min(s + u + PD, blocks - 1), fa[u], fb[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < PD - 1; ++u)
+            if (s + u < blocks) multiply(fa[u], fb[u]);
+    }
+    if (chi_m % 16 != 0) {
+        const int m = 16 * blocks + 4 * q;
+#pragma unroll
+        for (int i = 0; i < D; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool in = m + u < chi_m;
+                fa[0][i][u] = in ? gload2(A + (int64_t)i * chi_m + m + u) : make_float2(0.f, 0.f);
+                fb[0][i][u] = in ? gload2(B + ((int64_t)(m + u) * D + i) * chi_r) : make_float2(0.f, 0.f);
+            }
+        multiply(fa[0], fb[0]);
+    }
+
+    // theta[l, o1, o2, r] = sum G[(o1, o2), (p1, p2)] T[l, p1, p2, r]
+    double2 *Z = z_ptr<double>(ws, p);
+    const int LD = p.LD;
+    const bool transposed = (op.flags & 1) != 0;
+    const int r = r0 + l16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int l = l0 + 4 * e + q;
+        if (l >= chi_l || r >= chi_r) continue;
+#pragma unroll 1
+        for (int o = 0; o < D * D; ++o) {
+            double2 v = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int i = 0; i < D; ++i)
+#pragma unroll
+                for (int j = 0; j < D; ++j) {
+                    const float2 g = Gs[o * D * D + i * D + j];
+                    const double gx = g.x, gy = g.y, tx = re[i][j][e], ty = im[i][j][e];
+                    v.x = fma(gx, tx, fma(-gy, ty, v.x));
+                    v.y = fma(gx, ty, fma(gy, tx, v.y));
+                }
+            const int64_t row = (int64_t)l * D + o / D, col = (int64_t)(o % D) * chi_r + r;
+            Z[transposed ? col * LD + row : row * LD + col] = v;
         }
     }
 }
@@ -1967,8 +2100,18 @@ static hipError_t launch_theta_t(hipStream_t s, int D, const mpsx_two_site_op *d
     const dim3 g((unsigned)tiles), blk(256);
     switch (D) {
         case 1: hipLaunchKernelGGL(k_load<T>, g, blk, 0, s, d, count, ws); break;
-        case 2: hipLaunchKernelGGL((k_theta<2, T>), g, blk, 0, s, d, count, ws); break;
-        case 3: hipLaunchKernelGGL((k_theta<3, T>), g, blk, 0, s, d, count, ws); break;
+        case 2:
+            if constexpr (sizeof(T) == 8)
+                hipLaunchKernelGGL(k_theta64<2>, g, blk, 0, s, d, count, ws);
+            else
+                hipLaunchKernelGGL((k_theta<2, T>), g, blk, 0, s, d, count, ws);
+            break;
+        case 3:
+            if constexpr (sizeof(T) == 8)
+                hipLaunchKernelGGL(k_theta64<3>, g, blk, 0, s, d, count, ws);
+            else
+                hipLaunchKernelGGL((k_theta<3, T>), g, blk, 0, s, d, count, ws);
+            break;
         case 4: hipLaunchKernelGGL((k_theta<4, T>), g, blk, 0, s, d, count, ws); break;
         default: return hipErrorInvalidValue;
     }

@@ -166,12 +166,13 @@ MPSX_DEV unsigned long long peek(const double *at) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// NX: rows a one-workgroup group may have.
-template <int NX>
+// NX: rows a one-workgroup group may have; PW: parts their product with v is
+// summed from.
+template <int NX, int PW>
 struct TriShared {
     double2 v[2][EIG_MAX_N];  // reflectors of the previous and this step
     double2 w[EIG_MAX_N];
-    double2 p[NX], c[NX];     // the exchange of a one-workgroup group
+    double2 p[PW][NX], c[NX];  // the exchange of a one-workgroup group
     double2 red1[8];
     double red2[8];
     double2 xj, al;
@@ -204,12 +205,12 @@ MPSX_DEV double *slot_at(const Slots &s, int array, int i) {
 }
 
 // Step 3 on NL live rows (the last of the NG at r0), and the publication of
-// their entries of column J. MEM: the rows are in memory (A, row stride lda)
+// column J. MEM: the rows are in memory (A, row stride lda)
 // instead of registers.
 template <int CH, int RW, int NL, int NG, bool MEM, class SM>
 MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, const double2 *v, const double2 *w, const double2 *vn,
-                       int lane, const int (&row)[4], double2 (&acc)[4], int t0, int J, int n, bool alone,
-                       SM &sm, const Slots &sl) {
+                       int lane, const int (&row)[4], double2 (&acc)[4], int t0, int J, int n, SM &sm,
+                       const Slots &sl) {
     double2 vi[4], wi[4];
 #pragma unroll
     for (int q = NG - NL; q < NG; ++q) {
@@ -217,6 +218,13 @@ MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, co
         vi[q] = uniform_z(v[r]);
         wi[q] = uniform_z(w[r]);
     }
+    // Column J: up to 256 rows the wave that holds row J writes that,
+    // conjugated, chunk by chunk (the others save the instructions: 10.8
+    // instead of 12.7 thousand cycles a step at n = 256); above, where the row is long
+    // (1.1 us at n = 1024), every row its entry.
+    constexpr bool ROW = CH <= 4;
+    constexpr int qj = NG - NL;  // the only row here that can be row J
+    const bool has_j = ROW && row[qj] == J;
     const int tc = J >> 6, lc = J & 63;
 #pragma unroll
     for (int t = 0; t < CH; ++t) {
@@ -239,8 +247,16 @@ MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, co
             } else {
                 a[r0 + q][t] = x;
             }
+            if (ROW && q == qj && has_j && k >= J && k < n) {
+                if (MEM) {
+                    sm.c[k] = zconj(x);
+                } else {
+                    publish(slot_at(sl, 2, k - J), x.x);
+                    publish(slot_at(sl, 3, k - J), -x.y);
+                }
+            }
         }
-        if (t == tc && lane == lc) {
+        if (!ROW && t == tc && lane == lc) {
 #pragma unroll
             for (int q = NG - NL; q < NG; ++q) {
                 if (row[q] >= n) continue;
@@ -249,7 +265,7 @@ MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, co
                     x = A[row[q] * lda + k];
                 else
                     x = a[r0 + q][t];
-                if (alone) {
+                if (MEM) {
                     sm.c[row[q]] = x;
                 } else {
                     publish(slot_at(sl, 2, row[q] - J), x.x);
@@ -258,6 +274,39 @@ MPSX_DEV void tri_rows(double2 (&a)[RW][CH], double2 *A, int64_t lda, int r0, co
             }
         }
     }
+}
+
+// Step 3 of a one-workgroup group: A is Hermitian, so p' = A v' is summed down the
+// columns, in the lanes, without a reduction across them; the eight waves' parts
+// meet in LDS. Row J, conjugated, is column J.
+template <int RW, int T0, class SM>
+MPSX_DEV void tri_rows_alone(double2 (&a)[RW][2], const double2 *v, const double2 *w, const double2 *vn, int lane,
+                             int wave, int J, int n, SM &sm) {
+    double2 acc[2], vk[2], wk[2];
+#pragma unroll
+    for (int t = T0; t < 2; ++t) {
+        acc[t] = make_double2(0.0, 0.0);
+        vk[t] = v[lane + 64 * t];
+        wk[t] = w[lane + 64 * t];
+    }
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        const int row = 8 * r + wave;
+        if (row < J || row >= n) continue;
+        const double2 vi = v[row], wi = w[row], ni = vn[row];
+#pragma unroll
+        for (int t = T0; t < 2; ++t) {
+            double2 x = a[r][t];
+            x.x = fma(-vi.x, wk[t].x, fma(-vi.y, wk[t].y, fma(-wi.x, vk[t].x, fma(-wi.y, vk[t].y, x.x))));
+            x.y = fma(-vi.y, wk[t].x, fma(vi.x, wk[t].y, fma(-wi.y, vk[t].x, fma(wi.x, vk[t].y, x.y))));
+            acc[t].x = fma(x.x, ni.x, fma(x.y, ni.y, acc[t].x));
+            acc[t].y = fma(x.x, ni.y, fma(-x.y, ni.x, acc[t].y));
+            a[r][t] = x;
+            if (row == J) sm.c[lane + 64 * t] = zconj(x);
+        }
+    }
+#pragma unroll
+    for (int t = T0; t < 2; ++t) sm.p[wave][lane + 64 * t] = acc[t];
 }
 
 // MEM: one workgroup, the matrix copied to the Y rows (which hold no slots
@@ -270,7 +319,9 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
     const int n = p.C, Cp = p.Cp;
     const int tid = threadIdx.x;
     int wave = tid >> 6;
-    const bool alone = G == 1, vec = VW == 8 || wave < VW;
+    constexpr bool LANES = CH == 2 && !MEM;   // a group of one (up to 128 rows)
+    constexpr bool alone = CH == 2 || MEM;
+    const bool vec = VW == 8 || wave < VW;
     double2 *H = eig_h(ws, p);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
@@ -314,6 +365,15 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
     }
     __syncthreads();
     double2 tau = make_double2(0.0, 0.0);
+    // This workgroup's rows of reflector q to its panel: 256 bytes apart, so
+    // that they are shared out and come after what others wait for (one member in turn writing
+    // all of them before its pass cost 0.4 us a step at n = 512). Every
+    // workgroup has read H once the slots of step 1 are full.
+    auto panel = [&](int q, const double2 *v) {
+        for (int i = tid; i < n; i += 512)
+            if (i >= (q & ~15) && (alone || (i >> 3) % G == member))
+                H[(int64_t)(q >> 4) * 16 * Cp + (int64_t)i * 16 + (q & 15)] = v[i];
+    };
     int cur = 0, nref = n - 1;
     for (int j = 0; j < n; ++j) {
         // the lane and the wave through an empty asm statement: addresses are
@@ -327,42 +387,68 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
             double2 dot = make_double2(0.0, 0.0);
             const bool failed = sm.fail != 0;
             const Slots sl = slots_of(y, ld2, Cp, n, j);
+            double2 pv[EPT];
+            if (j == 0 || alone) {
 #pragma unroll
-            for (int s = 0; s < EPT; ++s) {
-                const int i = ti + 64 * VW * s;
-                double2 pv = make_double2(0.0, 0.0);
-                c[s] = make_double2(0.0, 0.0);
-                if (i >= j && i < n) {
+                for (int s = 0; s < EPT; ++s) {
+                    const int i = ti + 64 * VW * s;
+                    pv[s] = make_double2(0.0, 0.0);
+                    c[s] = make_double2(0.0, 0.0);
+                    if (i < j || i >= n) continue;
                     if (j == 0) {
                         c[s] = H[(int64_t)i * Cp];
-                    } else if (alone) {
-                        pv = sm.p[i];
-                        c[s] = sm.c[i];
                     } else {
-                        const double *a0 = slot_at(sl, 0, i - j), *a1 = slot_at(sl, 1, i - j),
-                                     *a2 = slot_at(sl, 2, i - j), *a3 = slot_at(sl, 3, i - j);
-                        unsigned long long b0, b1, b2, b3;
-                        int spin = failed ? kSpin : 0;
-                        while (true) {
-                            b0 = peek(a0);
-                            b1 = peek(a1);
-                            b2 = peek(a2);
-                            b3 = peek(a3);
-                            if (b0 != EIG_EMPTY && b1 != EIG_EMPTY && b2 != EIG_EMPTY && b3 != EIG_EMPTY) break;
-                            if (++spin > kSpin) {
-                                sm.fail = 1;
-                                break;
-                            }
+                        pv[s] = sm.p[0][i];
+                        if constexpr (LANES) {
+#pragma unroll
+                            for (int u = 1; u < 8; ++u) pv[s] = zadd(pv[s], sm.p[u][i]);
                         }
-                        pv = make_double2(__longlong_as_double((long long)b0), __longlong_as_double((long long)b1));
-                        c[s] = make_double2(__longlong_as_double((long long)b2), __longlong_as_double((long long)b3));
+                        c[s] = sm.c[i];
                     }
                 }
-                x[s] = zmul(tau, pv);
+            } else {
+                // all of this thread's slots in each look
+                unsigned long long b[EPT][4];
+                bool here[EPT];
+#pragma unroll
+                for (int s = 0; s < EPT; ++s) {
+                    const int i = ti + 64 * VW * s;
+                    here[s] = i < j || i >= n;
+                    b[s][0] = b[s][1] = b[s][2] = b[s][3] = 0;
+                }
+                int spin = failed ? kSpin : 0;
+                while (true) {
+#pragma unroll
+                    for (int s = 0; s < EPT; ++s)
+                        if (!here[s])
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) b[s][u] = peek(slot_at(sl, u, ti + 64 * VW * s - j));
+                    bool all = true;
+#pragma unroll
+                    for (int s = 0; s < EPT; ++s) {
+                        here[s] = b[s][0] != EIG_EMPTY && b[s][1] != EIG_EMPTY && b[s][2] != EIG_EMPTY &&
+                                  b[s][3] != EIG_EMPTY;
+                        all = all && here[s];
+                    }
+                    if (all) break;
+                    if (++spin > kSpin) {
+                        sm.fail = 1;
+                        break;
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < EPT; ++s) {
+                    pv[s] = make_double2(__longlong_as_double((long long)b[s][0]), __longlong_as_double((long long)b[s][1]));
+                    c[s] = make_double2(__longlong_as_double((long long)b[s][2]), __longlong_as_double((long long)b[s][3]));
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < EPT; ++s) {
+                x[s] = zmul(tau, pv[s]);
                 // conj(x) v
                 dot.x = fma(x[s].x, vown[s].x, fma(x[s].y, vown[s].y, dot.x));
                 dot.y = fma(x[s].x, vown[s].y, fma(-x[s].y, vown[s].x, dot.y));
-                if (i == j) sm.xj = x[s];
+                if (ti + 64 * VW * s == j) sm.xj = x[s];
             }
             double f = fold32(dot.x, dot.y);  // the two halves of the wave
             f = group_sum<16>(fold16(f, f));
@@ -381,7 +467,6 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
             const double2 alpha = zscale(zmul(tau, dot), -0.5);
             const double2 wj = zadd(sm.xj, alpha);  // v_j = 1 for j > 0; zero otherwise
             double nrm = 0.0;
-            const bool writer = j > 0 && member == j % G;
 #pragma unroll
             for (int s = 0; s < EPT; ++s) {
                 const int i = ti + 64 * VW * s;
@@ -393,11 +478,11 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
                 sm.w[i] = (i > j && i < n) ? w : make_double2(0.0, 0.0);
                 if (i > j + 1 && i < n) nrm = fma(col[s].x, col[s].x, fma(col[s].y, col[s].y, nrm));
                 if (i == j + 1) sm.al = col[s];
+                // (one workgroup: reflector j - 1 to its panel from the register)
+                if (LANES && j > 0 && i < n && i >= ((j - 1) & ~15))
+                    H[(int64_t)((j - 1) >> 4) * 16 * Cp + (int64_t)i * 16 + ((j - 1) & 15)] = v;
                 if (i == j) sm.dj = col[s].x;
                 if (member == 0 && i == j && !stop) ev.d[j] = col[s].x;
-                // reflector j - 1 to its panel (every workgroup has read H by now)
-                if (writer && i < n && i >= ((j - 1) & ~15))
-                    H[(int64_t)((j - 1) >> 4) * 16 * Cp + (int64_t)i * 16 + ((j - 1) & 15)] = v;
             }
             nrm = wave_sum64(nrm);
             if (lane == 0) sm.red2[wave] = nrm;
@@ -452,32 +537,39 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
             for (int q = 0; q < NG; ++q) live += row[q] >= J;
             if (live == 0) return;
             if (live == 1)
-                tri_rows<CH, RW, 1, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
+                tri_rows<CH, RW, 1, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, sm, sl);
             else if (live == 2)
-                tri_rows<CH, RW, 2, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
+                tri_rows<CH, RW, 2, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, sm, sl);
             else if (live == 3)
-                tri_rows<CH, RW, (NG < 3 ? NG : 3), NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
+                tri_rows<CH, RW, (NG < 3 ? NG : 3), NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, sm, sl);
             else
-                tri_rows<CH, RW, NG, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, alone, sm, sl);
+                tri_rows<CH, RW, NG, NG, MEM>(a, A, p.LD, g * NG, v, sm.w, vn, lane, row, acc, t0, J, n, sm, sl);
             const double s = wave_sum4(acc);
             const int q = lane >> 4, im = (lane >> 3) & 1;
             const int rq = 8 * (member + G * (g * NG + q)) + wave;
             if ((lane & 7) == 0 && q < NG && rq >= J && rq < n) {
                 if (alone)
-                    (im ? sm.p[rq].y : sm.p[rq].x) = s;
+                    (im ? sm.p[0][rq].y : sm.p[0][rq].x) = s;
                 else
                     publish(slot_at(sl, im, rq - J), s);
             }
         };
-        if constexpr (MEM) {
+        if constexpr (LANES) {
+            if (J < 64)
+                tri_rows_alone<RW, 0>(a, v, sm.w, vn, lane, wave, J, n, sm);
+            else
+                tri_rows_alone<RW, 1>(a, v, sm.w, vn, lane, wave, J, n, sm);
+        } else if constexpr (MEM) {
             for (int g = 0; g < (n + 8 * NG - 1) / (8 * NG); ++g) rows(g);
         } else {
 #pragma unroll
             for (int g = 0; g < RW / NG; ++g) rows(g);
         }
+        if (!LANES && j > 0) panel(j - 1, v);
         cur ^= 1;
         if (alone) __syncthreads();
     }
+    if (!LANES && nref > 0) panel(nref - 1, sm.v[cur]);
     if (member != 0) return;
     if (tid == 0) *ev.nref = nref;
     if (nref < n - 1 || sm.stop)
@@ -524,7 +616,7 @@ k_eig_map(const mpsx_two_site_op *ops, int count, int2 *map, int max_n) {
 
 __global__ void __launch_bounds__(512, 2)
 k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
-    __shared__ TriShared<128> sm;
+    __shared__ TriShared<128, 8> sm;
     if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
     __syncthreads();
     const int slot = sm.slot;
@@ -549,7 +641,7 @@ k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
 // memory: it waits for no other workgroup. The results have the same bits.
 __global__ void __launch_bounds__(512, 2)
 k_tridiag_one(const mpsx_two_site_op *ops, char *ws, int max_n) {
-    __shared__ TriShared<EIG_MAX_N> sm;
+    __shared__ TriShared<EIG_MAX_N, 1> sm;
     const mpsx_plan p = ops[blockIdx.x].plan;
     if (!eig_direct(p, max_n)) return;
     if (!(reinterpret_cast<const ProblemCtl *>(ws + p.ws_off)->group & kGroupLost)) return;

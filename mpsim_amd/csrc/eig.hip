@@ -41,7 +41,8 @@ struct EigVec {
     double2 *tau;        // reflector scalars
     double *dl, *zl;     // per merge: poles and weights of the secular equation
     double *zh, *rt;     // recomputed weights; roots as offsets from a pole
-    int *src, *base;     // row of S^T each new row comes from; pole a root is offset from
+    double *pb;          // pole a root is offset from
+    int *src;            // row of S^T each new row comes from
     int *kn;             // per merge (at index lo): non-deflated count
     double *rho;         // per merge (at index lo)
     int *nref;           // reflectors made
@@ -64,16 +65,16 @@ MPSX_DEV EigVec eig_vec(char *ws, const mpsx_plan &p) {
     v.zh = b + 5 * Cp;
     v.rt = b + 6 * Cp;
     v.rho = b + 7 * Cp;
-    int *i = reinterpret_cast<int *>(b + 8 * Cp);
+    v.pb = b + 8 * Cp;
+    int *i = reinterpret_cast<int *>(b + 9 * Cp);
     v.src = i;
-    v.base = i + Cp;
-    v.kn = i + 2 * Cp;
-    v.nref = i + 3 * Cp;
+    v.kn = i + Cp;
+    v.nref = i + 2 * Cp;
     return v;
 }
-// 256 + 16 + 64 + 12 bytes per padded row and a counter, in a rotation region
+// 256 + 16 + 72 + 8 bytes per padded row and a counter, in a rotation region
 // of 1024 bytes per padded row or a V ring of 2048.
-static_assert(256 + 16 + 64 + 16 <= 1024 && 1024 <= QR_RING * 16 * 16, "the small vectors fit the rotation region");
+static_assert(256 + 16 + 72 + 16 <= 1024 && 1024 <= QR_RING * 16 * 16, "the small vectors fit the rotation region");
 
 MPSX_DEV double2 *eig_h(char *ws, const mpsx_plan &p) {
     return reinterpret_cast<double2 *>(ws + h_off(p));
@@ -708,12 +709,12 @@ k_eig_t(const mpsx_two_site_op *ops, char *ws, int max_n) {
 // Leaves: the eigensystem of every 64 x 64 diagonal block of T, torn at each
 // entry, by six levels of merges in LDS. x: block, y: problem. Also scales T to
 // unit norm (es, d) for the merges above.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(LEAF_THREADS)
 k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
     constexpr int M = LEAF;
     __shared__ double S[M][M + 1], U[M][M + 1];
     __shared__ LeafShared L;
-    __shared__ double red[4];
+    __shared__ double red[8];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
     const int n = p.C, b0 = (int)blockIdx.x * M;
@@ -721,14 +722,14 @@ k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
     const int m = min(M, n - b0), tid = threadIdx.x;
     const EigVec ev = eig_vec(ws, p);
     double mx = 0.0;
-    for (int i = tid; i < n; i += 256) {
+    for (int i = tid; i < n; i += LEAF_THREADS) {
         mx = fmax(mx, fabs(ev.d[i]));
         if (i + 1 < n) mx = fmax(mx, fabs(ev.e[i]));
     }
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
     if ((tid & 63) == 0) red[tid >> 6] = mx;
     __syncthreads();
-    mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    mx = fmax(fmax(fmax(red[0], red[1]), fmax(red[2], red[3])), fmax(fmax(red[4], red[5]), fmax(red[6], red[7])));
     const double scale = mx > 0.0 ? 1.0 / mx : 1.0;
     auto off = [&](int i) { return (i >= 0 && i + 1 < n) ? ev.e[i] * scale : 0.0; };
     if (tid < M) {
@@ -739,12 +740,12 @@ k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
         L.e[tid] = off(i);
         if (i < n) ev.es[i] = off(i);
     }
-    leaf_conquer<256>(m, S, U, L);
+    leaf_conquer(m, S, U, L);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
     // both buffers of S^T: zero outside the block (the merges write their
     // own blocks only)
-    for (int j = tid >> 6; j < m; j += 4)
+    for (int j = tid >> 6; j < m; j += 8)
         for (int r = tid & 63; r < 2 * p.Cp; r += 64) {
             const int rr = r - b0;
             y[(int64_t)(b0 + j) * ld2 + r] = (rr >= 0 && rr < m) ? S[j][rr] : 0.0;
@@ -762,7 +763,7 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
     __shared__ int id[EIG_MAX_N], src[EIG_MAX_N];
     __shared__ int2 rot_i[EIG_MAX_N];
     __shared__ double2 rot_c[EIG_MAX_N];
-    __shared__ int sK, sR;
+    __shared__ int sK, sR, kept[8];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
     const int n = p.C, lo = (int)blockIdx.x * 2 * s;
@@ -806,8 +807,40 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
     }
     __syncthreads();
     const double rho = 2.0 * fabs(ee);
-    if (tid == 0) sK = deflate(m, rho, ds, zs, id, dl, zl, src, dd, rot_i, rot_c, &sR);
-    __syncthreads();
+    // The entries of negligible weight go to the end (in the order deflate() puts
+    // them there); only if two of the others then have to be rotated
+    // together is the serial pass made (0.2 us an entry).
+    int before = 0;
+    for (int b = 0; b < m; b += 512) {
+        const int i = b + tid;
+        const bool keep = i < m && rho * fabs(zs[i]) > kDeflate;
+        const unsigned long long mask = __ballot(keep);
+        if ((tid & 63) == 0) kept[tid >> 6] = __popcll(mask);
+        __syncthreads();
+        int at = before + __popcll(mask & ((1ULL << (tid & 63)) - 1)), all = 0;
+        for (int u = 0; u < 8; ++u) {
+            if (u < (tid >> 6)) at += kept[u];
+            all += kept[u];
+        }
+        if (keep) {
+            dl[at] = ds[i];
+            zl[at] = zs[i];
+            src[at] = id[i];
+        } else if (i < m) {
+            const int e = m - 1 - (i - at);
+            dd[e] = ds[i];
+            src[e] = id[i];
+        }
+        before += all;
+        __syncthreads();
+    }
+    bool some = false;
+    for (int i = tid; i + 1 < before; i += 512) some = some || may_deflate(before, i, rho, dl, zl);
+    if (tid == 0) sK = before;
+    if (__syncthreads_or(some)) {
+        if (tid == 0) sK = deflate(m, rho, ds, zs, id, dl, zl, src, dd, rot_i, rot_c, &sR);
+        __syncthreads();
+    }
     const int K = sK, nr = sR;
     for (int r = tid; r < m; r += 512)
         for (int q = 0; q < nr; ++q) {
@@ -833,148 +866,156 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
     }
 }
 
-// The secular roots of a level's merges, 16 lanes per root: 16 roots per
-// workgroup (x; a merge's 2 s >= 128 rows are whole workgroups), y: problem.
+// (The four kernels of a level at 512 rows, us, with the poles one by one, staged
+// rows and a serial deflation -> now: merge 101 -> 26, roots 41 -> 10, weights 18 -> 5,
+// vectors 66 -> 21.)
+//
+// The secular roots of a level's merges, a wave per root: 4 roots per workgroup
+// (x; all of one merge, whose first row is a multiple of 128), y: problem.
 __global__ void __launch_bounds__(256)
 k_eig_roots(const mpsx_two_site_op *ops, char *ws, int max_n, int s) {
-    __shared__ double dl[EIG_MAX_N], zl[EIG_MAX_N];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
-    const int n = p.C, r0 = (int)blockIdx.x * 16;
-    if (s >= n || r0 >= n) return;
-    const int lo = r0 & ~(2 * s - 1);
+    const int n = p.C, row = (int)blockIdx.x * 4 + wave_id(), sub = threadIdx.x & 63;
+    if (s >= n || row >= n) return;
+    const int lo = row & ~(2 * s - 1), j = row - lo;
     const EigVec ev = eig_vec(ws, p);
     const int K = ev.kn[lo];
-    if (r0 - lo >= K) return;
-    for (int i = threadIdx.x; i < K; i += 256) {
-        dl[i] = ev.dl[lo + i];
-        zl[i] = ev.zl[lo + i];
-    }
-    __syncthreads();
-    const int j = r0 - lo + ((int)threadIdx.x >> 4), sub = threadIdx.x & 15;
     if (j >= K) return;
-    int bs;
+    const double *dl = ev.dl + lo, *zl = ev.zl + lo;
+    double d[EIG_MAX_N / 64], z2[EIG_MAX_N / 64];
+#pragma unroll
+    for (int u = 0; u < EIG_MAX_N / 64; ++u) {
+        const int i = sub + 64 * u;
+        d[u] = 1e200;
+        z2[u] = 0.0;
+        if (64 * u >= K) continue;
+        if (i < K) {
+            const double z = zl[i];
+            d[u] = dl[i];
+            z2[u] = z * z;
+        }
+    }
+    const int nx = min(j + 1, K - 1);
+    const double dj = dl[j], dn = dl[nx];
     double root;
-    secular_root<16>(K, dl, zl, ev.rho[lo], j, sub, &bs, &root);
+    const double pole = secular_root<64, EIG_MAX_N / 64>(K, d, z2, dj, dn, zl[j], zl[nx], ev.rho[lo], j, sub, &root) ? dn : dj;
     if (sub == 0) {
-        ev.base[lo + j] = bs;
-        ev.rt[lo + j] = root;
-        ev.d[lo + j] = dl[bs] + root;
+        ev.pb[row] = pole;
+        ev.rt[row] = root;
+        ev.d[row] = pole + root;
     }
 }
 
-// The recomputed weights, 16 lanes per pole, split as k_eig_roots.
+// The recomputed weights, a wave per pole, split as k_eig_roots.
 __global__ void __launch_bounds__(256)
 k_eig_weights(const mpsx_two_site_op *ops, char *ws, int max_n, int s) {
-    __shared__ double dl[EIG_MAX_N], rt[EIG_MAX_N];
-    __shared__ int base[EIG_MAX_N];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
-    const int n = p.C, r0 = (int)blockIdx.x * 16;
-    if (s >= n || r0 >= n) return;
-    const int lo = r0 & ~(2 * s - 1);
+    const int n = p.C, row = (int)blockIdx.x * 4 + wave_id(), sub = threadIdx.x & 63;
+    if (s >= n || row >= n) return;
+    const int lo = row & ~(2 * s - 1), i = row - lo;
     const EigVec ev = eig_vec(ws, p);
     const int K = ev.kn[lo];
-    if (r0 - lo >= K) return;
-    for (int i = threadIdx.x; i < K; i += 256) {
-        dl[i] = ev.dl[lo + i];
-        rt[i] = ev.rt[lo + i];
-        base[i] = ev.base[lo + i];
-    }
-    __syncthreads();
-    const int i = r0 - lo + ((int)threadIdx.x >> 4), sub = threadIdx.x & 15;
     if (i >= K) return;
-    const double v = zhat<16>(K, dl, base, rt, i, sub);
-    if (sub == 0) ev.zh[lo + i] = copysign(v, ev.zl[lo + i]);
+    double v = group_prod<16>(zhat_factors<64>(K, ev.dl + lo, ev.pb + lo, ev.rt + lo, i, sub));
+    v *= __shfl_xor(v, 16, 64);
+    v *= __shfl_xor(v, 32, 64);
+    if (sub == 0) ev.zh[row] = copysign(sqrt(fmax(v, 0.0)), ev.zl[row]);
 }
 
 // Rows of the merged S^T (buffer buf ^ 1): row j < K is sum_i u_ij S^T[src_i],
 // u_ij = zh_i / (d_i - lambda_j), normalised; the deflated rows are copied. A
-// 64 x 64 tile per workgroup on the FP64 matrix cores, the entries of u formed
-// while they are staged (one division each, repeated by the tile's few
-// column neighbours, instead of a pass over memory). x: row tile * column
-// tiles + column tile of a merge, z: merge, y: problem.
+// wave has 16 rows and 32 columns on the FP64 matrix cores and the entries of u
+// formed in its lanes (lane l poles 4 (l / 16) .. + 3 of a block of 16); the
+// rows of S^T are on their way a block ahead, their indices two. Staged through
+// LDS in 64 x 64 tiles a block of 16 poles took 2 us. x: 64-row tile * column
+// tiles + 32-column tile of a merge, z: merge, y: problem.
 __global__ void __launch_bounds__(256)
 k_eig_vectors(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf) {
-    constexpr int TK = 16;
-    __shared__ double As[64][TK + 1];
-    __shared__ double Bs[TK][64 + 1];
-    __shared__ double nrm[64];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
     const int n = p.C, lo = (int)blockIdx.z * 2 * s;
     if (s >= n || lo >= n) return;
     const int hi = min(lo + 2 * s, n), m = hi - lo;
-    const int ct = (2 * s) / 64, j0 = ((int)blockIdx.x / ct) * 64, c0 = ((int)blockIdx.x % ct) * 64;
+    const int ct = (2 * s) / 32, j0 = ((int)blockIdx.x / ct) * 64, c0 = ((int)blockIdx.x % ct) * 32;
     if (j0 >= m || c0 >= m) return;
     const EigVec ev = eig_vec(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
     const double *in = eig_y(ws, p) + (int64_t)buf * p.Cp + lo;
     double *out = eig_y(ws, p) + (int64_t)(buf ^ 1) * p.Cp + lo;
     const int K = ev.kn[lo];
-    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), l16 = lane & 15, lq = lane >> 4;
-    const int wm = wave >> 1, wn = wave & 1;
-    if (j0 < K) {
-        // thread: row j of the tile, 4 of the 16 poles of a stage
-        const int aj = tid >> 2, ai = (tid & 3) * 4;
-        const bool jok = j0 + aj < K;
-        double db = 0.0, tj = 0.0, nn = 0.0;
-        if (jok) {
-            db = ev.dl[lo + ev.base[lo + j0 + aj]];
-            tj = ev.rt[lo + j0 + aj];
-        }
-        mfma_d4 acc[2][2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-        for (int k0 = 0; k0 < K; k0 += TK) {
+    const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, q = lane >> 4;
+    const int j1 = j0 + 16 * wave_id();  // this wave's rows
+    if (j1 < K) {
+        const int j = min(j1 + l16, K - 1);
+        const double db = ev.pb[lo + j], tj = ev.rt[lo + j];
+        // columns beyond the merge repeat its last (never stored)
+        const double *col[2] = {in + min(c0 + l16, m - 1), in + min(c0 + 16 + l16, m - 1)};
+        const int blocks = (K + 15) / 16;
+        struct Poles {
+            double zh[4], dl[4];
+            int src[4];
+        };
+        auto poles = [&](int b, Poles &x) {  // of block b, or of the last again
+            const int i0 = lo + 16 * min(b, blocks - 1) + 4 * q;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const int i = k0 + ai + t;
-                double u = 0.0;
-                if (jok && i < K) u = ev.zh[lo + i] * recip((ev.dl[lo + i] - db) - tj);
+                const bool on = i0 + t < lo + K;
+                x.zh[t] = on ? ev.zh[i0 + t] : 0.0;
+                x.dl[t] = on ? ev.dl[i0 + t] : 1e200;
+                x.src[t] = on ? ev.src[i0 + t] : lo;
+            }
+        };
+        auto rows = [&](const Poles &x, double (&v)[2][4]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) v[c][t] = col[c][x.src[t] * ld2];
+        };
+        mfma_d4 acc[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+        double nn = 0.0;
+        auto multiply = [&](const Poles &x, const double (&v)[2][4]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const double u = x.zh[t] * recip((x.dl[t] - db) - tj);
                 nn = fma(u, u, nn);
-                As[aj][ai + t] = u;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) acc[c] = mfma16d(u, v[c][t], acc[c]);
             }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int bk = (tid >> 6) + 4 * t, bc = tid & 63;
-                const int i = k0 + bk;
-                Bs[bk][bc] = (i < K && c0 + bc < m) ? in[(int64_t)ev.src[lo + i] * ld2 + c0 + bc] : 0.0;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < TK / 4; ++q) {
-                const int kk = 4 * q + lq;
-                double av[2], bv[2];
-#pragma unroll
-                for (int a = 0; a < 2; ++a) av[a] = As[32 * wm + 16 * a + l16][kk];
-#pragma unroll
-                for (int b = 0; b < 2; ++b) bv[b] = Bs[kk][32 * wn + 16 * b + l16];
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int b = 0; b < 2; ++b) acc[a][b] = mfma16d(av[a], bv[b], acc[a][b]);
-            }
-            __syncthreads();
+        };
+        Poles x0, x1, x2;
+        double v0[2][4], v1[2][4];
+        poles(0, x0);
+        poles(1, x1);
+        rows(x0, v0);
+        for (int b = 0; b < blocks; b += 2) {
+            rows(x1, v1);
+            poles(b + 2, x2);
+            multiply(x0, v0);
+            if (b + 1 >= blocks) break;
+            rows(x2, v0);
+            x0 = x2;
+            poles(b + 3, x2);
+            multiply(x1, v1);
+            x1 = x2;
         }
-        nn = group_sum<4>(nn);
-        if ((tid & 3) == 0) nrm[aj] = jok ? 1.0 / sqrt(nn) : 0.0;
-        __syncthreads();
+        nn += __shfl_xor(nn, 16, 64);
+        nn += __shfl_xor(nn, 32, 64);
+        const double f = 1.0 / sqrt(nn);
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int r = 0; r < 4; ++r) {
+            const int jj = 4 * r + q;
+            const double fj = __shfl(f, jj, 64);
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int jj = 32 * wm + 16 * a + 4 * r + lq, cc = c0 + 32 * wn + 16 * b + l16;
-                    if (j0 + jj < K && cc < m) out[(int64_t)(lo + j0 + jj) * ld2 + cc] = acc[a][b][r] * nrm[jj];
-                }
+            for (int c = 0; c < 2; ++c)
+                if (j1 + jj < K && c0 + 16 * c + l16 < m)
+                    out[(int64_t)(lo + j1 + jj) * ld2 + c0 + 16 * c + l16] = acc[c][r] * fj;
+        }
     }
     if (j0 + 64 > K)  // deflated rows
-        for (int e = tid; e < 64 * 64; e += 256) {
-            const int j = j0 + (e >> 6), cc = c0 + (e & 63);
+        for (int e = tid; e < 64 * 32; e += 256) {
+            const int j = j0 + (e >> 5), cc = c0 + (e & 31);
             if (j >= K && j < m && cc < m) out[(int64_t)(lo + j) * ld2 + cc] = in[(int64_t)ev.src[lo + j] * ld2 + cc];
         }
 }
@@ -984,11 +1025,13 @@ k_eig_vectors(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf) 
 // eigenvector a column) in the matrix-core output layout in registers (eight
 // waves; wave w the 16-row chunks w, w + 8, ...), the panels' block
 // reflectors I - V T V^H from the last to the first. x: strip, y: problem.
-// CH chunks a wave: 4 up to 512 rows, 8 up to 1024. Bound: the three
-// barriers a panel at two workgroups per CU (CH = 4) and the FP64 matrix
-// cores; V is read once per strip, from the L2.
+// CH chunks a wave: 4 up to 512 rows, 8 up to 1024. Registers for two waves a
+// SIMD: for four, CH = 4 spilled (one strip set of 512 rows 333 us, now 274;
+// 28 of them 944, now 990). Bound: the FP64 matrix cores of a strip's one
+// compute unit and the three barriers a panel; V is read once per strip, from
+// the L2.
 template <int CH>
-__global__ void __launch_bounds__(512, CH == 4 ? 4 : 2)
+__global__ void __launch_bounds__(512, 2)
 k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
     __shared__ double2 Wp[8][16][17];
     __shared__ double2 Wt[16][17], Ws[16][17], Ts[16][17];
@@ -1099,15 +1142,15 @@ hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int coun
 
 hipError_t launch_eig_conquer(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n) {
     const unsigned y = (unsigned)count;
-    hipLaunchKernelGGL(k_eig_leaf, dim3((unsigned)((n + 63) / 64), y), dim3(256), 0, s, d, ws, max_n);
+    hipLaunchKernelGGL(k_eig_leaf, dim3((unsigned)((n + 63) / 64), y), dim3(LEAF_THREADS), 0, s, d, ws, max_n);
     int buf = 0;
     for (int h = 64; h < n; h *= 2, buf ^= 1) {
         const unsigned nodes = (unsigned)((n + 2 * h - 1) / (2 * h)), tiles = (unsigned)(2 * h / 64);
-        const unsigned roots = (unsigned)((n + 15) / 16);
+        const unsigned roots = (unsigned)((n + 3) / 4);
         hipLaunchKernelGGL(k_eig_merge, dim3(nodes, y), dim3(512), 0, s, d, ws, max_n, h, buf, h == 64 ? 1 : 0);
         hipLaunchKernelGGL(k_eig_roots, dim3(roots, y), dim3(256), 0, s, d, ws, max_n, h);
         hipLaunchKernelGGL(k_eig_weights, dim3(roots, y), dim3(256), 0, s, d, ws, max_n, h);
-        hipLaunchKernelGGL(k_eig_vectors, dim3(tiles * tiles, y, nodes), dim3(256), 0, s, d, ws, max_n, h, buf);
+        hipLaunchKernelGGL(k_eig_vectors, dim3(2 * tiles * tiles, y, nodes), dim3(256), 0, s, d, ws, max_n, h, buf);
     }
     return hipGetLastError();
 }

@@ -180,61 +180,92 @@ MPSX_DEV double recip(double x) {
     return fma(r, fma(-x, r, 1.0), r);
 }
 
+// A lane's value as a wave-uniform one.
+MPSX_DEV double lane_f64(double x, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                            __builtin_amdgcn_readlane(__double2loint(x), lane));
+}
+
 // Root j of 1 + rho sum_i z_i^2 / (d_i - lambda), 0 <= j < K, by L lanes (sub
-// = lane in the group): lambda = dl[base] + tau with base the nearer of the
-// two poles around it, so that every difference d_i - lambda is accurate.
-template <int L>
-MPSX_DEV void secular_root(int K, const double *dl, const double *zl, double rho, int j, int sub, int *base,
-                           double *root) {
+// = lane in the group): lambda = d_org + root with org the nearer of the two
+// poles around it, so that every difference d_i - lambda is accurate. A lane
+// has the poles sub, sub + L, ... and their squared weights in registers (far
+// away and zero beyond K) and works on four at a time: one by one from LDS, the
+// chain of a reciprocal took 440 cycles a pole. d is shifted by the origin.
+// dj, dn, zj, zn: pole j and j + 1 and their weights. Returns org - j.
+template <int L, int U>
+MPSX_DEV int secular_root(int K, double (&d)[U], const double (&z2)[U], double dj, double dn, double zj, double zn,
+                          double rho, int j, int sub, double *root) {
+    static_assert(U % 4 == 0 && (L == 8 || L == 64), "poles a lane");
     const bool last = j == K - 1;
-    const double dj = dl[j];
-    int org = j;
+    int org = 0;
     double lo, hi, t;
+    auto sum = [](double x) { return L == 64 ? wave_sum64(x) : group_sum<8>(x); };
     if (last) {
         double s = 0.0;
-        for (int i = sub; i < K; i += L) s = fma(zl[i], zl[i], s);
-        s = group_sum<L>(s);
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += z2[u];
+        s = sum(s);
         lo = 0.0;
         hi = rho * s * (1.0 + 4.0 * kEps);
         t = K == 1 ? rho * s : 0.5 * hi;
     } else {
-        const double gap = dl[j + 1] - dj, mid = 0.5 * gap;
+        const double gap = dn - dj, mid = 0.5 * gap;
         double c0 = 0.0;
-        for (int i = sub; i < K; i += L) {
-            if (i == j || i == j + 1) continue;
-            c0 = fma(zl[i] * zl[i], recip((dl[i] - dj) - mid), c0);
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += 4) {
+            if (L * u0 >= K) break;
+#pragma unroll
+            for (int u = u0; u < u0 + 4; ++u) {
+                const int i = sub + L * u;
+                const double q = z2[u] * recip((d[u] - dj) - mid);
+                c0 += (i == j || i == j + 1) ? 0.0 : q;
+            }
         }
-        c0 = group_sum<L>(c0);
-        const double s = rho * zl[j] * zl[j], v = rho * zl[j + 1] * zl[j + 1], c = fma(rho, c0, 1.0);
+        c0 = sum(c0);
+        const double s = rho * zj * zj, v = rho * zn * zn, c = fma(rho, c0, 1.0);
         const bool left = c + (v - s) / mid >= 0.0;
-        org = left ? j : j + 1;
+        org = left ? 0 : 1;
         lo = left ? 0.0 : -mid;
         hi = left ? mid : 0.0;
         // c + s / (p1 - t) + v / (p2 - t) = 0 with the poles at 0 and +-gap
         const double A = left ? fma(c, gap, s + v) : fma(-c, gap, s + v);
         const double B = left ? s * gap : -v * gap;
         const double sq = sqrt(fmax(fma(A, A, -4.0 * c * B), 0.0));
-        t = A > 0.0 ? 2.0 * B / (A + sq) : (A - sq) / (2.0 * c);
+        t = A > 0.0 ? 2.0 * B * recip(A + sq) : (A - sq) * recip(2.0 * c);
     }
     if (K > 1) {
         if (!(t > lo && t < hi)) t = 0.5 * (lo + hi);
-        const double dorg = dl[org], p1 = dj - dorg, p2 = last ? 0.0 : dl[j + 1] - dorg;
+        const double dorg = org ? dn : dj, p1 = dj - dorg, p2 = last ? 0.0 : dn - dorg;
+#pragma unroll
+        for (int u = 0; u < U; ++u) d[u] -= dorg;
         for (int it = 0; it < 64; ++it) {
             double psi = 0.0, dpsi = 0.0, phi = 0.0, dphi = 0.0;
-            for (int i = sub; i < K; i += L) {
-                const double r = recip((dl[i] - dorg) - t), q = zl[i] * zl[i] * r, dq = q * r;
-                if (i <= j) {
-                    psi += q;
-                    dpsi += dq;
-                } else {
-                    phi += q;
-                    dphi += dq;
+#pragma unroll
+            for (int u0 = 0; u0 < U; u0 += 4) {
+                if (L * u0 >= K) break;
+#pragma unroll
+                for (int u = u0; u < u0 + 4; ++u) {
+                    const double zl = sub + L * u <= j ? z2[u] : 0.0, zr = z2[u] - zl;
+                    const double r = recip(d[u] - t), ql = zl * r, qr = zr * r;
+                    psi += ql;
+                    phi += qr;
+                    dpsi = fma(ql, r, dpsi);
+                    dphi = fma(qr, r, dphi);
                 }
             }
-            psi = rho * group_sum<L>(psi);
-            phi = rho * group_sum<L>(phi);
-            dpsi = rho * group_sum<L>(dpsi);
-            dphi = rho * group_sum<L>(dphi);
+            if (L == 64) {
+                const double f = group_sum<16>(fold16(fold32(psi, phi), fold32(dpsi, dphi)));
+                psi = rho * lane_f64(f, 0);
+                dpsi = rho * lane_f64(f, 16);
+                phi = rho * lane_f64(f, 32);
+                dphi = rho * lane_f64(f, 48);
+            } else {
+                psi = rho * group_sum<8>(psi);
+                phi = rho * group_sum<8>(phi);
+                dpsi = rho * group_sum<8>(dpsi);
+                dphi = rho * group_sum<8>(dphi);
+            }
             const double g = 1.0 + psi + phi;
             if (fabs(g) <= kEps * (8.0 * (1.0 + fabs(psi) + fabs(phi)) + fabs(t) * (dpsi + dphi))) break;
             if (g < 0.0)
@@ -244,15 +275,15 @@ MPSX_DEV void secular_root(int K, const double *dl, const double *zl, double rho
             double tn;
             if (last) {
                 // c - s / t = 0 through the pole at the origin
-                tn = dpsi * t * t / fma(dpsi, t, g);
+                tn = dpsi * t * t * recip(fma(dpsi, t, g));
             } else {
                 const double D1 = p1 - t, D2 = p2 - t;
                 const double s = dpsi * D1 * D1, v = dphi * D2 * D2, c = g - dpsi * D1 - dphi * D2;
                 const double A = fma(c, D1 + D2, s + v), B = D1 * D2 * g;
                 const double sq = sqrt(fmax(fma(A, A, -4.0 * c * B), 0.0));
                 const double q = 0.5 * (A + copysign(sq, A));
-                double eta = B / q;  // of the two roots, the one between the poles
-                if (!(eta > D1 && eta < D2)) eta = q / c;
+                double eta = B * recip(q);  // of the two roots, the one between the poles
+                if (!(eta > D1 && eta < D2)) eta = q * recip(c);
                 tn = t + eta;
             }
             if (!(tn > lo && tn < hi)) tn = 0.5 * (lo + hi);
@@ -260,151 +291,169 @@ MPSX_DEV void secular_root(int K, const double *dl, const double *zl, double rho
             t = tn;
         }
     }
-    *base = org;
     *root = t;
+    return org;
 }
 
-// |z_i| for which the computed roots are the exact ones (Gu & Eisenstat), by
-// L lanes.
+// |z_i| for which the computed roots are the exact ones (Gu & Eisenstat): the
+// factors sub, sub + L, ... of its square. pb, rt: pole and offset of a root.
 template <int L>
-MPSX_DEV double zhat(int K, const double *dl, const int *base, const double *rt, int i, int sub) {
+MPSX_DEV double zhat_factors(int K, const double *dl, const double *pb, const double *rt, int i, int sub) {
     const double di = dl[i];
     double pr = 1.0;
+#pragma unroll 4
     for (int j = sub; j < K; j += L) {
-        const double num = (dl[base[j]] - di) + rt[j];
+        const double num = (pb[j] - di) + rt[j];
         const double den = j < i ? dl[j] - di : (j < K - 1 ? dl[j + 1] - di : 1.0);
-        pr *= num / den;
+        pr *= num * recip(den);
     }
-    return sqrt(fmax(group_prod<L>(pr), 0.0));
+    return pr;
 }
 
 // The eigensystem of a tridiagonal block of m <= 64 rows, torn at every entry.
-constexpr int LEAF = 64;
+constexpr int LEAF = 64, LEAF_THREADS = 512;
 struct LeafShared {
     double d[LEAF], e[LEAF];  // in: the torn diagonal and the off-diagonal, scaled; out: the eigenvalues in d
-    double z[LEAF], ds[LEAF], zs[LEAF], dl[LEAF], zl[LEAF], dd[LEAF], zh[LEAF], rt[LEAF];
-    int id[LEAF], src[LEAF], base[LEAF], kn[LEAF], nrot[LEAF];
+    double ds[LEAF], zs[LEAF], dl[LEAF], zl[LEAF], dd[LEAF], zh[LEAF], rt[LEAF], pb[LEAF];
+    int id[LEAF], src[LEAF], kn[LEAF], nrot[LEAF];
     int2 rot_i[LEAF];
     double2 rot_c[LEAF];
 };
-// Merges of 1, 2, 4, ... rows in LDS by a workgroup of NT threads (a multiple
-// of 256); on return row j of S is eigenvector j. L.d and L.e are written by
+// Merges of 1, 2, 4, ... rows in LDS by a workgroup of LEAF_THREADS, eight
+// lanes a row; on return row j of S is eigenvector j. L.d and L.e are written by
 // the first LEAF threads before the call.
-template <int NT>
+// Bound: latency, about 8 us a level (18 with the poles one by one and the
+// rows on the vector units).
 MPSX_DEV void leaf_conquer(int m, double (*S)[LEAF + 1], double (*U)[LEAF + 1], LeafShared &L) {
     constexpr int M = LEAF;
-    const int tid = threadIdx.x;
-    for (int e = tid; e < M * M; e += NT) S[e >> 6][e & 63] = (e >> 6) == (e & 63) ? 1.0 : 0.0;
+    const int tid = threadIdx.x, g = tid >> 3, sub = tid & 7;
+    for (int e = tid; e < M * M; e += LEAF_THREADS) S[e >> 6][e & 63] = (e >> 6) == (e & 63) ? 1.0 : 0.0;
     __syncthreads();
     for (int s = 1; s < m; s <<= 1) {
         const int h = 2 * s;
-        // the first threads serve one index each: index tid, its merge [lo, hi)
-        const int lo = tid & ~(h - 1), mid = lo + s, hi = min(lo + h, m);
-        const bool merge = tid < m && mid < hi;
-        const double ee = merge ? L.e[mid - 1] : 0.0;
-        if (tid < m)
-            L.z[tid] = merge ? S[tid][tid < mid ? mid - 1 : mid] *
-                                   (tid >= mid && ee < 0.0 ? -0.7071067811865476 : 0.7071067811865476)
-                             : 0.0;
-        __syncthreads();
-        if (tid < m) {
-            const double key = sort_key(L.d[tid]);
+        // index g, its merge [lo, hi)
+        const int lo = g & ~(h - 1), mid = lo + s, hi = min(lo + h, m), gj = g - lo;
+        const double ee = mid < hi ? L.e[mid - 1] : 0.0, rho = 2.0 * fabs(ee);
+        if (g < m) {
+            const double dg = L.d[g], key = sort_key(dg);
             int rank = 0;
-            for (int o = lo; o < hi; ++o) {
+            for (int o = lo + sub; o < hi; o += 8) {
                 const double ko = sort_key(L.d[o]);
-                rank += (ko < key) || (ko == key && o < tid);
+                rank += (ko < key) || (ko == key && o < g);
             }
-            L.ds[lo + rank] = L.d[tid];
-            L.zs[lo + rank] = L.z[tid];
-            L.id[lo + rank] = tid;
+            rank += __builtin_amdgcn_mov_dpp(rank, 0xB1, 0xf, 0xf, true);
+            rank += __builtin_amdgcn_mov_dpp(rank, 0x4E, 0xf, 0xf, true);
+            rank += __builtin_amdgcn_mov_dpp(rank, 0x141, 0xf, 0xf, true);
+            if (sub == 0) {
+                L.ds[lo + rank] = dg;
+                L.zs[lo + rank] = mid < hi ? S[g][g < mid ? mid - 1 : mid] *
+                                                 (g >= mid && ee < 0.0 ? -0.7071067811865476 : 0.7071067811865476)
+                                           : 0.0;
+                L.id[lo + rank] = g;
+                if (gj == 0) L.kn[lo] = hi - lo;  // until something deflates
+            }
         }
-        if (tid < m && tid == lo) L.kn[lo] = hi - lo;  // until something deflates
         __syncthreads();
-        if (tid < m) {
-            if (may_deflate(hi - lo, tid - lo, 2.0 * fabs(ee), L.ds + lo, L.zs + lo)) L.kn[lo] = -1;
-            L.dl[tid] = L.ds[tid];
-            L.zl[tid] = L.zs[tid];
-            L.src[tid] = L.id[tid];
-            if (tid == lo) L.nrot[lo] = 0;
+        if (sub == 0) {
+            if (g < m) {
+                if (may_deflate(hi - lo, gj, rho, L.ds + lo, L.zs + lo)) L.kn[lo] = -1;
+                L.dl[g] = L.ds[g];
+                L.zl[g] = L.zs[g];
+                L.src[g] = L.id[g];
+                if (gj == 0) L.nrot[lo] = 0;
+            } else {
+                L.src[g] = g;
+            }
         }
         __syncthreads();
-        if (tid < m && tid == lo && L.kn[lo] < 0)
-            L.kn[lo] = deflate(hi - lo, 2.0 * fabs(ee), L.ds + lo, L.zs + lo, L.id + lo, L.dl + lo, L.zl + lo,
+        if (sub == 0 && g < m && gj == 0 && L.kn[lo] < 0)
+            L.kn[lo] = deflate(hi - lo, rho, L.ds + lo, L.zs + lo, L.id + lo, L.dl + lo, L.zl + lo,
                                L.src + lo, L.dd + lo, L.rot_i + lo, L.rot_c + lo, &L.nrot[lo]);
         __syncthreads();
-        if (tid < m) {  // component tid of the merge's rows
-            for (int r = 0; r < L.nrot[lo]; ++r) {
-                const int2 ab = L.rot_i[lo + r];
-                const double2 cs = L.rot_c[lo + r];
+        if (tid < m) {  // component tid of its merge's rows
+            const int tlo = tid & ~(h - 1);
+            for (int r = 0; r < L.nrot[tlo]; ++r) {
+                const int2 ab = L.rot_i[tlo + r];
+                const double2 cs = L.rot_c[tlo + r];
                 const double xa = S[ab.x][tid], xb = S[ab.y][tid];
                 S[ab.x][tid] = cs.x * xa + cs.y * xb;
                 S[ab.y][tid] = cs.x * xb - cs.y * xa;
             }
         }
-        // four lanes per root
-        const int g = tid >> 2, sub = tid & 3;
-        const int glo = g & ~(h - 1), gmid = glo + s, gj = g - glo;
-        const int K = g < m ? L.kn[glo] : 0;
+        const int K = g < m ? L.kn[lo] : 0;
+        double db = 0.0, tj = 0.0;
         if (gj < K) {
-            int bs;
-            double root;
-            secular_root<4>(K, L.dl + glo, L.zl + glo, 2.0 * fabs(L.e[gmid - 1]), gj, sub, &bs, &root);
+            double d[8], z2[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int i = sub + 8 * u;
+                d[u] = i < K ? L.dl[lo + i] : 1e200;
+                const double z = i < K ? L.zl[lo + i] : 0.0;
+                z2[u] = z * z;
+            }
+            const int nx = min(gj + 1, K - 1);
+            const double dj = L.dl[g], dn = L.dl[lo + nx];
+            db = secular_root<8, 8>(K, d, z2, dj, dn, L.zl[g], L.zl[lo + nx], rho, gj, sub, &tj) ? dn : dj;
             if (sub == 0) {
-                L.base[g] = bs;
-                L.rt[g] = root;
+                L.pb[g] = db;
+                L.rt[g] = tj;
             }
         }
         __syncthreads();
         if (gj < K) {
-            const double v = zhat<4>(K, L.dl + glo, L.base + glo, L.rt + glo, gj, sub);
-            if (sub == 0) L.zh[g] = copysign(v, L.zl[g]);
+            const double v = group_prod<8>(zhat_factors<8>(K, L.dl + lo, L.pb + lo, L.rt + lo, gj, sub));
+            if (sub == 0) L.zh[g] = copysign(sqrt(fmax(v, 0.0)), L.zl[g]);
         }
         __syncthreads();
-        if (gj < K) {
-            const double db = L.dl[glo + L.base[g]], tj = L.rt[g];
-            double nn = 0.0;
-            for (int i = sub; i < K; i += 4) {
-                const double u = L.zh[glo + i] * recip((L.dl[glo + i] - db) - tj);
-                U[g][i] = u;
-                nn = fma(u, u, nn);
+        // Row g of the blocks of max(h, 16) columns that multiply the old rows:
+        // u over the merge's poles, a unit vector for a deflated row, zero elsewhere.
+        const int hb = max(h, 16), off = lo & (hb - 1);
+        {
+            double u[8], nn = 0.0;
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const int i = sub + 8 * t - off;
+                u[t] = 0.0;
+                if (8 * t < hb && gj < K) {
+                    if (i >= 0 && i < K) u[t] = L.zh[lo + i] * recip((L.dl[lo + i] - db) - tj);
+                    nn = fma(u[t], u[t], nn);
+                }
             }
-            nn = group_sum<4>(nn);
-            const double f = 1.0 / sqrt(nn);
-            for (int i = sub; i < K; i += 4) U[g][i] *= f;
+            nn = group_sum<8>(nn);
+            const double f = gj < K ? 1.0 / sqrt(nn) : 0.0;
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                if (8 * t < hb) U[g][sub + 8 * t] = gj < K ? u[t] * f : (sub + 8 * t - off == gj ? 1.0 : 0.0);
+        }
+        const double dn = g < m ? (gj < K ? db + tj : L.dd[g]) : 0.0;
+        __syncthreads();
+        // New rows = U (old rows in the order of src) on the matrix cores, block by
+        // block: hb / 16 squared tiles a block, hb / 4 in all, two at most a wave.
+        const int lane = tid & 63, wave = wave_id(), l16 = lane & 15, q = lane >> 4;
+        const int tb = hb / 16, per = tb * tb;
+        mfma_d4 acc[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const int t = wave + 8 * w;
+            acc[w] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+            if (t >= hb / 4) continue;
+            const int b0 = (t / per) * hb, ti = (t % per) / tb, tj2 = (t % per) % tb;
+            for (int k = 0; k < hb; k += 16)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    acc[w] = mfma16d(U[b0 + 16 * ti + l16][k + 4 * v + q],
+                                     S[L.src[b0 + k + 4 * v + q]][b0 + 16 * tj2 + l16], acc[w]);
         }
         __syncthreads();
-        // The new rows, held in registers until every old row has been read:
-        // thread (wave, lane r) the rows wave, wave + NT / 64, ... of column
-        // r's merge (the columns outside a merge stay zero), so that a pole
-        // costs one read of S and a broadcast of u for each row.
-        constexpr int W = NT / 64;
-        const int r = tid & 63, wv = wave_id(), rlo = r & ~(h - 1);
-        const int Kr = r < m ? L.kn[rlo] : 0, nr = r < m ? min(h, m - rlo) : 0;
-        double v[M / W];
 #pragma unroll
-        for (int t = 0; t < M / W; ++t) v[t] = 0.0;
-#pragma unroll 4
-        for (int i = 0; i < Kr; ++i) {
-            const double x = S[L.src[rlo + i]][r];
+        for (int w = 0; w < 2; ++w) {
+            const int t = wave + 8 * w;
+            if (t >= hb / 4) continue;
+            const int b0 = (t / per) * hb, ti = (t % per) / tb, tj2 = (t % per) % tb;
 #pragma unroll
-            for (int t = 0; t < M / W; ++t) {
-                if (W * t >= h) break;
-                v[t] = fma(U[(rlo + wv + W * t) & (M - 1)][i], x, v[t]);
-            }
+            for (int r = 0; r < 4; ++r) S[b0 + 16 * ti + 4 * r + q][b0 + 16 * tj2 + l16] = acc[w][r];
         }
-#pragma unroll
-        for (int t = 0; t < M / W; ++t) {
-            const int jj = wv + W * t;
-            if (jj >= Kr && jj < nr) v[t] = S[L.src[rlo + jj]][r];  // deflated: copied
-        }
-        const double dn = tid < m ? ((tid - lo) < L.kn[lo] ? L.dl[lo + L.base[tid]] + L.rt[tid] : L.dd[tid]) : 0.0;
-        __syncthreads();
-#pragma unroll
-        for (int t = 0; t < M / W; ++t) {
-            const int jj = wv + W * t;
-            if (jj < nr) S[rlo + jj][r] = v[t];
-        }
-        if (tid < m) L.d[tid] = dn;
+        if (sub == 0 && g < m) L.d[g] = dn;
         __syncthreads();
     }
 }

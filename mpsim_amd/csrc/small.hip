@@ -35,7 +35,7 @@
 namespace {
 
 constexpr int SN = 64;    // rows
-constexpr int ST = 512;   // threads
+constexpr int ST = LEAF_THREADS;  // 512
 constexpr int SW = ST / 64;
 
 struct SmallShared {
@@ -60,10 +60,6 @@ struct SmallShared {
     int any, nref;
 };
 
-MPSX_DEV double lane_f64(double x, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
-                            __builtin_amdgcn_readlane(__double2loint(x), lane));
-}
 MPSX_DEV double2 lane_z(double2 v, int lane) { return make_double2(lane_f64(v.x, lane), lane_f64(v.y, lane)); }
 
 // H = X X^H from the rows of Z, both triangles. Wave w forms the 16 x 16 tiles
@@ -523,7 +519,7 @@ k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int 
                 sm.L.e[tid] = ev * f;
                 sm.L.d[tid] = dv * f - fabs(ev * f) - (tid > 0 ? fabs(below * f) : 0.0);
             }
-            leaf_conquer<ST>(m, sm.S, sm.U, sm.L);
+            leaf_conquer(m, sm.S, sm.U, sm.L);
             small_back(m, sm);
         } else if (m <= 8) {
             small_jacobi8(m, sm, null2, 0.01 * tol);

@@ -710,14 +710,26 @@ k_eig_t(const mpsx_two_site_op *ops, char *ws, int max_n) {
 // entry, by six levels of merges in LDS. x: block, y: problem. Also scales T to
 // unit norm (es, d) for the merges above.
 __global__ void __launch_bounds__(LEAF_THREADS)
-k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
+k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n, int leaves) {
     constexpr int M = LEAF;
     __shared__ double S[M][M + 1], U[M][M + 1];
     __shared__ LeafShared L;
     __shared__ double red[8];
     const mpsx_plan p = ops[blockIdx.y].plan;
     if (!eig_direct(p, max_n)) return;
-    const int n = p.C, b0 = (int)blockIdx.x * M;
+    const int n = p.C;
+    if ((int)blockIdx.x >= leaves) {
+        // both buffers of S^T are zero outside the leaves' blocks (the merges
+        // write their own blocks only): eight rows a workgroup
+        const int row = 8 * ((int)blockIdx.x - leaves) + (threadIdx.x >> 6);
+        if (row >= n) return;
+        double *yr = eig_y(ws, p) + (int64_t)row * 2 * p.LD;
+        const int l0 = row & ~(M - 1);
+        for (int r = threadIdx.x & 63; r < 2 * p.Cp; r += 64)
+            if (r < l0 || r >= min(l0 + M, n)) yr[r] = 0.0;
+        return;
+    }
+    const int b0 = (int)blockIdx.x * M;
     if (b0 >= n) return;
     const int m = min(M, n - b0), tid = threadIdx.x;
     const EigVec ev = eig_vec(ws, p);
@@ -743,13 +755,10 @@ k_eig_leaf(const mpsx_two_site_op *ops, char *ws, int max_n) {
     leaf_conquer(m, S, U, L);
     double *y = eig_y(ws, p);
     const int64_t ld2 = 2 * (int64_t)p.LD;
-    // both buffers of S^T: zero outside the block (the merges write their
-    // own blocks only)
-    for (int j = tid >> 6; j < m; j += 8)
-        for (int r = tid & 63; r < 2 * p.Cp; r += 64) {
-            const int rr = r - b0;
-            y[(int64_t)(b0 + j) * ld2 + r] = (rr >= 0 && rr < m) ? S[j][rr] : 0.0;
-        }
+    for (int j = tid >> 6; j < m; j += 8) {
+        const int rr = tid & 63;
+        if (rr < m) y[(int64_t)(b0 + j) * ld2 + b0 + rr] = S[j][rr];
+    }
     if (tid < m) ev.rt[b0 + tid] = L.d[tid];
 }
 
@@ -1142,7 +1151,9 @@ hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int coun
 
 hipError_t launch_eig_conquer(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n) {
     const unsigned y = (unsigned)count;
-    hipLaunchKernelGGL(k_eig_leaf, dim3((unsigned)((n + 63) / 64), y), dim3(LEAF_THREADS), 0, s, d, ws, max_n);
+    const int leaves = (n + 63) / 64;
+    hipLaunchKernelGGL(k_eig_leaf, dim3((unsigned)(leaves + (n + 7) / 8), y), dim3(LEAF_THREADS), 0, s, d, ws, max_n,
+                       leaves);
     int buf = 0;
     for (int h = 64; h < n; h *= 2, buf ^= 1) {
         const unsigned nodes = (unsigned)((n + 2 * h - 1) / (2 * h)), tiles = (unsigned)(2 * h / 64);

@@ -1988,11 +1988,11 @@ __global__ void k_sweep_end(const mpsx_two_site_op *ops, int count, char *ws, in
 // One workgroup per problem: stable descending order of the row norms
 // (ties keep the lower row index), singular values, discarded weight, and
 // a count of problems left unconverged (when `unconverged` is not null).
-constexpr int SORT_LDS = 4096;
-__global__ void __launch_bounds__(256)
+constexpr int SORT_LDS = 4096, SORT_THREADS = 1024;
+__global__ void __launch_bounds__(SORT_THREADS)
 k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int small) {
     __shared__ double sg[SORT_LDS];
-    __shared__ double red[4];
+    __shared__ double red[SORT_THREADS / 64];
     const int pi = blockIdx.x;
     if (pi >= count) return;
     const mpsx_two_site_op &op = ops[pi];
@@ -2003,32 +2003,52 @@ k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int s
     int *perm = perm_ptr(ws, p);
     const bool in_lds = C <= SORT_LDS;
     if (in_lds)
-        for (int i = threadIdx.x; i < C; i += 256) sg[i] = sort_key(sig[i]);
+        for (int i = threadIdx.x; i < C; i += SORT_THREADS) sg[i] = sort_key(sig[i]);
     __syncthreads();
     double disc = 0.0;
-    for (int i = threadIdx.x; i < C; i += 256) {
-        const double si = in_lds ? sg[i] : sort_key(sig[i]);
-        int rank = 0;
-        // sixteen LDS reads in flight (one at a time: 64 us for 512 rows, 246 for 1024)
-        if (in_lds) {
+    if (in_lds) {
+        // eight lanes a row up to 128 rows, ..., one above 512; sixteen LDS reads in
+        // flight: 25 us for 512 rows and 85 for 1024, bound by the LDS reads
+        // (256 threads, one read at a time: 64 and 246)
+        int lanes = 1;
+        while (lanes < 8 && 2 * lanes * C <= SORT_THREADS) lanes *= 2;
+        const int sub = threadIdx.x & (lanes - 1);
+        for (int e = threadIdx.x; e < lanes * C; e += SORT_THREADS) {
+            const int i = e / lanes;
+            const double si = sg[i];
+            int rank = 0;
 #pragma unroll 16
-            for (int j = 0; j < C; ++j) rank += (sg[j] > si) || (sg[j] == si && j < i);
-        } else {
+            for (int j = sub; j < C; j += lanes) rank += (sg[j] > si) || (sg[j] == si && j < i);
+            for (int o = 1; o < lanes; o <<= 1) rank += __shfl_xor(rank, o, 64);
+            if (sub == 0) {
+                perm[rank] = i;
+                if (rank >= k) disc += sig[i];
+            }
+        }
+    } else {
+        for (int i = threadIdx.x; i < C; i += SORT_THREADS) {
+            const double si = sort_key(sig[i]);
+            int rank = 0;
             for (int j = 0; j < C; ++j) {
                 const double sj = sort_key(sig[j]);
                 rank += (sj > si) || (sj == si && j < i);
             }
+            perm[rank] = i;
+            if (rank >= k) disc += sig[i];
         }
-        perm[rank] = i;
-        if (rank >= k) disc += sig[i];
     }
-    disc = block_sum_256(disc, red);
+    for (int o = 32; o > 0; o >>= 1) disc += __shfl_down(disc, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = disc;
     __syncthreads();
+    if (threadIdx.x == 0) {
+        disc = 0.0;
+        for (int w = 0; w < SORT_THREADS / 64; ++w) disc += red[w];
+    }
     if (threadIdx.x == 0 && op.discarded) *op.discarded = disc;
     if (threadIdx.x == 0 && unconverged && p.nb >= 2 && !ctl_ptr(ws, p)->conv)
         atomicAdd(unconverged, 1);
     if (op.s_out)
-        for (int j = threadIdx.x; j < k; j += 256) {
+        for (int j = threadIdx.x; j < k; j += SORT_THREADS) {
             op.s_out[j] = (float)sqrt(sig[perm[j]]);
         }
 }
@@ -2190,7 +2210,7 @@ hipError_t launch_sweep_end(hipStream_t s, const mpsx_two_site_op *d, int count,
 
 hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
                        int *unconverged, int small) {
-    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(256), 0, s, d, count, ws, unconverged, small);
+    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(SORT_THREADS), 0, s, d, count, ws, unconverged, small);
     return hipGetLastError();
 }
 

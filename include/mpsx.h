@@ -87,6 +87,12 @@ typedef struct {
 int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h,
                         const mpsx_site_op *d, int count);
 
+/* The same for at most MPSX_SITE_NOW gates whose descriptors travel in the
+ * launch's arguments (no device table). Refused on a stream being captured. */
+#define MPSX_SITE_NOW 16
+
+int mpsx_apply_one_site_now(mpsx_stream stream, const mpsx_site_op *h, int count);
+
 /* ------------------------------------------------------------------------
  * Two-site update on adjacent sites (i, i+1).
  * Replaces the arithmetic of MPS.apply_two_qudit_gate

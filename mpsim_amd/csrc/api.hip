@@ -251,12 +251,11 @@ int mpsx_put(mpsx_stream stream, void *dst, const void *src, size_t bytes) {
 }
 
 // ---------------------------------------------------------------- one-site
-int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h, const mpsx_site_op *d,
-                        int count) {
-    if (count < 0) return fail(MPSX_EINVAL, "count < 0");
-    if (count == 0) return MPSX_OK;
-    if (!h || !d) return fail(MPSX_EINVAL, "null descriptor table");
-    if (count > 65535) return fail(MPSX_EINVAL, "count %d > 65535", count);
+}  // extern "C"
+
+namespace {
+// d: the device table, or null for descriptors in the launch's arguments.
+int one_site_run(hipStream_t stream, const mpsx_site_op *h, const mpsx_site_op *d, int count) {
     int64_t max_pairs = 0;
     uint32_t dmask = 0;  // bit d: some op has qudit dimension d
     for (int i = 0; i < count; ++i) {
@@ -270,8 +269,30 @@ int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h, const mpsx_si
         if (pairs > 0) dmask |= 1u << o.d;
     }
     if (max_pairs == 0) return MPSX_OK;
-    HIP_TRY(timed("k_one_site", (hipStream_t)stream, [&] { return launch_one_site((hipStream_t)stream, d, count, max_pairs, dmask); }), "k_one_site");
+    HIP_TRY(timed("k_one_site", stream, [&] { return launch_one_site(stream, h, d, count, max_pairs, dmask); }), "k_one_site");
     return MPSX_OK;
+}
+}  // namespace
+
+extern "C" {
+
+int mpsx_apply_one_site(mpsx_stream stream, const mpsx_site_op *h, const mpsx_site_op *d,
+                        int count) {
+    if (count < 0) return fail(MPSX_EINVAL, "count < 0");
+    if (count == 0) return MPSX_OK;
+    if (!h || !d) return fail(MPSX_EINVAL, "null descriptor table");
+    if (count > 65535) return fail(MPSX_EINVAL, "count %d > 65535", count);
+    return one_site_run((hipStream_t)stream, h, d, count);
+}
+
+int mpsx_apply_one_site_now(mpsx_stream stream, const mpsx_site_op *h, int count) {
+    if (count < 0 || count > MPSX_SITE_NOW) return fail(MPSX_EINVAL, "count %d outside [0,%d]", count, MPSX_SITE_NOW);
+    if (count == 0) return MPSX_OK;
+    if (!h) return fail(MPSX_EINVAL, "null descriptor table");
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing((hipStream_t)stream, &cap), "hipStreamIsCapturing");
+    if (cap != hipStreamCaptureStatusNone) return fail(MPSX_EINVAL, "mpsx_apply_one_site_now on a stream being captured");
+    return one_site_run((hipStream_t)stream, h, nullptr, count);
 }
 
 // ---------------------------------------------------------------- scale
@@ -550,7 +571,8 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         HIP_TRY(timed("k_small", stream,
                       [&] { return launch_small(stream, d, count, ws, r.tol, r.null_rel, r.unconverged); }),
                 "k_small");
-    if (rest) {
+    // the norms of theta: for the convergence tests of the problems that iterate
+    if (rest && (rows_nb > 0 || has_rounds)) {
         HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows, small); }), "k_rownorm");
         HIP_TRY(timed("k_fro", stream, [&] { return launch_fro(stream, d, count, ws, r.null_rel, small); }), "k_fro");
     }

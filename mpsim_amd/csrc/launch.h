@@ -6,8 +6,9 @@
 
 #include "../../include/mpsx.h"
 
-hipError_t launch_one_site(hipStream_t s, const mpsx_site_op *d, int count, int64_t max_pairs,
-                           uint32_t dmask);
+// d: the table on the device, or null: h (at most MPSX_SITE_NOW) goes with the launch.
+hipError_t launch_one_site(hipStream_t s, const mpsx_site_op *h, const mpsx_site_op *d, int count,
+                           int64_t max_pairs, uint32_t dmask);
 hipError_t launch_put(hipStream_t s, void *dst, const void *src, size_t bytes);
 hipError_t launch_scale(hipStream_t s, const mpsx_scale_op *d, int count, int64_t max_n);
 hipError_t launch_gemm(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gemm_op *d, int count, int64_t max_m,

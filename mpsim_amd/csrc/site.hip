@@ -51,8 +51,15 @@ MPSX_DEV void one_site_generic(const mpsx_site_op &op, const float2 *g, int64_t 
 
 // One kernel per qudit dimension 2..4 (ops of other dimensions return at
 // once), launched for the dimensions a call has.
-template <int D>
-__global__ void __launch_bounds__(256) k_one_site(const mpsx_site_op *ops) {
+// Ops: the descriptors in device memory, or in the launch's arguments
+// (SiteArgs: for one gate at a time, which a launch of k_put before it, 5 us,
+// would double).
+struct SiteArgs {
+    mpsx_site_op op[MPSX_SITE_NOW];
+    MPSX_DEV const mpsx_site_op &operator[](unsigned i) const { return op[i]; }
+};
+template <int D, class Ops>
+__global__ void __launch_bounds__(256) k_one_site(Ops ops) {
     __shared__ float2 g[D * D];
     const mpsx_site_op op = ops[blockIdx.y];
     if (op.d != D) return;
@@ -68,7 +75,8 @@ __global__ void __launch_bounds__(256) k_one_site(const mpsx_site_op *ops) {
 // Every other dimension (1, and 5..16). Kept apart from the unrolled kernels
 // because its runtime-indexed input array lives in scratch memory, which
 // every launch of a kernel that has it must reserve.
-__global__ void __launch_bounds__(256) k_one_site_gen(const mpsx_site_op *ops) {
+template <class Ops>
+__global__ void __launch_bounds__(256) k_one_site_gen(Ops ops) {
     __shared__ float2 g[SITE_MAXD * SITE_MAXD];
     const mpsx_site_op op = ops[blockIdx.y];
     const int d = op.d;
@@ -124,15 +132,23 @@ static unsigned blocks_for(int64_t n, int64_t per_block, unsigned cap) {
     return (unsigned)b;
 }
 
-hipError_t launch_one_site(hipStream_t s, const mpsx_site_op *d, int count, int64_t max_pairs,
-                           uint32_t dmask) {
+template <class Ops>
+static hipError_t launch_one_site_t(hipStream_t s, Ops ops, int count, int64_t max_pairs, uint32_t dmask) {
     dim3 grid(blocks_for(max_pairs, 256, 8192), (unsigned)count);
-    if (dmask & (1u << 2)) hipLaunchKernelGGL(k_one_site<2>, grid, dim3(256), 0, s, d);
-    if (dmask & (1u << 3)) hipLaunchKernelGGL(k_one_site<3>, grid, dim3(256), 0, s, d);
-    if (dmask & (1u << 4)) hipLaunchKernelGGL(k_one_site<4>, grid, dim3(256), 0, s, d);
+    if (dmask & (1u << 2)) hipLaunchKernelGGL((k_one_site<2, Ops>), grid, dim3(256), 0, s, ops);
+    if (dmask & (1u << 3)) hipLaunchKernelGGL((k_one_site<3, Ops>), grid, dim3(256), 0, s, ops);
+    if (dmask & (1u << 4)) hipLaunchKernelGGL((k_one_site<4, Ops>), grid, dim3(256), 0, s, ops);
     if (dmask & ~((1u << 2) | (1u << 3) | (1u << 4)))
-        hipLaunchKernelGGL(k_one_site_gen, grid, dim3(256), 0, s, d);
+        hipLaunchKernelGGL(k_one_site_gen<Ops>, grid, dim3(256), 0, s, ops);
     return hipGetLastError();
+}
+
+hipError_t launch_one_site(hipStream_t s, const mpsx_site_op *h, const mpsx_site_op *d, int count,
+                           int64_t max_pairs, uint32_t dmask) {
+    if (d) return launch_one_site_t(s, d, count, max_pairs, dmask);
+    SiteArgs args = {};
+    memcpy(args.op, h, sizeof(mpsx_site_op) * (size_t)count);
+    return launch_one_site_t(s, args, count, max_pairs, dmask);
 }
 
 hipError_t launch_scale(hipStream_t s, const mpsx_scale_op *d, int count, int64_t max_n) {

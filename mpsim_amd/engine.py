@@ -226,6 +226,9 @@ class Engine:
             return
         tab = np.array(rows, dtype=nat.SITE_OP)
         stream = self.stream
+        if len(rows) <= nat.SITE_NOW and self.lib.mpsx_apply_one_site_now(
+                stream, tab.ctypes.data, len(rows)) == nat.MPSX_OK:
+            return
         dtab = nat.put_table(tab, self.dev, stream)
         nat.check(self.lib.mpsx_apply_one_site(stream, tab.ctypes.data, dtab.data_ptr(),
                                                len(rows)))

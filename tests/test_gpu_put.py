@@ -62,3 +62,28 @@ def test_chain_of_products(links, size):
     chain.flush()
     err = np.linalg.norm(cur.cpu().numpy() - want)
     assert err <= links * size * 2.0 ** -23 * np.sqrt(size)
+
+
+@pytest.mark.parametrize("count", [1, 15, 16, 17])
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5])
+def test_one_site_gates_with_and_without_a_device_table(count, d):
+    """The same bits from mpsx_apply_one_site_now (up to 16 gates) and from a device table."""
+    import torch
+    from mpsim_amd import _native as nat
+    from mpsim_amd.engine import Engine
+    eng = Engine.get()
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(count + 100 * d)
+    lib, stream = nat.load(), eng.stream
+    g = torch.randn(d, d, dtype=torch.complex64, device="cuda", generator=gen)
+    ts = [torch.randn(3 + i, d, 5, dtype=torch.complex64, device="cuda", generator=gen) for i in range(count)]
+    one = [torch.empty_like(t) for t in ts]
+    two = [torch.empty_like(t) for t in ts]
+    eng.one_site([(t, o, g) for t, o in zip(ts, one)])
+    tab = np.array([(nat.ptr(t), nat.ptr(o), nat.ptr(g), t.shape[0], t.shape[2], d, 0) for t, o in zip(ts, two)],
+                   dtype=nat.SITE_OP)
+    dtab = nat.to_device_table(tab, eng.dev)
+    nat.check(lib.mpsx_apply_one_site(stream, tab.ctypes.data, dtab.data_ptr(), count))
+    assert all(torch.equal(torch.view_as_real(x), torch.view_as_real(y)) for x, y in zip(one, two))
+    code = lib.mpsx_apply_one_site_now(stream, tab.ctypes.data, count)
+    assert (code == nat.MPSX_OK) == (count <= nat.SITE_NOW)

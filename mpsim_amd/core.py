@@ -374,11 +374,12 @@ class MPS:
         The environment after a prefix of sites is E[b, y, a, x]: b / a the
         bra / ket values of the kept sites so far, y / x the open bra / ket
         bond. Per site A[x, s, x']:
-          F[b, y, a, (s, x')] = sum_x E[b, y, a, x] A[x, s, x']       (one GEMM)
-          kept:   E'[(b, t), y', (a, s), x'] = sum_y conj(A[y, t, y']) F[b, y, a, s, x']
+          kept:   F[b, y, a, s, x'] = sum_x E[b, y, a, x] A[x, s, x']   (one GEMM)
+                  E'[(b, t), y', (a, s), x'] = sum_y conj(A[y, t, y']) F[b, y, a, s, x']
                   (one GEMM per b)
-          traced: E'[b, y', a, x'] = sum_{y, s} conj(A[y, s, y']) F[b, y, a, s, x']
-                  (one GEMM per (b, a), accumulated over s)
+          traced: F[b, y, s, a, x'] = the same sum                    (one GEMM per (a, s))
+                  E'[b, y', a, x'] = sum_{y, s} conj(A[y, s, y']) F[b, y, s, a, x']
+                  (one GEMM per b: y and s are one index of both)
         """
         torch = self._engine.torch
         dev, eng, d = self._engine.dev, self._engine, self._qudit_dimension
@@ -388,10 +389,15 @@ class MPS:
         kb = ka = 1
         for i, a in enumerate(self._tensors):
             xl, _, xr = a.shape
-            f = torch.empty((kb, xl, ka, d * xr), dtype=torch.complex64, device=dev)
-            chain.gemm([dict(A=env, B=a, C=f, m=kb * xl * ka, n=d * xr, k=xl, lda=xl,
-                             ldb=d * xr, ldc=d * xr)])
             row_f = ka * d * xr
+            f = torch.empty((kb * xl, row_f), dtype=torch.complex64, device=dev)
+            if i in keep or ka == 1:
+                chain.gemm([dict(A=env, B=a, C=f, m=kb * xl * ka, n=d * xr, k=xl, lda=xl,
+                                 ldb=d * xr, ldc=d * xr)])
+            else:
+                chain.gemm([dict(A=(env, c * xl), B=(a, s * xr), C=(f, (s * ka + c) * xr), m=kb * xl,
+                                 n=xr, k=xl, lda=ka * xl, ldb=d * xr, ldc=row_f)
+                            for c in range(ka) for s in range(d)])
             if i in keep:
                 nxt = torch.empty((kb, d, xr, ka, d, xr), dtype=torch.complex64, device=dev)
                 chain.gemm([dict(A=a, B=(f, b * xl * row_f), C=(nxt, b * d * xr * ka * d * xr),
@@ -400,12 +406,9 @@ class MPS:
                 kb, ka = kb * d, ka * d
             else:
                 nxt = torch.empty((kb, xr, ka, xr), dtype=torch.complex64, device=dev)
-                for s in range(d):
-                    chain.gemm([dict(A=(a, s * xr), B=(f, b * xl * row_f + c * d * xr + s * xr),
-                                     C=(nxt, b * xr * ka * xr + c * xr), m=xr, n=xr, k=xl,
-                                     lda=d * xr, ldb=row_f, ldc=ka * xr,
-                                     flags=nat.GEMM_CONJ_A | (nat.GEMM_ACCUM if s else 0))
-                                for b in range(kb) for c in range(ka)])
+                chain.gemm([dict(A=a, B=(f, b * xl * row_f), C=(nxt, b * xr * ka * xr), m=xr,
+                                 n=ka * xr, k=xl * d, lda=xr, ldb=ka * xr, ldc=ka * xr,
+                                 flags=nat.GEMM_CONJ_A) for b in range(kb)])
             env = nxt
         chain.flush()
         return env.reshape(kb, ka).transpose(0, 1)

@@ -236,7 +236,8 @@ def run_qutrit(args, eng, svd):
     circ = brickwork_haar(48, depth, 3, maxsvals=1024, seed=4)
     flops, _, updates = circuit_work(circ)
     svd_f, _ = svd_flops(circ, svd.block_switch or 64, gram_min_rows(svd))
-    kset = round_kernels(svd)
+    rows = 3072
+    kset = svd_kernels(svd, rows)
     peak = PEAK_FP32_MFMA if svd.fp32 else PEAK_FP64_MFMA
     dc = prepare(circ, eng)
     torch.cuda.synchronize()
@@ -247,19 +248,19 @@ def run_qutrit(args, eng, svd):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     nat.profile_enable(False)
-    busy = nat.profile_busy(busy_kernels(svd))
+    busy = nat.profile_busy(busy_kernels(svd, rows))
     kern = nat.profile_read(reset=True)
-    jr_n = round_launches(kern, kset)
+    jr_n = unit_launches(kern, kset)
     ach = svd_f["big"] / (busy * 1e-3) / 1e12 if busy else 0.0
     line = base_line("2-site gate updates/s, 48 qutrits chi<=1024", updates / dt, "2-site updates/s",
                      args, 1e3 * dt, {"workload": f"48 qutrits, brickwork depth {depth}, 9x9 Haar, "
                                       "maxsvals=1024", "updates": updates})
-    line["roofline"] = {"kernel": "+".join(busy_kernels(svd)), "bound": "mfma", "achieved": round(ach, 3),
+    line["roofline"] = {"kernel": "+".join(busy_kernels(svd, rows)), "bound": "mfma", "achieved": round(ach, 3),
                         "peak": peak, "unit": "TFLOP/s",
-                        "frac": round(ach / peak, 5), "rounds": jr_n,
+                        "frac": round(ach / peak, 5), "units": jr_n,
                         "frac_of_fp32_mfma_peak": round(ach / PEAK_FP32_MFMA, 5),
                         "achieved_basis": "SVD flops of the updates with 32-row pivots / busy time "
-                                          "of their round kernels"}
+                                          "of their SVD kernels"}
     line["extra"] = {"kernel_ms": {k: round(v[0], 2) for k, v in sorted(kern.items())},
                      "bond_dimensions_max": max(dc.mps.bond_dimensions()),
                      "algorithmic_tflops_per_s": round(flops / dt / 1e12, 3)}
@@ -460,31 +461,44 @@ def gram_min_rows(svd):
     return 64 if not svd.fp32 and svd.method == 0 else 0
 
 
-def round_kernels(svd):
-    """Kernels of one Jacobi round of the updates with 32-row pivots: the
-    eigensolve and update launches of the Gram method (the default; with
-    fp32_sweeps > 0 also those of its FP32 phase), else the one-sided round
-    kernel."""
+# the direct solver's kernels: H, its tridiagonal form, that form's eigensystem, Y, X <- Y X
+DIRECT = ["k_hgram", "k_tridiag", "k_eig_conquer", "k_eig_back", "k_hxgemm"]
+
+
+def direct_solver(svd):
+    """Whether the updates of more than 64 rows take the direct eigensolver
+    (up to 1024 rows; the Gram method without an FP32 phase)."""
+    return not svd.fp32 and svd.method == 0 and svd.fp32_sweeps <= 0
+
+
+def svd_kernels(svd, rows):
+    """Kernels of the SVD of the updates with 32-row pivots, the largest of
+    `rows` rows: the direct solver's (the default), beyond 1024 rows (or with
+    fp32_sweeps > 0) the eigensolve and update launches of the Gram method's
+    rounds, else the one-sided round kernel."""
     if not svd.fp32 and svd.method == 0:
         ks = ["k_hsolve", "k_hround", "k_hupdate"]
-        return ks + [k + "32" for k in ks] if svd.fp32_sweeps > 0 else ks
+        if svd.fp32_sweeps > 0:
+            return ks + [k + "32" for k in ks]
+        return DIRECT if rows <= 1024 else DIRECT + ks
     return [("k_jacobi_round32" if svd.fp32 else "k_jacobi_round64") + "<32>"]
 
 
-def busy_kernels(svd):
-    """Kernels whose launch intervals make the SVD's busy time: the round
-    kernels, and with preconditioning the Householder QR that precedes the
-    Gram rounds (it does part of the work that the SVD flops count)."""
-    ks = round_kernels(svd)
-    if svd.precondition and not svd.fp32 and svd.method == 0 and svd.fp32_sweeps <= 0:
+def busy_kernels(svd, rows):
+    """Kernels whose launch intervals make the SVD's busy time: svd_kernels,
+    and where preconditioned rounds run the Householder QR that precedes them
+    (it does part of the work that the SVD flops count)."""
+    ks = svd_kernels(svd, rows)
+    if svd.precondition and direct_solver(svd) and rows > 1024:
         ks = ks + ["k_qr_order", "k_qr_permute", "k_qr_step"]
     return ks
 
 
-def round_launches(kern, kset):
-    """Rounds run: one eigensolve launch (k_hsolve* or k_hround*) per round
-    of the Gram method, one launch per round of the one-sided method."""
-    eig = [k for k in kset if k.startswith("k_hsolve") or k.startswith("k_hround")] or kset
+def unit_launches(kern, kset):
+    """Units run: one tridiagonal launch per group of the direct solver, one
+    eigensolve launch (k_hsolve* or k_hround*) per round of the Gram method, one
+    launch per round of the one-sided method."""
+    eig = [k for k in kset if k == "k_tridiag" or k.startswith("k_hsolve") or k.startswith("k_hround")] or kset
     return sum(kern.get(k, (0.0, 0))[1] for k in eig)
 
 
@@ -516,7 +530,7 @@ def svd_flops(circuit, switch=64, min_rows=0):
 
 
 def load_traffic():
-    path = os.path.join(ROOT, "profiles", "traffic_jacobi_round.json")
+    path = os.path.join(ROOT, "profiles", "traffic_direct_solver.json")
     try:
         with open(path) as f:
             return json.load(f)
@@ -563,7 +577,8 @@ def main():
     circ = brickwork_haar(64, 20, 2, maxsvals=256, seed=2)
     flops, bytes_, updates = circuit_work(circ)
     svd_f, _ = svd_flops(circ, svd.block_switch or 64, gram_min_rows(svd))
-    kset = round_kernels(svd)
+    rows = 512  # of theta at the cap
+    kset = svd_kernels(svd, rows)
 
     dc = prepare(circ, eng)
     for _ in range(args.warmup):
@@ -592,36 +607,35 @@ def main():
     nat.profile_enable(True)
     ptimes = timed_steps()
     nat.profile_enable(False)
-    jr_busy = nat.profile_busy(busy_kernels(svd))
+    jr_busy = nat.profile_busy(busy_kernels(svd, rows))
     full = nat.profile_read_full(reset=True)
     kern = {k: (v["total_ms"], v["launches"]) for k, v in full.items()}
     total = sum(times)
     value = updates * args.steps / total
     ms_per_step = 1e3 * total / args.steps
 
-    # The roofline unit is one Jacobi round of the updates with 32-row pivots
-    # (k_hsolve / k_hround + k_hupdate for the Gram method, one
-    # k_jacobi_round launch otherwise). Large two-site calls run as four concurrent groups on four
-    # streams, so rounds overlap: throughput is the SVD flops over the busy
-    # time of the round kernels (the union of all their launch intervals);
-    # the per-round figure (flops per round / average round duration) is
-    # reported beside it.
+    # The roofline unit is one solve of a group of updates with 32-row pivots: its
+    # k_hgram + k_tridiag + k_eig_conquer + k_eig_back + k_hxgemm launches (one
+    # round of the Gram or one-sided method where those are asked for).
+    # Large two-site calls run as four concurrent groups on four
+    # streams, so the groups overlap: throughput is the SVD flops over the busy
+    # time of these kernels (the union of all their launch intervals);
+    # the per-unit figure (flops per unit / average duration) is reported
+    # beside it.
     dom = "+".join(kset)
     jr_ms = sum(kern.get(k, (0.0, 0))[0] for k in kset)
-    # rounds: one eigensolve launch each (k_hsolve opens a sweep, k_hround runs
-    # the next round's eigensolves beside the current round's update)
-    jr_n = round_launches(kern, kset)
+    jr_n = unit_launches(kern, kset)
     dom_f = svd_f["big"] * args.steps
     achieved = dom_f / (jr_busy * 1e-3) / 1e12 if jr_busy > 0 else 0.0
     per_round = dom_f / (jr_ms * 1e-3) / 1e12 if jr_ms > 0 else 0.0
     traffic = load_traffic()
-    tbytes = (traffic.get("bytes_per_round")
+    tbytes = (traffic.get("bytes_per_unit")
               if traffic and traffic.get("kernel") == "+".join(kset) else None)
-    # executed FP64 MFMA flops per round (SQ_INSTS_VALU_MFMA_MOPS_F64 x 512 from a
+    # executed FP64 MFMA flops per unit (SQ_INSTS_VALU_MFMA_MOPS_F64 x 512 from a
     # counter pass) over the live busy time
     mc = (traffic or {}).get("mfma_counters")
     roofline = {
-        "kernel": "+".join(busy_kernels(svd)),
+        "kernel": "+".join(busy_kernels(svd, rows)),
         "bound": "mfma",
         "achieved": round(achieved, 3),
         "peak": peak,
@@ -631,28 +645,28 @@ def main():
         # denominator of the FP32-MFMA formulation of this SVD
         "frac_of_fp32_mfma_peak": round(achieved / PEAK_FP32_MFMA, 5),
         "traffic": tbytes,
-        "traffic_unit": "HBM bytes per round (calibrated FETCH_SIZE + WRITE_SIZE)",
+        "traffic_unit": "HBM bytes per solve of a group (calibrated FETCH_SIZE + WRITE_SIZE)",
         "achieved_basis": "algorithmic SVD flops of the updates with 32-row pivots / busy time of "
-                          "their round kernels (union of launch intervals, HIP events on the launch "
+                          "their SVD kernels (union of launch intervals, HIP events on the launch "
                           "streams), from a profiled repeat of the timed steps",
         "profiled_pass_updates_per_s": round(updates * args.steps / sum(ptimes), 3),
         "busy_ms": round(jr_busy, 3),
         "concurrency": round(jr_ms / jr_busy, 3) if jr_busy > 0 else None,
-        "achieved_per_round": round(per_round, 3),
-        "rounds": jr_n,
-        "avg_round_us": round(1e3 * jr_ms / max(jr_n, 1), 3),
+        "achieved_per_unit": round(per_round, 3),
+        "units": jr_n,
+        "avg_unit_us": round(1e3 * jr_ms / max(jr_n, 1), 3),
         "avg_launch_us": {k: round(1e3 * kern[k][0] / max(kern[k][1], 1), 3)
-                          for k in busy_kernels(svd) if k in kern},
+                          for k in busy_kernels(svd, rows) if k in kern},
         "executed_mfma_frac_counters": (
-            round(mc["executed_flop_per_round"] * jr_n / (jr_busy * 1e-3) / 1e12 / peak, 4)
+            round(mc["executed_flop_per_unit"] * jr_n / (jr_busy * 1e-3) / 1e12 / peak, 4)
             if (mc and not svd.fp32 and jr_busy > 0 and mc.get("kernel") == dom) else None),
-        "algorithmic_flops_per_round": dom_f / max(jr_n, 1),
+        "algorithmic_flops_per_unit": dom_f / max(jr_n, 1),
         "algorithmic_unit": "SVD term 4(4p^2q+8pq^2+9q^3) of the updates with 32-row pivots",
     }
 
     extra = {
         "kernel_ms_per_step": {k: round(v[0] / args.steps, 3) for k, v in sorted(kern.items())},
-        "round_kernels": dom,
+        "svd_kernels": dom,
         "sweeps_last_layer": eng.last_sweeps,
         "algorithmic_tflops_per_s": round(flops * args.steps / total / 1e12, 3),
         "algorithmic_hbm_gb_per_s": round(bytes_ * args.steps / total / 1e9, 3),
@@ -718,8 +732,8 @@ def main():
         "data": "synthetic (seeded Haar gates)",
         "config": {"workload": "64-qubit brickwork depth 20, Haar 4x4 gates, maxsvals=256, "
                                "layer-batched",
-                   "arithmetic": ("complex64 site tensors and theta; Jacobi working matrix, "
-                                  "Gram and rotations in " + ("FP32" if args.fp32 else "FP64")), "qubits": 64, "depth": 20, "maxsvals": 256,
+                   "arithmetic": ("complex64 site tensors; theta, working matrix, Gram and "
+                                  "eigensolver in " + ("FP32" if args.fp32 else "FP64")), "qubits": 64, "depth": 20, "maxsvals": 256,
                    "updates_per_step": updates, "parallelism": "single GPU"},
         "roofline": roofline,
         "cpu_baseline": cpu,

@@ -111,10 +111,12 @@ int mpsx_apply_one_site_now(mpsx_stream stream, const mpsx_site_op *h, int count
  * divides by a singular value: a blocked one-sided Jacobi on theta's rows up
  * to 64 of them, above that the eigenvectors of the rows' Gram matrix, by a
  * direct solver (tridiagonal form, divide and conquer) up to 1024 rows and
- * by Jacobi rounds beyond. theta is formed in
- * complex FP64 for d = 2 and 3 (FP32 for other d and with rotation_fp32); by
- * default the rotations are stored and applied in complex FP64 (FP64 matrix cores), which keeps each truncated update as accurate
- * as a complex64 LAPACK SVD. With rotation_fp32 set they run in FP32
+ * by Jacobi rounds beyond. (Up to 64 rows of at most 512 columns the rows
+ * that are not orthogonal yet go through the same direct route in one
+ * workgroup.) theta is formed in complex FP64 for d = 2 and 3 (FP32 for
+ * other d and with rotation_fp32); by default everything after it is
+ * complex FP64 (FP64 matrix cores), which keeps each truncated update as
+ * accurate as a complex64 LAPACK SVD. With rotation_fp32 set they run in FP32
  * (faster, about 1e-6 relative error per update).
  *
  * Plain split: with gate == NULL and d == 1 the op factorises the M x N

@@ -487,6 +487,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     int64_t groups = 0;      // the direct solver's workgroup table (as planned)
     int64_t eig_slots = 0;   // workgroups the direct solver launches
     int eig_n = 0;           // its largest problem
+    int64_t eig_tiles = 0;   // 32 x 32 tiles of its largest X
     bool eig_small = false, eig_large = false;
     int qr_c = 0, qr_r = 0, qr_rc = 0, qr_np = 0;  // QR-preconditioned problems: max C, R, R + C, panels
     bool qr_small = false, qr_large = false;  // some of at most 512 rows, some above
@@ -523,15 +524,16 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
             has_gram = true;
             has_mixed = has_mixed || p.method == 2;
             if (max_n < 0) max_n = direct_max(count);
-            gram_nb = std::max(gram_nb, eig_direct(p, max_n) ? p.Cp / 16 : p.nb);
-            gram_c = std::max(gram_c, (p.R + 31) / 32);
             if (eig_direct(p, EIG_MAX_N)) groups += eig_group(p.C);
             if (eig_direct(p, max_n)) {
                 eig_slots += eig_group(p.C);
                 eig_n = std::max(eig_n, (int)p.C);
+                eig_tiles = std::max(eig_tiles, (int64_t)((p.C + 31) / 32) * ((p.R + 31) / 32));
                 (p.C <= 512 ? eig_small : eig_large) = true;
             } else {
                 has_rounds = true;
+                gram_nb = std::max(gram_nb, p.nb);
+                gram_c = std::max(gram_c, (p.R + 31) / 32);
                 round_nb = std::max(round_nb, p.nb);
                 gram_y = std::max(gram_y, p.nb / 4 + (p.Cp + 63) / 64);
             }
@@ -595,11 +597,12 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
 
     int sweeps = 0;
     bool converged = false;
-    if (pairs > 0 && (has_gram || rows_nb > 0))
+    if (pairs > 0 && (has_rounds || rows_nb > 0))
         HIP_TRY(timed("k_owner", stream, [&] { return launch_owner(stream, d, count, owner); }), "k_owner");
-    if (has_gram)
+    if (has_rounds)
         HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 0, max_n); }), "k_hgram");
     if (eig_slots > 0) {
+        HIP_TRY(timed("k_hgram", stream, [&] { return launch_eig_gram(stream, d, count, ws, max_n, eig_n); }), "k_eig_gemm");
         HIP_TRY(timed("k_tridiag", stream,
                       [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128); }),
                 "k_tridiag");
@@ -713,7 +716,10 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
 
     if (has_gram) {
         HIP_TRY(timed("k_hxcopy", stream, [&] { return launch_hxcopy(stream, d, count, ws, rows, max_n); }), "k_hxcopy");
-        HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 0, gram_nb, max_n); }), "k_hxgemm");
+        if (has_rounds)
+            HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_hxgemm(stream, d, owner, ws, pairs, gram_c, 0, gram_nb, max_n); }), "k_hxgemm");
+        if (eig_slots > 0)
+            HIP_TRY(timed("k_hxgemm", stream, [&] { return launch_eig_apply(stream, d, count, ws, max_n, eig_tiles); }), "k_eig_gemm");
     }
     if (rest) {
         HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows, small); }), "k_rownorm");

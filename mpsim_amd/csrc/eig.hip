@@ -582,6 +582,133 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
 
 }  // namespace
 
+// ---------------------------------------------- H = X X^H and X <- Y X
+// A 32 x 32 tile of the result a workgroup, its four waves 16 of every 64 k:
+// fragments straight from memory (lane l k = 4 (l / 16) .. + 3 of a wave's
+// block in its four matrix instructions), three real products a complex one,
+// the waves' sums meeting in LDS in a fixed order.
+//   GRAM:  H (both triangles, from the tiles ti <= tj), A = B^H = X
+//   else:  X = Y Xc, Xc the copy of X in the H region (row stride R)
+// x: tile, y: problem. (A problem's tiles on one XCD, for its L2, gained nothing at 28
+// problems of 512 rows and left XCDs idle beside fewer or uneven ones.)
+// Bound: the FP64 matrix cores. Against 16 x 16 tiles of H and 32 x 32 or
+// LDS-staged ones of X (us): 28 of 512 x 512: H 629 -> 266, X 631 -> 387; one: 30 -> 25
+// and 31 -> 24; a layer with four of 1024 x 1024: 754 -> 250 and 1193 -> 358.
+template <bool GRAM>
+__global__ void __launch_bounds__(256, 2)
+k_eig_gemm(const mpsx_two_site_op *ops, char *ws, int max_n) {
+    __shared__ double2 part[4][32][33];
+    const mpsx_plan p = ops[blockIdx.y].plan;
+    int t = (int)blockIdx.x;
+    if (!eig_direct(p, max_n)) return;
+    const int n = p.C, Cp = p.Cp, R = p.R, nt = (n + 31) / 32;
+    int ti, tj;
+    if (GRAM) {
+        ti = 0;
+        while (ti < nt && t >= nt - ti) t -= nt - ti++;
+        if (ti >= nt) return;
+        tj = ti + t;
+    } else {
+        const int nc = (R + 31) / 32;
+        ti = t / nc;
+        tj = t % nc;
+        if (ti >= nt) return;
+    }
+    double2 *Z = reinterpret_cast<double2 *>(ws + z_off(p));
+    double2 *H = eig_h(ws, p);
+    const int tid = threadIdx.x, lane = tid & 63, wave = wave_id(), l16 = lane & 15, q = lane >> 4;
+    const int64_t LD = p.LD;
+    const int K = GRAM ? R : n;
+    // rows and columns beyond the matrix repeat its last one (never stored)
+    const double2 *A[2], *B[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        const int i = min(32 * ti + 16 * a + l16, n - 1), j = 32 * tj + 16 * a + l16;
+        A[a] = Z + (GRAM ? 0 : R) + i * LD;
+        B[a] = GRAM ? Z + min(j, n - 1) * LD : H + min(j, R - 1);
+    }
+    mfma_d4 acc[2][2][3];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) acc[a][b][u] = mfma_d4{0.0, 0.0, 0.0, 0.0};
+    auto multiply = [&](const double2 (&x)[2][4], const double2 (&y)[2][4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            double xs[2], ys[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                xs[a] = x[a][u].x + x[a][u].y;
+                ys[a] = GRAM ? y[a][u].x - y[a][u].y : y[a][u].x + y[a][u].y;
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    acc[a][b][0] = mfma16d(x[a][u].x, y[b][u].x, acc[a][b][0]);
+                    acc[a][b][1] = mfma16d(x[a][u].y, y[b][u].y, acc[a][b][1]);
+                    acc[a][b][2] = mfma16d(xs[a], ys[b], acc[a][b][2]);
+                }
+        }
+    };
+    double2 x[2][4], y[2][4];
+    int k0 = 16 * wave;
+    for (; k0 + 16 <= K; k0 += 64) {
+        const int k = k0 + 4 * q;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                x[a][u] = A[a][k + u];
+                y[a][u] = GRAM ? B[a][k + u] : B[a][(int64_t)(k + u) * R];
+            }
+        multiply(x, y);
+    }
+    if (k0 < K) {
+        const int k = k0 + 4 * q;
+        const double2 zero = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                x[a][u] = k + u < K ? A[a][k + u] : zero;
+                y[a][u] = k + u < K ? (GRAM ? B[a][k + u] : B[a][(int64_t)(k + u) * R]) : zero;
+            }
+        multiply(x, y);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double p1 = acc[a][b][0][r], p2 = acc[a][b][1][r], p3 = acc[a][b][2][r];
+                part[wave][16 * a + 4 * r + q][16 * b + l16] =
+                    GRAM ? make_double2(p1 + p2, p3 - p1 + p2) : make_double2(p1 - p2, p3 - p1 - p2);
+            }
+    __syncthreads();
+    auto entry = [&](int i, int j) {
+        return zadd(zadd(part[0][i][j], part[2][i][j]), zadd(part[1][i][j], part[3][i][j]));
+    };
+    for (int e = tid; e < 32 * 32; e += 256) {
+        const int i = e >> 5, j = e & 31, gi = 32 * ti + i, gj = 32 * tj + j;
+        if (GRAM) {
+            if (gi < n && gj < n) {
+                double2 v = entry(i, j);
+                if (gi == gj) v.y = 0.0;
+                H[(int64_t)gi * Cp + gj] = v;
+            }
+            // the mirrored tile, by rows of its own
+            if (ti != tj && 32 * tj + i < n && 32 * ti + j < n)
+                H[(int64_t)(32 * tj + i) * Cp + 32 * ti + j] = zconj(entry(j, i));
+        } else if (gi < n && gj < R) {
+            Z[gi * LD + gj] = entry(i, j);
+        }
+    }
+}
+
 // Table of the workgroups of k_tridiag: entry s = (problem, member << 8 |
 // group size), the problems with the largest groups first. One workgroup.
 __global__ void __launch_bounds__(256)
@@ -1175,5 +1302,16 @@ hipError_t launch_eig_back(hipStream_t s, const mpsx_two_site_op *d, int count, 
     if (large)
         hipLaunchKernelGGL(k_eig_back<8>, dim3((unsigned)((n + 15) / 16), (unsigned)count), dim3(512), 0, s, d, ws,
                            max_n);
+    return hipGetLastError();
+}
+
+hipError_t launch_eig_gram(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n) {
+    const unsigned nt = (unsigned)((n + 31) / 32), tiles = nt * (nt + 1) / 2;
+    hipLaunchKernelGGL(k_eig_gemm<true>, dim3(tiles, (unsigned)count), dim3(256), 0, s, d, ws, max_n);
+    return hipGetLastError();
+}
+
+hipError_t launch_eig_apply(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int64_t tiles) {
+    hipLaunchKernelGGL(k_eig_gemm<false>, dim3((unsigned)tiles, (unsigned)count), dim3(256), 0, s, d, ws, max_n);
     return hipGetLastError();
 }

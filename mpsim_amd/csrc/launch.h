@@ -73,6 +73,10 @@ hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, c
 // `large`: some of at most 512 rows, some above.
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
                               int slots, bool grouped);
+// H = X X^H, and at the end X <- Y X (tiles: 32 x 32 ones of the largest X).
+hipError_t launch_eig_gram(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
+hipError_t launch_eig_apply(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n,
+                            int64_t tiles);
 hipError_t launch_eig_conquer(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
 hipError_t launch_eig_back(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n,
                            bool small, bool large);

@@ -1169,11 +1169,8 @@ MPSX_DEV int rr_pivot(int item, int r, int n) {
 // The choice goes by the Jacobi's rows, 16 nb: for a tall QR-preconditioned
 // problem they are fewer than the working matrix's Cp rows, and the
 // launchers size their grids from nb too.
-// The direct solver works on all Cp rows (p.nb may count fewer blocks): its
-// tiles beyond the problem's nb / 2 slots are taken in further passes.
 constexpr int kTiledGemmRows = 512;
-MPSX_DEV int gram_rows(const mpsx_plan &p, int max_n) { return eig_direct(p, max_n) ? p.Cp : 16 * p.nb; }
-MPSX_DEV bool tiled_gemm(const mpsx_plan &p, int max_n) { return gram_rows(p, max_n) > kTiledGemmRows; }
+MPSX_DEV bool tiled_gemm(const mpsx_plan &p) { return 16 * p.nb > kTiledGemmRows; }
 
 // One workgroup per upper 16x16 block tile (bi <= bj) of H = X X^H. x: the
 // problem's pivot slot j (nb/2 per problem), y in [0, nb]; the tile is
@@ -1191,15 +1188,14 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     __shared__ double2 part[4][16][17];
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if ((STAGE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p, max_n)) return;
+    if ((STAGE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p) || eig_direct(p, max_n)) return;
     if (STAGE == 1 && blockIdx.x == p.pair_base && blockIdx.y == 0 && threadIdx.x == 0) {
         ProblemCtl *ctl = ctl_ptr(ws, p);
         ctl->conv = 0;
         ctl->counter = 0;
     }
     if ((int)blockIdx.y > p.nb) return;
-    const bool direct = eig_direct(p, max_n);
-    const int nb = gram_rows(p, max_n) / 16;
+    const int nb = p.nb;
     for (int tile = (int)(blockIdx.x - p.pair_base) * (p.nb + 1) + (int)blockIdx.y; tile < nb * (nb + 1) / 2;
          tile += p.nb / 2 * (p.nb + 1)) {
     int rem = tile, bi = 0;
@@ -1219,7 +1215,7 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     // in the tile's second operand and add exact zeros, so they are skipped
     // (the sums are bitwise those of the full loop).
     int cs = wave * 16;
-    if (STAGE == 0 && p.method == 3 && !direct && 16 * bj >= cs + 16) cs += 64 * ((16 * bj - 16 - cs) / 64 + 1);
+    if (STAGE == 0 && p.method == 3 && 16 * bj >= cs + 16) cs += 64 * ((16 * bj - 16 - cs) / 64 + 1);
     for (int c0 = cs; c0 < R; c0 += 64) {
         const int cq = c0 + 4 * lq;
         double2 va[4], vb[4];
@@ -1249,11 +1245,6 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
         h_store<true>(ws, p, idx, v);
     else
         h_ptr(ws, p)[idx] = v;
-    if (direct && bi != bj) {  // the direct solver reads whole rows: the mirrored tile too
-        const double2 e = part[0][j][i], f = part[1][j][i], g = part[2][j][i], h = part[3][j][i];
-        h_ptr(ws, p)[(int64_t)(bj * 16 + i) * p.Cp + bi * 16 + j] =
-            make_double2((e.x + g.x) + (f.x + h.x), -((e.y + g.y) + (f.y + h.y)));
-    }
     __syncthreads();  // part is read before the next tile
     }
 }
@@ -1786,7 +1777,7 @@ __global__ void __launch_bounds__(256)
 k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
-    if ((MODE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p, max_n)) return;
+    if ((MODE == 0 ? p.method < 1 : p.method != 2) || tiled_gemm(p) || eig_direct(p, max_n)) return;
     const int R = p.R, LD = p.LD, Cp = p.Cp;
     const int col0 = (int)blockIdx.y * 32;
     if (col0 >= R) return;
@@ -1800,7 +1791,7 @@ k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int ldx = MODE == 0 ? R : LD;
     double2 *Out = MODE == 0 ? Z : t64_ptr(ws, p);
     const int ldo = MODE == 0 ? LD : R;
-    const int rows = gram_rows(p, max_n);
+    const int rows = 16 * p.nb;
     for (int row0 = (int)(blockIdx.x - p.pair_base) * 32 + 16 * tm; row0 < rows; row0 += 16 * p.nb) {
     const double2 *yrow = Z + (int64_t)(row0 + l16) * LD + R;  // A = Y[row0 + l16][k]
     mfma_d4 a1 = {0.0, 0.0, 0.0, 0.0}, a2 = a1, a3 = a1;
@@ -1851,7 +1842,7 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int pi = owner[blockIdx.x];
     const mpsx_plan p = ops[pi].plan;
     const bool mixed_only = MODE == 1 || MODE == 3;
-    if ((mixed_only ? p.method != 2 : p.method < 1) || !tiled_gemm(p, max_n)) return;
+    if ((mixed_only ? p.method != 2 : p.method < 1) || !tiled_gemm(p) || eig_direct(p, max_n)) return;
     if (MODE == 1 && blockIdx.x == p.pair_base && blockIdx.y == 0 && threadIdx.x == 0) {
         ProblemCtl *ctl = ctl_ptr(ws, p);
         ctl->conv = 0;
@@ -1943,7 +1934,6 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
                         h_store<true>(ws, p, idx, v);
                     else
                         h_ptr(ws, p)[idx] = v;
-                    if (j0 > i0 && eig_direct(p, max_n)) h_ptr(ws, p)[(int64_t)j * Cp + i] = zconj(v);
                 } else if (MODE == 2) {
                     Z[(int64_t)i * LD + j] = v;
                 } else {

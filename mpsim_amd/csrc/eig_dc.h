@@ -323,7 +323,8 @@ struct LeafShared {
 // lanes a row; on return row j of S is eigenvector j. L.d and L.e are written by
 // the first LEAF threads before the call.
 // Bound: latency, about 8 us a level (18 with the poles one by one and the
-// rows on the vector units).
+// rows on the vector units); the deflation in one wave rather than one lane takes 30 us
+// off a block with negligible weights.
 MPSX_DEV void leaf_conquer(int m, double (*S)[LEAF + 1], double (*U)[LEAF + 1], LeafShared &L) {
     constexpr int M = LEAF;
     const int tid = threadIdx.x, g = tid >> 3, sub = tid & 7;
@@ -350,19 +351,39 @@ MPSX_DEV void leaf_conquer(int m, double (*S)[LEAF + 1], double (*U)[LEAF + 1], 
                                                  (g >= mid && ee < 0.0 ? -0.7071067811865476 : 0.7071067811865476)
                                            : 0.0;
                 L.id[lo + rank] = g;
-                if (gj == 0) L.kn[lo] = hi - lo;  // until something deflates
             }
         }
         __syncthreads();
-        if (sub == 0) {
-            if (g < m) {
-                if (may_deflate(hi - lo, gj, rho, L.ds + lo, L.zs + lo)) L.kn[lo] = -1;
-                L.dl[g] = L.ds[g];
-                L.zl[g] = L.zs[g];
-                L.src[g] = L.id[g];
-                if (gj == 0) L.nrot[lo] = 0;
+        // The first wave, a lane a sorted entry: those of negligible weight go to the end
+        // of their merge (in the order deflate() puts them there); if two of
+        // the others have to be rotated together (kn < 0), deflate() starts over.
+        if (tid < M) {
+            const int r = tid, rl = r & ~(h - 1), rm = rl + s, rh = min(rl + h, m);
+            const bool on = r < m;
+            const double rr = rm < rh ? 2.0 * fabs(L.e[rm - 1]) : 0.0;
+            const double z = on ? L.zs[r] : 0.0, d = on ? L.ds[r] : 0.0;
+            const bool keep = on && rr * fabs(z) > kDeflate;
+            const unsigned long long mine = __ballot(keep) & ((h == 64 ? ~0ULL : (1ULL << h) - 1) << rl);
+            const int before = __popcll(mine & ((1ULL << r) - 1));
+            const unsigned long long after = r < 63 ? mine >> (r + 1) : 0ULL;
+            const int nx = after ? r + __ffsll((long long)after) : r;
+            const double zn = __shfl(z, nx, 64), dn = __shfl(d, nx, 64);
+            const bool pair = keep && after && fabs((dn - d) * z * zn) <= kDeflate * fma(z, z, zn * zn);
+            const unsigned long long pairs = __ballot(pair) & ((h == 64 ? ~0ULL : (1ULL << h) - 1) << rl);
+            if (keep) {
+                L.dl[rl + before] = d;
+                L.zl[rl + before] = z;
+                L.src[rl + before] = L.id[r];
+            } else if (on) {
+                const int e = rh - 1 - (r - rl - before);
+                L.dd[e] = d;
+                L.src[e] = L.id[r];
             } else {
-                L.src[g] = g;
+                L.src[r] = r;
+            }
+            if (on && r == rl) {
+                L.kn[r] = pairs ? -1 : __popcll(mine);
+                L.nrot[r] = 0;
             }
         }
         __syncthreads();

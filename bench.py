@@ -248,14 +248,14 @@ def run_qutrit(args, eng, svd):
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
     nat.profile_enable(False)
-    busy = nat.profile_busy(busy_kernels(svd, rows))
+    busy = nat.profile_busy(kset)
     kern = nat.profile_read(reset=True)
     jr_n = unit_launches(kern, kset)
     ach = svd_f["big"] / (busy * 1e-3) / 1e12 if busy else 0.0
     line = base_line("2-site gate updates/s, 48 qutrits chi<=1024", updates / dt, "2-site updates/s",
                      args, 1e3 * dt, {"workload": f"48 qutrits, brickwork depth {depth}, 9x9 Haar, "
                                       "maxsvals=1024", "updates": updates})
-    line["roofline"] = {"kernel": "+".join(busy_kernels(svd, rows)), "bound": "mfma", "achieved": round(ach, 3),
+    line["roofline"] = {"kernel": "+".join(kset), "bound": "mfma", "achieved": round(ach, 3),
                         "peak": peak, "unit": "TFLOP/s",
                         "frac": round(ach / peak, 5), "units": jr_n,
                         "frac_of_fp32_mfma_peak": round(ach / PEAK_FP32_MFMA, 5),
@@ -465,12 +465,6 @@ def gram_min_rows(svd):
 DIRECT = ["k_hgram", "k_tridiag", "k_eig_conquer", "k_eig_back", "k_hxgemm"]
 
 
-def direct_solver(svd):
-    """Whether the updates of more than 64 rows take the direct eigensolver
-    (up to 1024 rows; the Gram method without an FP32 phase)."""
-    return not svd.fp32 and svd.method == 0 and svd.fp32_sweeps <= 0
-
-
 def svd_kernels(svd, rows):
     """Kernels of the SVD of the updates with 32-row pivots, the largest of
     `rows` rows: the direct solver's (the default), beyond 1024 rows (or with
@@ -482,16 +476,6 @@ def svd_kernels(svd, rows):
             return ks + [k + "32" for k in ks]
         return DIRECT if rows <= 1024 else DIRECT + ks
     return [("k_jacobi_round32" if svd.fp32 else "k_jacobi_round64") + "<32>"]
-
-
-def busy_kernels(svd, rows):
-    """Kernels whose launch intervals make the SVD's busy time: svd_kernels,
-    and where preconditioned rounds run the Householder QR that precedes them
-    (it does part of the work that the SVD flops count)."""
-    ks = svd_kernels(svd, rows)
-    if svd.precondition and direct_solver(svd) and rows > 1024:
-        ks = ks + ["k_qr_order", "k_qr_permute", "k_qr_step"]
-    return ks
 
 
 def unit_launches(kern, kset):
@@ -607,7 +591,7 @@ def main():
     nat.profile_enable(True)
     ptimes = timed_steps()
     nat.profile_enable(False)
-    jr_busy = nat.profile_busy(busy_kernels(svd, rows))
+    jr_busy = nat.profile_busy(kset)
     full = nat.profile_read_full(reset=True)
     kern = {k: (v["total_ms"], v["launches"]) for k, v in full.items()}
     total = sum(times)
@@ -635,7 +619,7 @@ def main():
     # counter pass) over the live busy time
     mc = (traffic or {}).get("mfma_counters")
     roofline = {
-        "kernel": "+".join(busy_kernels(svd, rows)),
+        "kernel": "+".join(kset),
         "bound": "mfma",
         "achieved": round(achieved, 3),
         "peak": peak,
@@ -656,7 +640,7 @@ def main():
         "units": jr_n,
         "avg_unit_us": round(1e3 * jr_ms / max(jr_n, 1), 3),
         "avg_launch_us": {k: round(1e3 * kern[k][0] / max(kern[k][1], 1), 3)
-                          for k in busy_kernels(svd, rows) if k in kern},
+                          for k in kset if k in kern},
         "executed_mfma_frac_counters": (
             round(mc["executed_flop_per_unit"] * jr_n / (jr_busy * 1e-3) / 1e12 / peak, 4)
             if (mc and not svd.fp32 and jr_busy > 0 and mc.get("kernel") == dom) else None),

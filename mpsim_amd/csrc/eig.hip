@@ -130,8 +130,8 @@ MPSX_DEV int eig_levels(int n) {
 // values that gates of low Schmidt rank leave make such H.
 //
 // Bound: the step's latency: an exchange (about 2 us), three barriers, and
-// instruction issue; 4.6 us a step at n = 512, 4.1 at 128. The whole update
-// of 512 x 512 takes 3.6 ms, with the Jacobi rounds (300 launches of 37 us,
+// instruction issue; 4.5 us a step at n = 512, 3.1 at 128. The whole update
+// of 512 x 512 takes 3.0 ms, with the Jacobi rounds (300 launches of 37 us,
 // behind a QR of 1.6 ms) it took 13.2. k_tridiag_one: 28 ms at 512, 0.3 s at
 // 1024.
 constexpr int kSpin = 1 << 21;  // polls of a slot of a whole group (seconds): never reached

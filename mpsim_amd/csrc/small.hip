@@ -20,8 +20,8 @@
 // formed again from Z before every test, so nothing is lost to H's rounding.
 //
 // Bound: latency. A column of the tridiagonal form is about 2 us (instruction
-// issue and two barriers), the leaf's six levels 110 us; the kernel takes 340 us
-// at 64 x 64, 85 at 16, 20 at 4. The launch sequence of the same steps
+// issue and a barrier), the leaf's six levels 60 us; the kernel takes 280 us
+// at 64 x 64, 75 at 16, 20 at 4. The launch sequence of the same steps
 // (16 launches of 5 us and more, a poll per sweep) took 1100 us at 64 x 64 and
 // 170 at 4 x 4.
 #include <hip/hip_runtime.h>

@@ -227,7 +227,9 @@ int mpsx_two_site_plan(mpsx_two_site_op *h, int count,
 
 /* Batched two-site update. Problems are independent (disjoint site pairs,
  * possibly of different circuits). `sweeps_out` (host, may be NULL)
- * receives the number of outer sweeps launched. */
+ * receives the number of outer sweeps launched. The kernels work in `ws`
+ * until the stream gets past them, which may be after the call returns: a call
+ * on another stream that uses the same `ws` is ordered behind by the caller. */
 int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h,
                   const mpsx_two_site_op *d, int count,
                   const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,

@@ -161,6 +161,12 @@ class Engine:
         self._wss: list = []        # workspaces of the helper streams' groups
         self._helpers: list = []    # (stream, single-thread executor) per helper group
         self._keep: list = []       # device tables of the last call, alive until the next
+        # Calls share the workspaces and return while their kernels run: one call is
+        # enqueued at a time, and a call on another stream than the last one's
+        # waits for that to end.
+        self._enqueue = threading.RLock()
+        self._used = None           # stream of the last call
+        self._used_end = None       # event: the last call's end on that stream
 
     @classmethod
     def get(cls, dev=None) -> "Engine":
@@ -186,12 +192,34 @@ class Engine:
         cur = self._wss[slot - 1] if slot else self._ws
         if cur is None or cur.numel() < nbytes:
             grow = max(nbytes, 0 if cur is None else int(cur.numel() * 1.25))
+            if cur is not None and self._used is not None:
+                # its memory returns to the stream it was allocated on, which need
+                # not be the one that worked on it last (and that this one follows)
+                cur.record_stream(self._used)
             cur = self.torch.empty(max(grow, 1024), dtype=self.torch.uint8, device=self.dev)
             if slot:
                 self._wss[slot - 1] = cur
             else:
                 self._ws = cur
         return cur
+
+    def _take_workspaces(self, cur) -> None:
+        """Orders the stream `cur` behind the last call's work in the workspaces.
+        An event behind every call costs the stream a few us, so one on the
+        default stream, which outlives the engine, is recorded only when another
+        stream takes over."""
+        last = self._used
+        if last is not None and last.cuda_stream != cur.cuda_stream:
+            if not last.cuda_stream:
+                self._leave_workspaces(last, True)
+            cur.wait_event(self._used_end)
+        self._used = cur
+
+    def _leave_workspaces(self, cur, now: bool = False) -> None:
+        if now or cur.cuda_stream:
+            if self._used_end is None:
+                self._used_end = self.torch.cuda.Event()
+            self._used_end.record(cur)
 
     def gate(self, mat: np.ndarray):
         """Device complex64 copy of a gate matrix (cached by content)."""
@@ -322,10 +350,21 @@ class Engine:
         stream and each other group from its own worker thread on its own
         helper stream: the latency-bound pivot eigensolves of one group then
         overlap the matrix-core phases of the others. Each problem's
-        arithmetic is the same either way."""
-        n = len(items)
-        if n == 0:
+        arithmetic is the same either way. Calls on other streams and from other
+        threads are ordered: the workspaces are the engine's."""
+        if len(items) == 0:
             return []
+        with self._enqueue:
+            cur = self.torch.cuda.current_stream(self.dev)
+            self._take_workspaces(cur)
+            try:
+                return self._two_site(items, svd, cur)
+            finally:
+                self._leave_workspaces(cur)
+
+    def _two_site(self, items: Sequence[TwoSiteItem], svd: Optional[SvdConfig], cur
+                  ) -> List[TwoSiteResult]:
+        n = len(items)
         cfg = (svd or self.svd).to_c()
         self._keep = []
         big = [i for i, it in enumerate(items) if _rows(it) >= self.split_rows]
@@ -333,7 +372,7 @@ class Engine:
         if ways < 2 or len(big) < self.split_min or cfg.check_every == 0:
             outs, tab, dtab, ws = self._prepare_two_site(items, cfg)
             self._keep = [dtab]
-            self.last_sweeps = self._run_two_site(tab, dtab, ws, cfg, self.stream)
+            self.last_sweeps = self._run_two_site(tab, dtab, ws, cfg, int(cur.cuda_stream))
             return outs
         # groups of equal estimated work (rows^2 * row length per problem),
         # largest problems first, each to the least loaded group
@@ -354,7 +393,6 @@ class Engine:
         from concurrent.futures import ThreadPoolExecutor
         while len(self._helpers) < len(grp) - 1:
             self._helpers.append((torch.cuda.Stream(self.dev), ThreadPoolExecutor(max_workers=1)))
-        cur = torch.cuda.current_stream(self.dev)
         fork = torch.cuda.Event()
         fork.record(cur)
         dev = self.dev

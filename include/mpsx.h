@@ -235,6 +235,21 @@ int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h,
                   const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
                   int *sweeps_out);
 
+/* mpsx_two_site made to take, for tests, a route that a call otherwise takes only
+ * on some devices or under load. Every kernel ends as it does without.
+ *   ROUNDS  the Gram problems of up to 1024 rows take the Jacobi rounds (plan.method
+ *           3: behind the QR) instead of the direct solver, as in calls of more
+ *           than 65535 problems and on partitions of few compute units;
+ *   LOST    the direct solver's groups of workgroups are given up from the start, as
+ *           when several launches keep each other from forming theirs. */
+#define MPSX_FORCE_ROUNDS 1
+#define MPSX_FORCE_LOST 2
+
+int mpsx_two_site_forced(mpsx_stream stream, const mpsx_two_site_op *h,
+                         const mpsx_two_site_op *d, int count,
+                         const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
+                         int *sweeps_out, int force);
+
 /* ------------------------------------------------------------------------
  * mpsx_two_site on a fixed, library-owned device workspace.
  * No counterpart in the reference (which allocates through numpy on every

@@ -461,9 +461,10 @@ namespace {
 // The two-site driver behind mpsx_two_site. `may_poll` false: never read
 // device memory back (no convergence poll; the sweep limit and the
 // device-side early exit bound the work) and create no profiling events.
+// `force`: MPSX_FORCE_* bits.
 int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_site_op *d,
                  int count, const Resolved &r, char *ws, size_t ws_bytes, int *sweeps_out,
-                 bool may_poll, size_t *need_out = nullptr) {
+                 bool may_poll, size_t *need_out = nullptr, int force = 0) {
     if (sweeps_out) *sweeps_out = 0;
     if (count < 0) return fail(MPSX_EINVAL, "count < 0");
     if (count == 0) return MPSX_OK;
@@ -523,7 +524,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         if (p.nb > 0 && p.method >= 1) {
             has_gram = true;
             has_mixed = has_mixed || p.method == 2;
-            if (max_n < 0) max_n = direct_max(count);
+            if (max_n < 0) max_n = (force & MPSX_FORCE_ROUNDS) ? 0 : direct_max(count);
             if (eig_direct(p, EIG_MAX_N)) groups += eig_group(p.C);
             if (eig_direct(p, max_n)) {
                 eig_slots += eig_group(p.C);
@@ -562,8 +563,9 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     const bool can_poll = may_poll && r.check_every > 0 && cap == hipStreamCaptureStatusNone;
 
     const bool f32 = r.fp32;
+    const int group0 = (force & MPSX_FORCE_LOST) ? EIG_GROUP_LOST : 0;
     const bool rest = rows > 0 && other;  // some problem takes the launch sequence below
-    if (rest) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n, small); }), "k_init_rows");
+    if (rest) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n, small, group0); }), "k_init_rows");
     for (int D = 1; D <= 4; ++D)
         if (has_d[D] && tiles > 0) HIP_TRY(timed("k_theta", stream, [&] { return launch_theta(stream, f32, D, d, count, ws, tiles); }), "k_theta");
     bool has_gen = false;
@@ -753,6 +755,15 @@ int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h, const mpsx_two_
                   int *sweeps_out) {
     return two_site_run((hipStream_t)stream, h, d, count, resolve(opts), static_cast<char *>(ws),
                         ws_bytes, sweeps_out, true);
+}
+
+int mpsx_two_site_forced(mpsx_stream stream, const mpsx_two_site_op *h, const mpsx_two_site_op *d,
+                         int count, const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
+                         int *sweeps_out, int force) {
+    if (force & ~(MPSX_FORCE_ROUNDS | MPSX_FORCE_LOST))
+        return fail(MPSX_EINVAL, "unknown force bits 0x%x", force);
+    return two_site_run((hipStream_t)stream, h, d, count, resolve(opts), static_cast<char *>(ws),
+                        ws_bytes, sweeps_out, true, nullptr, force);
 }
 
 

@@ -212,6 +212,8 @@ MPSX_HD int eig_group(int n) {
 // The value of an exchange slot that is not written yet (a NaN no arithmetic
 // produces, see k_tridiag).
 constexpr unsigned long long EIG_EMPTY = 0x7ff4dead5eedbeefULL;
+// ProblemCtl.group of a problem whose group was given up (form_group).
+constexpr int EIG_GROUP_LOST = 1 << 30;
 MPSX_HD int64_t problem_bytes(const mpsx_plan &p) {
     if (p.method == 0) return align_up(z_off(p) - p.ws_off + (int64_t)p.zbytes * p.Cp * p.LD, 256);
     if (p.method == 1) return align_up(qflag_off(p) - p.ws_off + 2 * 4LL * (p.nb / 2), 256);

@@ -136,7 +136,6 @@ MPSX_DEV int eig_levels(int n) {
 // 1024.
 constexpr int kSpin = 1 << 21;  // polls of a slot of a whole group (seconds): never reached
 constexpr long long kFormTicks = 4000000;  // 40 ms at 100 MHz
-constexpr int kGroupLost = 1 << 30;
 
 // Whether the group is whole; one thread of each of its workgroups asks.
 MPSX_DEV bool form_group(int *state, int G, int spread) {
@@ -144,10 +143,10 @@ MPSX_DEV bool form_group(int *state, int G, int spread) {
     int s = __hip_atomic_fetch_add(state, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
     const long long start = wall_clock64(), limit = kFormTicks * (1 + (spread & 3));
     while (true) {
-        if (s & kGroupLost) return false;
+        if (s & EIG_GROUP_LOST) return false;
         if (s >= G) return true;
         if (wall_clock64() - start > limit) {
-            if (__hip_atomic_compare_exchange_strong(state, &s, s | kGroupLost, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+            if (__hip_atomic_compare_exchange_strong(state, &s, s | EIG_GROUP_LOST, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT))
                 return false;
             continue;  // s is the newer value
@@ -772,7 +771,7 @@ k_tridiag_one(const mpsx_two_site_op *ops, char *ws, int max_n) {
     __shared__ TriShared<EIG_MAX_N, 1> sm;
     const mpsx_plan p = ops[blockIdx.x].plan;
     if (!eig_direct(p, max_n)) return;
-    if (!(reinterpret_cast<const ProblemCtl *>(ws + p.ws_off)->group & kGroupLost)) return;
+    if (!(reinterpret_cast<const ProblemCtl *>(ws + p.ws_off)->group & EIG_GROUP_LOST)) return;
     switch (eig_class(p.C)) {
         case 0: break;  // a group of one
         case 1: tridiag<4, 8, true>(p, ws, 0, 1, sm); break;

@@ -21,8 +21,9 @@ hipError_t launch_gemm_rows(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gem
 // max_n: rows up to which the Gram problems take the direct eigensolver
 // (eig_direct; 0: none do). small: 1 when the one-workgroup kernel takes the
 // problems small_route selects; the others of these launches pass them by.
+// group: what ProblemCtl.group starts from (0, or EIG_GROUP_LOST).
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows, int max_n, int small);
+                            int64_t rows, int max_n, int small, int group);
 hipError_t launch_theta(hipStream_t s, bool f32, int D, const mpsx_two_site_op *d, int count, char *ws,
                         int64_t tiles);
 hipError_t launch_theta_gen(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,

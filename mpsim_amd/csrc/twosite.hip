@@ -70,7 +70,7 @@ MPSX_DEV double block_sum_256(double v, double *red) {
 // rows <- 0. Row 0 of each problem also resets its control block.
 template <class T>
 __global__ void __launch_bounds__(256)
-k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n, int small) {
+k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n, int small, int group) {
     using Z2 = typename Cx<T>::type;
     if (blockIdx.x == 0 && threadIdx.x < 64) {
         reinterpret_cast<TwoSiteHeader *>(ws)->active[threadIdx.x] = 0;
@@ -101,7 +101,7 @@ k_init_rows(const mpsx_two_site_op *ops, int count, char *ws, int max_n, int sma
         ctl->counter = 0;
         ctl->conv = (p.C == 0 || p.R == 0 || direct) ? 1 : 0;
         ctl->sweeps = 0;
-        ctl->group = 0;
+        ctl->group = group;
     }
 }
 
@@ -2098,15 +2098,15 @@ k_gather(const mpsx_two_site_op *ops, int count, char *ws, int small) {
 // ---------------------------------------------------------------- launchers
 template <class T>
 static void launch_init_rows_t(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                               int64_t rows, int max_n, int small) {
-    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n, small);
+                               int64_t rows, int max_n, int small, int group) {
+    hipLaunchKernelGGL(k_init_rows<T>, dim3((unsigned)rows), dim3(256), 0, s, d, count, ws, max_n, small, group);
 }
 hipError_t launch_init_rows(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
-                            int64_t rows, int max_n, int small) {
+                            int64_t rows, int max_n, int small, int group) {
     if (f32)
-        launch_init_rows_t<float>(s, d, count, ws, rows, max_n, small);
+        launch_init_rows_t<float>(s, d, count, ws, rows, max_n, small, group);
     else
-        launch_init_rows_t<double>(s, d, count, ws, rows, max_n, small);
+        launch_init_rows_t<double>(s, d, count, ws, rows, max_n, small, group);
     return hipGetLastError();
 }
 

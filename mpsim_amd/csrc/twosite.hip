@@ -1194,11 +1194,10 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
         ctl->conv = 0;
         ctl->counter = 0;
     }
-    if ((int)blockIdx.y > p.nb) return;
     const int nb = p.nb;
-    for (int tile = (int)(blockIdx.x - p.pair_base) * (p.nb + 1) + (int)blockIdx.y; tile < nb * (nb + 1) / 2;
-         tile += p.nb / 2 * (p.nb + 1)) {
-    int rem = tile, bi = 0;
+    if ((int)blockIdx.y > nb) return;
+    int rem = (int)(blockIdx.x - p.pair_base) * (nb + 1) + (int)blockIdx.y;
+    int bi = 0;
     while (rem >= nb - bi) {
         rem -= nb - bi;
         ++bi;
@@ -1245,8 +1244,6 @@ k_hgram(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
         h_store<true>(ws, p, idx, v);
     else
         h_ptr(ws, p)[idx] = v;
-    __syncthreads();  // part is read before the next tile
-    }
 }
 
 // Workgroup size of the eigensolve kernel (eight waves measured slower than
@@ -1791,8 +1788,7 @@ k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int ldx = MODE == 0 ? R : LD;
     double2 *Out = MODE == 0 ? Z : t64_ptr(ws, p);
     const int ldo = MODE == 0 ? LD : R;
-    const int rows = 16 * p.nb;
-    for (int row0 = (int)(blockIdx.x - p.pair_base) * 32 + 16 * tm; row0 < rows; row0 += 16 * p.nb) {
+    const int row0 = (int)(blockIdx.x - p.pair_base) * 32 + 16 * tm;
     const double2 *yrow = Z + (int64_t)(row0 + l16) * LD + R;  // A = Y[row0 + l16][k]
     mfma_d4 a1 = {0.0, 0.0, 0.0, 0.0}, a2 = a1, a3 = a1;
     for (int k0 = 0; k0 < Cp; k0 += 16) {
@@ -1815,7 +1811,6 @@ k_hxgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
         for (int r = 0; r < 4; ++r)
             Out[(int64_t)(row0 + 4 * r + lq) * ldo + col] =
                 make_double2(a1[r] - a2[r], a3[r] - a1[r] - a2[r]);
-    }
     }
 }
 
@@ -1850,9 +1845,9 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     }
     const bool gram = MODE <= 1;
     const int Cp = p.Cp, R = p.R, LD = p.LD;
-    const int j0 = (int)blockIdx.y * TM;
+    const int i0 = (int)(blockIdx.x - p.pair_base) * TM, j0 = (int)blockIdx.y * TM;
     const int ncols = gram ? Cp : R, K = gram ? R : Cp;
-    if (j0 >= ncols) return;
+    if (i0 >= Cp || j0 >= ncols || (gram && j0 < i0)) return;
     double2 *Z = z_ptr<double>(ws, p);
     // row-major sources: A rows (length K), and for the Gram the rows of X
     // that form B = X^H; for MODES 2, 3 B = X[k][j]
@@ -1863,8 +1858,6 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, lq = lane >> 4;
     const int wm = wave >> 1, wn = wave & 1;
-    for (int i0 = (int)(blockIdx.x - p.pair_base) * TM; i0 < Cp; i0 += TM * (p.nb / 2)) {
-    if (gram && j0 < i0) break;
     mfma_d4 acc[2][2][3];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -1940,7 +1933,6 @@ k_hgemm(const mpsx_two_site_op *ops, const int *owner, char *ws, int max_n) {
                     t64_ptr(ws, p)[(int64_t)i * R + j] = v;
                 }
             }
-    }
 }
 
 // Round workgroup -> problem table (one workgroup per problem), so that the

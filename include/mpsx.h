@@ -166,8 +166,11 @@ typedef struct {
     mpsx_plan plan;    /* library-owned, see mpsx_two_site_plan          */
 } mpsx_two_site_op;
 
-/* max_sweeps, check_every, inner_sweeps, tol and unconverged concern the
- * problems that iterate; the direct solver does not. */
+/* max_sweeps, check_every and inner_sweeps concern the problems whose sweeps the
+ * host launches: the one-sided rounds and the Gram method's beyond the direct
+ * solver. The one-workgroup kernel of small problems repeats on the device, up to
+ * 30 passes, until the rows are orthogonal within tol; the direct solver does
+ * not iterate. */
 typedef struct {
     int32_t block;      /* Jacobi block width b (pivot is 2b x 2b); 0 = auto  */
     int32_t max_sweeps; /* outer sweep limit; 0 = default (30)              */
@@ -181,9 +184,11 @@ typedef struct {
     int32_t rotation_fp32;/* 0: FP64 working matrix (default; tol default
                            1e-7); 1: FP32 working matrix (tol default 1e-5) */
     int32_t *unconverged;/* device int or NULL: incremented once per problem
-                           whose last launched sweep still rotated (the
-                           device-side status when check_every = 0); the
-                           caller zeroes it                                 */
+                           whose last launched sweep still rotated, whose
+                           30 passes in one workgroup were not enough or whose
+                           direct solve gave up a wait (the device-side
+                           status when check_every = 0); the caller zeroes
+                           it                                               */
     int32_t method;     /* MPSX_SVD_AUTO (0): the Gram method for FP64
                            problems with b = 16 and nb >= 6 (more than 64
                            rows), rows otherwise;
@@ -227,7 +232,9 @@ int mpsx_two_site_plan(mpsx_two_site_op *h, int count,
 
 /* Batched two-site update. Problems are independent (disjoint site pairs,
  * possibly of different circuits). `sweeps_out` (host, may be NULL)
- * receives the number of outer sweeps launched. The kernels work in `ws`
+ * receives the number of outer sweeps launched. Returns MPSX_ENOTCONV if a
+ * problem did not converge (with check_every = 0 and under capture only
+ * opts->unconverged says so); for that it waits for the stream. The kernels work in `ws`
  * until the stream gets past them, which may be after the call returns: a call
  * on another stream that uses the same `ws` is ordered behind by the caller. */
 int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h,
@@ -235,15 +242,27 @@ int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h,
                   const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
                   int *sweeps_out);
 
+/* mpsx_two_site without the wait at its end: it waits only where sweeps are polled.
+ * A problem of the one-workgroup kernel or the direct solver that does not
+ * converge sets *late to 1 (pinned host memory, or NULL), which the host may read
+ * once the stream has got past the call, and clears itself. */
+int mpsx_two_site_async(mpsx_stream stream, const mpsx_two_site_op *h,
+                        const mpsx_two_site_op *d, int count,
+                        const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
+                        int *sweeps_out, int *late);
+
 /* mpsx_two_site made to take, for tests, a route that a call otherwise takes only
  * on some devices or under load. Every kernel ends as it does without.
  *   ROUNDS  the Gram problems of up to 1024 rows take the Jacobi rounds (plan.method
  *           3: behind the QR) instead of the direct solver, as in calls of more
  *           than 65535 problems and on partitions of few compute units;
  *   LOST    the direct solver's groups of workgroups are given up from the start, as
- *           when several launches keep each other from forming theirs. */
+ *           when several launches keep each other from forming theirs;
+ *   TIMEOUT a wait inside a group ends at its first look, as after some seconds
+ *           otherwise: its problem is reported as not converged. */
 #define MPSX_FORCE_ROUNDS 1
 #define MPSX_FORCE_LOST 2
+#define MPSX_FORCE_TIMEOUT 4
 
 int mpsx_two_site_forced(mpsx_stream stream, const mpsx_two_site_op *h,
                          const mpsx_two_site_op *d, int count,

@@ -65,7 +65,7 @@ class NotConvergedWarning(RuntimeWarning):
 
 EXPORTS = ("mpsx_version", "mpsx_last_error", "mpsx_device_info", "mpsx_sizeof",
            "mpsx_put", "mpsx_apply_one_site", "mpsx_apply_one_site_now", "mpsx_two_site_plan",
-           "mpsx_two_site", "mpsx_two_site_forced", "mpsx_two_site_static",
+           "mpsx_two_site", "mpsx_two_site_async", "mpsx_two_site_forced", "mpsx_two_site_static",
            "mpsx_gemm",
            "mpsx_scale", "mpsx_profile_enable", "mpsx_profile_read", "mpsx_profile_busy",
            "mpsx_graph_begin", "mpsx_graph_end", "mpsx_graph_launch", "mpsx_graph_destroy")
@@ -96,6 +96,7 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
         lib.mpsx_two_site_plan.argtypes = [vp, i32, ctypes.POINTER(SvdOpts), ctypes.POINTER(sz)]
         lib.mpsx_two_site.argtypes = [vp, vp, vp, i32, ctypes.POINTER(SvdOpts), vp, sz,
                                       ctypes.POINTER(i32)]
+        lib.mpsx_two_site_async.argtypes = lib.mpsx_two_site.argtypes + [vp]
         lib.mpsx_two_site_forced.argtypes = lib.mpsx_two_site.argtypes + [i32]
         lib.mpsx_two_site_static.argtypes = [vp, vp, vp, i32, ctypes.POINTER(SvdOpts),
                                              ctypes.POINTER(i32)]
@@ -112,7 +113,7 @@ def load(path: Optional[str] = None) -> ctypes.CDLL:
         lib.mpsx_graph_destroy.argtypes = [vp]
         for name in ("mpsx_put", "mpsx_apply_one_site", "mpsx_apply_one_site_now",
                      "mpsx_two_site_plan", "mpsx_two_site",
-                     "mpsx_two_site_forced", "mpsx_two_site_static", "mpsx_gemm",
+                     "mpsx_two_site_async", "mpsx_two_site_forced", "mpsx_two_site_static", "mpsx_gemm",
                      "mpsx_scale", "mpsx_device_info", "mpsx_profile_enable",
                      "mpsx_profile_read", "mpsx_profile_busy", "mpsx_graph_begin", "mpsx_graph_end",
                      "mpsx_graph_launch", "mpsx_graph_destroy"):
@@ -160,7 +161,7 @@ def to_device_table(table: np.ndarray, dev):
     return raw.to(dev, non_blocking=False)
 
 
-FORCE_ROUNDS, FORCE_LOST = 1, 2  # MPSX_FORCE_*
+FORCE_ROUNDS, FORCE_LOST, FORCE_TIMEOUT = 1, 2, 4  # MPSX_FORCE_*
 PUT_MAX = 16384  # MPSX_PUT_MAX
 SITE_NOW = 16    # MPSX_SITE_NOW
 

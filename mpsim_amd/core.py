@@ -244,13 +244,13 @@ class MPS:
 
     def get_nodes(self, copy: bool = True) -> List[Node]:
         """Host copies of the site tensors as Nodes ([chi_l, d, chi_r])."""
-        return [Node(t.detach().cpu().numpy(), name=self._prefix + str(i))
+        return [Node(self._engine.host(t.detach()), name=self._prefix + str(i))
                 for i, t in enumerate(self._tensors)]
 
     def get_node(self, node_index: int, copy: bool = True) -> Node:
         t = self._tensors[node_index]
         i = node_index % self._nqudits
-        return Node(t.detach().cpu().numpy(), name=self._prefix + str(i))
+        return Node(self._engine.host(t.detach()), name=self._prefix + str(i))
 
     def get_free_edge_of(self, node_index: int, copy: bool = True) -> Edge:
         """core.py:443-451: the physical leg of a site (axis 1 of the
@@ -272,7 +272,7 @@ class MPS:
         """core.py:483-500: psi with site 0 the most significant digit."""
         if not self.is_valid():
             raise ValueError("MPS is not valid.")
-        return self._wavefunction_device().cpu().numpy()
+        return self._engine.host(self._wavefunction_device())
 
     def _wavefunction_device(self):
         torch = self._engine.torch
@@ -305,7 +305,7 @@ class MPS:
             raise ValueError("MPS is invalid.")
         if not other.is_valid():
             raise ValueError("Other MPS is invalid.")
-        return complex(self._inner_device(other).item())
+        return complex(self._engine.host(self._inner_device(other)))
 
     def _inner_device(self, other: "MPS"):
         """E[y, x] = sum conj(other) self over the sites left of the cut."""
@@ -361,7 +361,7 @@ class MPS:
         if min(idx) < 0 or max(idx) > self._nqudits - 1:
             raise IndexError("One or more invalid node indices.")
         kept = sorted(idx)
-        rho = self._rdm_device(kept).cpu().numpy()
+        rho = self._engine.host(self._rdm_device(kept))
         m, d = len(kept), self._qudit_dimension
         pos = [kept.index(i) for i in idx]
         rho = rho.reshape([d] * (2 * m)).transpose(pos + [m + p for p in pos])
@@ -482,7 +482,7 @@ class MPS:
     def _marginal_probabilities(self) -> np.ndarray:
         """float32 [n, d] marginals with rounding-level negatives set to zero
         (a zero-probability value can come out as -1e-9 in FP32)."""
-        p = self._marginals_device().cpu().numpy().astype(np.float32)
+        p = self._engine.host(self._marginals_device()).astype(np.float32)
         p[(p < 0) & (p > -1e-6)] = 0.0
         return p
 
@@ -550,7 +550,7 @@ class MPS:
         full = min(M, N)
         res = self._engine.two_site([SplitItem(mat, full, absorb_left, want_s=True)])[0]
         err = threshold * self.norm()
-        s = res.s.double().cpu().numpy() if full else np.zeros(0)
+        s = self._engine.host(res.s.double()) if full else np.zeros(0)
         tails = np.sqrt(np.cumsum(np.square(s[::-1])))
         keep = min(full, int(np.count_nonzero(tails > err)))
         a = res.a_out.reshape(M, full)[:, :keep].contiguous()
@@ -813,7 +813,7 @@ class MPS:
         for a, b in zip(self._tensors, other._tensors):
             if tuple(a.shape) != tuple(b.shape):
                 return False
-            if not np.allclose(a.cpu().numpy(), b.cpu().numpy()):
+            if not np.allclose(self._engine.host(a), self._engine.host(b)):
                 return False
         return True
 

@@ -461,10 +461,11 @@ namespace {
 // The two-site driver behind mpsx_two_site. `may_poll` false: never read
 // device memory back (no convergence poll; the sweep limit and the
 // device-side early exit bound the work) and create no profiling events.
-// `force`: MPSX_FORCE_* bits.
+// `late`: set by the kernels of problems that the polls do not cover (nothing if
+// null); `wait`: their status is waited for instead. `force`: MPSX_FORCE_* bits.
 int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_site_op *d,
                  int count, const Resolved &r, char *ws, size_t ws_bytes, int *sweeps_out,
-                 bool may_poll, size_t *need_out = nullptr, int force = 0) {
+                 bool may_poll, size_t *need_out, int *late, bool wait, int force) {
     if (sweeps_out) *sweeps_out = 0;
     if (count < 0) return fail(MPSX_EINVAL, "count < 0");
     if (count == 0) return MPSX_OK;
@@ -563,6 +564,15 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     const bool can_poll = may_poll && r.check_every > 0 && cap == hipStreamCaptureStatusNone;
 
     const bool f32 = r.fp32;
+    // the kernels that iterate (or wait) on the device alone say so in a word of
+    // pinned memory
+    wait = wait && can_poll && (has_small || eig_slots > 0);
+    if (wait) {
+        int *buf = poll_buffer();
+        if (!buf) return fail(MPSX_EHIP, "hipHostMalloc of the poll buffer failed");
+        late = buf + 1;
+        __atomic_store_n(late, 0, __ATOMIC_RELAXED);
+    }
     const int group0 = (force & MPSX_FORCE_LOST) ? EIG_GROUP_LOST : 0;
     const bool rest = rows > 0 && other;  // some problem takes the launch sequence below
     if (rest) HIP_TRY(timed("k_init_rows", stream, [&] { return launch_init_rows(stream, f32, d, count, ws, rows, max_n, small, group0); }), "k_init_rows");
@@ -573,7 +583,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     if (has_gen && tiles > 0) HIP_TRY(timed("k_theta", stream, [&] { return launch_theta_gen(stream, f32, d, count, ws, tiles); }), "k_theta");
     if (has_small)
         HIP_TRY(timed("k_small", stream,
-                      [&] { return launch_small(stream, d, count, ws, r.tol, r.null_rel, r.unconverged); }),
+                      [&] { return launch_small(stream, d, count, ws, r.tol, r.null_rel, r.unconverged, late); }),
                 "k_small");
     // the norms of theta: for the convergence tests of the problems that iterate
     if (rest && (rows_nb > 0 || has_rounds)) {
@@ -606,7 +616,8 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     if (eig_slots > 0) {
         HIP_TRY(timed("k_hgram", stream, [&] { return launch_eig_gram(stream, d, count, ws, max_n, eig_n); }), "k_eig_gemm");
         HIP_TRY(timed("k_tridiag", stream,
-                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128); }),
+                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128,
+                                                  (force & MPSX_FORCE_TIMEOUT) != 0); }),
                 "k_tridiag");
         HIP_TRY(timed("k_eig_conquer", stream,
                       [&] { return launch_eig_conquer(stream, d, count, ws, max_n, eig_n); }),
@@ -725,12 +736,17 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     }
     if (rest) {
         HIP_TRY(timed("k_rownorm", stream, [&] { return launch_rownorm(stream, f32, d, count, ws, rows, small); }), "k_rownorm");
-        HIP_TRY(timed("k_sort", stream, [&] { return launch_sort(stream, d, count, ws, r.unconverged, small); }), "k_sort");
+        HIP_TRY(timed("k_sort", stream, [&] { return launch_sort(stream, d, count, ws, r.unconverged, late, max_n, small); }), "k_sort");
         if (outs > 0) HIP_TRY(timed("k_gather", stream, [&] { return launch_gather(stream, f32, d, count, ws, outs, small); }), "k_gather");
     }
     if (sweeps_out) *sweeps_out = sweeps;
     if (can_poll && !converged)
         return fail(MPSX_ENOTCONV, "Jacobi SVD not converged after %d sweeps", sweeps);
+    if (wait) {
+        HIP_TRY(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        if (__atomic_load_n(late, __ATOMIC_ACQUIRE))
+            return fail(MPSX_ENOTCONV, "SVD of a small or direct problem not converged");
+    }
     return MPSX_OK;
 }
 
@@ -743,7 +759,7 @@ int mpsx_internal_two_site(hipStream_t stream, const mpsx_two_site_op *h,
                            char *ws, size_t ws_bytes, int *sweeps_out, bool may_poll,
                            size_t *need_out) {
     return two_site_run(stream, h, d, count, resolve(opts), ws, ws_bytes, sweeps_out, may_poll,
-                        need_out);
+                        need_out, nullptr, false, 0);
 }
 
 int mpsx_internal_fail(int code, const char *msg) { return fail(code, "%s", msg); }
@@ -754,16 +770,23 @@ int mpsx_two_site(mpsx_stream stream, const mpsx_two_site_op *h, const mpsx_two_
                   int count, const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
                   int *sweeps_out) {
     return two_site_run((hipStream_t)stream, h, d, count, resolve(opts), static_cast<char *>(ws),
-                        ws_bytes, sweeps_out, true);
+                        ws_bytes, sweeps_out, true, nullptr, nullptr, true, 0);
+}
+
+int mpsx_two_site_async(mpsx_stream stream, const mpsx_two_site_op *h, const mpsx_two_site_op *d,
+                        int count, const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
+                        int *sweeps_out, int *late) {
+    return two_site_run((hipStream_t)stream, h, d, count, resolve(opts), static_cast<char *>(ws),
+                        ws_bytes, sweeps_out, true, nullptr, late, false, 0);
 }
 
 int mpsx_two_site_forced(mpsx_stream stream, const mpsx_two_site_op *h, const mpsx_two_site_op *d,
                          int count, const mpsx_svd_opts *opts, void *ws, size_t ws_bytes,
                          int *sweeps_out, int force) {
-    if (force & ~(MPSX_FORCE_ROUNDS | MPSX_FORCE_LOST))
+    if (force & ~(MPSX_FORCE_ROUNDS | MPSX_FORCE_LOST | MPSX_FORCE_TIMEOUT))
         return fail(MPSX_EINVAL, "unknown force bits 0x%x", force);
     return two_site_run((hipStream_t)stream, h, d, count, resolve(opts), static_cast<char *>(ws),
-                        ws_bytes, sweeps_out, true, nullptr, force);
+                        ws_bytes, sweeps_out, true, nullptr, nullptr, true, force);
 }
 
 

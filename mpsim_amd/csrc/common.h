@@ -221,6 +221,11 @@ MPSX_HD int64_t problem_bytes(const mpsx_plan &p) {
     return align_up(t_off(p) - p.ws_off + 16 * h_elems(p), 256);
 }
 
+// Sets a word that the host reads (pinned memory), or nothing if it is null.
+MPSX_DEV void tell_host(int *word) {
+    if (word) __hip_atomic_store(word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Sort key: NaN below everything, so that ranks are a permutation.
 MPSX_DEV double sort_key(double x) { return x == x ? x : -__builtin_huge_val(); }
 

@@ -310,9 +310,10 @@ MPSX_DEV void tri_rows_alone(double2 (&a)[RW][2], const double2 *v, const double
 }
 
 // MEM: one workgroup, the matrix copied to the Y rows (which hold no slots
-// then); every sum is formed in the same order as by a group.
+// then); every sum is formed in the same order as by a group. spin_limit: looks at a
+// slot after which the group is reported as not converged.
 template <int CH, int RW, bool MEM, class SM>
-MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
+MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, int spin_limit, SM &sm) {
     constexpr int VW = CH > 4 ? 8 : 4;        // waves that hold the vectors
     constexpr int EPT = CH > VW ? CH / VW : 1;  // vector elements per thread of theirs
     constexpr int NG = RW < 4 ? RW : 4;       // rows per reduction
@@ -416,7 +417,7 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
                     here[s] = i < j || i >= n;
                     b[s][0] = b[s][1] = b[s][2] = b[s][3] = 0;
                 }
-                int spin = failed ? kSpin : 0;
+                int spin = failed ? spin_limit : 0;
                 while (true) {
 #pragma unroll
                     for (int s = 0; s < EPT; ++s)
@@ -431,7 +432,7 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
                         all = all && here[s];
                     }
                     if (all) break;
-                    if (++spin > kSpin) {
+                    if (++spin > spin_limit) {
                         sm.fail = 1;
                         break;
                     }
@@ -570,6 +571,7 @@ MPSX_DEV void tridiag(const mpsx_plan &p, char *ws, int member, int G, SM &sm) {
         if (alone) __syncthreads();
     }
     if (!LANES && nref > 0) panel(nref - 1, sm.v[cur]);
+    if (!alone && tid == 0 && sm.fail) reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->conv = 0;
     if (member != 0) return;
     if (tid == 0) *ev.nref = nref;
     if (nref < n - 1 || sm.stop)
@@ -742,7 +744,7 @@ k_eig_map(const mpsx_two_site_op *ops, int count, int2 *map, int max_n) {
 }
 
 __global__ void __launch_bounds__(512, 2)
-k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
+k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int spin_limit) {
     __shared__ TriShared<128, 8> sm;
     if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
     __syncthreads();
@@ -757,10 +759,10 @@ k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots) {
     __syncthreads();
     if (!sm.whole) return;
     switch (eig_class(p.C)) {
-        case 0: tridiag<2, 16, false>(p, ws, member, G, sm); break;
-        case 1: tridiag<4, 8, false>(p, ws, member, G, sm); break;
-        case 2: tridiag<8, 4, false>(p, ws, member, G, sm); break;
-        default: tridiag<16, 2, false>(p, ws, member, G, sm); break;
+        case 0: tridiag<2, 16, false>(p, ws, member, G, spin_limit, sm); break;
+        case 1: tridiag<4, 8, false>(p, ws, member, G, spin_limit, sm); break;
+        case 2: tridiag<8, 4, false>(p, ws, member, G, spin_limit, sm); break;
+        default: tridiag<16, 2, false>(p, ws, member, G, spin_limit, sm); break;
     }
 }
 
@@ -774,9 +776,9 @@ k_tridiag_one(const mpsx_two_site_op *ops, char *ws, int max_n) {
     if (!(reinterpret_cast<const ProblemCtl *>(ws + p.ws_off)->group & EIG_GROUP_LOST)) return;
     switch (eig_class(p.C)) {
         case 0: break;  // a group of one
-        case 1: tridiag<4, 8, true>(p, ws, 0, 1, sm); break;
-        case 2: tridiag<8, 4, true>(p, ws, 0, 1, sm); break;
-        default: tridiag<16, 2, true>(p, ws, 0, 1, sm); break;
+        case 1: tridiag<4, 8, true>(p, ws, 0, 1, 0, sm); break;
+        case 2: tridiag<8, 4, true>(p, ws, 0, 1, 0, sm); break;
+        default: tridiag<16, 2, true>(p, ws, 0, 1, 0, sm); break;
     }
 }
 
@@ -1266,10 +1268,10 @@ k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
 
 // ---------------------------------------------------------------- launchers
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots, bool grouped) {
+                              int slots, bool grouped, bool no_wait) {
     hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, static_cast<int2 *>(map), max_n);
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)slots), dim3(512), 0, s, d, static_cast<const int2 *>(map), ws,
-                       slots);
+                       slots, no_wait ? 0 : kSpin);
     if (grouped)
         hipLaunchKernelGGL(k_tridiag_one, dim3((unsigned)count), dim3(512), 0, s, d, ws, max_n);
     return hipGetLastError();

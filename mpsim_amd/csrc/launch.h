@@ -38,13 +38,14 @@ hipError_t launch_jacobi_round(hipStream_t s, bool f32, int b, const mpsx_two_si
                                int inner_sweeps);
 hipError_t launch_sweep_end(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
                             int sweep, bool fp32_phase, int small);
+// unconverged, late: mpsx_svd_opts.unconverged and mpsx_two_site_async's word.
 hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                       int *unconverged, int small);
+                       int *unconverged, int *late, int max_n, int small);
 hipError_t launch_gather(hipStream_t s, bool f32, const mpsx_two_site_op *d, int count, char *ws,
                          int64_t outs, int small);
 // The one-workgroup kernel (small.hip), from theta to the factors.
 hipError_t launch_small(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, double tol, double null_rel,
-                        int *unconverged);
+                        int *unconverged, int *late);
 hipError_t launch_hgram(hipStream_t s, const mpsx_two_site_op *d, const int *owner, char *ws,
                         int64_t pairs, int max_nb, int stage, int max_n);
 hipError_t launch_hsolve(hipStream_t s, bool f32h, const mpsx_two_site_op *d, const int *owner, char *ws,
@@ -70,10 +71,11 @@ hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, c
                           int strips, int max_c, bool small, bool large, int max_n);
 // Direct eigensolver (eig.hip) of the problems eig_direct selects: the
 // tridiagonal form (`map`: room for `slots` int2, the workgroups of all their
-// groups; `grouped`: some group has more than one), the eigensystem of T, and Y. n: the largest C among them; `small`,
+// groups; `grouped`: some group has more than one; `no_wait`: a group's waits end at
+// their first look), the eigensystem of T, and Y. n: the largest C among them; `small`,
 // `large`: some of at most 512 rows, some above.
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots, bool grouped);
+                              int slots, bool grouped, bool no_wait);
 // H = X X^H, and at the end X <- Y X (tiles: 32 x 32 ones of the largest X).
 hipError_t launch_eig_gram(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
 hipError_t launch_eig_apply(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n,

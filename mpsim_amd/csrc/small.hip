@@ -35,6 +35,7 @@
 namespace {
 
 constexpr int SN = 64;    // rows
+constexpr int kPasses = 30;  // then the problem is reported as not converged
 constexpr int ST = LEAF_THREADS;  // 512
 constexpr int SW = ST / 64;
 
@@ -448,7 +449,7 @@ MPSX_DEV void small_apply(double2 *Z, int64_t LD, int rows, int n, int R, bool f
 
 // One workgroup per problem; theta (X) is in the workspace.
 __global__ void __launch_bounds__(ST, 2)
-k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int *unconverged) {
+k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int *unconverged, int *late) {
     __shared__ SmallShared sm;
     const mpsx_two_site_op &op = ops[blockIdx.x];
     const mpsx_plan p = op.plan;
@@ -458,7 +459,7 @@ k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int 
     double2 *Z = reinterpret_cast<double2 *>(ws + z_off(p));
     double null2 = 0.0;
     bool first = true, done = false;
-    for (int it = 0; it < 30 && !done; ++it) {
+    for (int it = 0; it < kPasses && !done; ++it) {
         small_gram(Z, LD, n, R, sm);
         if (it == 0) {
             const double fro2 = wave_sum64(lane < n ? sm.A[lane][lane].x : 0.0);
@@ -529,7 +530,10 @@ k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int 
         small_apply(Z, LD, n, m, R, first, sm);
         first = false;
     }
-    if (!done && tid == 0 && unconverged) atomicAdd(unconverged, 1);
+    if (!done && tid == 0) {
+        if (unconverged) atomicAdd(unconverged, 1);
+        tell_host(late);
+    }
 
     // norms, order, factors
     for (int row = wave; row < n; row += SW) {
@@ -581,7 +585,7 @@ k_small(const mpsx_two_site_op *ops, char *ws, double tol, double null_rel, int 
 }
 
 hipError_t launch_small(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, double tol, double null_rel,
-                        int *unconverged) {
-    hipLaunchKernelGGL(k_small, dim3((unsigned)count), dim3(ST), 0, s, d, ws, tol, null_rel, unconverged);
+                        int *unconverged, int *late) {
+    hipLaunchKernelGGL(k_small, dim3((unsigned)count), dim3(ST), 0, s, d, ws, tol, null_rel, unconverged, late);
     return hipGetLastError();
 }

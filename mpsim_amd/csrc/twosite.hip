@@ -1969,10 +1969,11 @@ __global__ void k_sweep_end(const mpsx_two_site_op *ops, int count, char *ws, in
 // ---------------------------------------------------------------- finalize
 // One workgroup per problem: stable descending order of the row norms
 // (ties keep the lower row index), singular values, discarded weight, and
-// a count of problems left unconverged (when `unconverged` is not null).
+// a count of problems left unconverged (when `unconverged` is not null; a
+// direct problem, which the host does not poll, tells it by `late`).
 constexpr int SORT_LDS = 4096, SORT_THREADS = 1024;
 __global__ void __launch_bounds__(SORT_THREADS)
-k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int small) {
+k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int *late, int max_n, int small) {
     __shared__ double sg[SORT_LDS];
     __shared__ double red[SORT_THREADS / 64];
     const int pi = blockIdx.x;
@@ -2027,8 +2028,10 @@ k_sort(const mpsx_two_site_op *ops, int count, char *ws, int *unconverged, int s
         for (int w = 0; w < SORT_THREADS / 64; ++w) disc += red[w];
     }
     if (threadIdx.x == 0 && op.discarded) *op.discarded = disc;
-    if (threadIdx.x == 0 && unconverged && p.nb >= 2 && !ctl_ptr(ws, p)->conv)
-        atomicAdd(unconverged, 1);
+    if (threadIdx.x == 0 && p.nb >= 2 && !ctl_ptr(ws, p)->conv) {
+        if (unconverged) atomicAdd(unconverged, 1);
+        if (eig_direct(p, max_n)) tell_host(late);
+    }
     if (op.s_out)
         for (int j = threadIdx.x; j < k; j += SORT_THREADS) {
             op.s_out[j] = (float)sqrt(sig[perm[j]]);
@@ -2191,8 +2194,9 @@ hipError_t launch_sweep_end(hipStream_t s, const mpsx_two_site_op *d, int count,
 }
 
 hipError_t launch_sort(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws,
-                       int *unconverged, int small) {
-    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(SORT_THREADS), 0, s, d, count, ws, unconverged, small);
+                       int *unconverged, int *late, int max_n, int small) {
+    hipLaunchKernelGGL(k_sort, dim3((unsigned)count), dim3(SORT_THREADS), 0, s, d, count, ws, unconverged, late,
+                       max_n, small);
     return hipGetLastError();
 }
 

@@ -5,6 +5,7 @@ there is no other implementation to fall back on.
 """
 from __future__ import annotations
 
+import ctypes
 import threading
 import warnings
 from collections import OrderedDict
@@ -141,6 +142,7 @@ class Engine:
     """Owns the device, a gate cache and a grow-only workspace."""
 
     _engines: Dict[int, "Engine"] = {}
+    _late_words: Dict[int, object] = {}  # per device, held until the process ends
     _lock = threading.Lock()
 
     def __init__(self, dev):
@@ -165,7 +167,15 @@ class Engine:
         # enqueued at a time, and a call on another stream than the last one's
         # waits for that to end.
         self._enqueue = threading.RLock()
+        # set by a kernel (pinned host memory) when a problem did not converge in a
+        # call that had returned by then; report() says so
+        idx = self.dev.index if self.dev.index is not None else 0
+        self._late_word = self._late_words.setdefault(
+            idx, torch.zeros(1, dtype=torch.int32, pin_memory=True))
+        self._late_ptr = self._late_word.data_ptr()
+        self._late = ctypes.c_int32.from_address(self._late_ptr)
         self._used = None           # stream of the last call
+        self._used_handle = -1
         self._used_end = None       # event: the last call's end on that stream
 
     @classmethod
@@ -209,17 +219,31 @@ class Engine:
         default stream, which outlives the engine, is recorded only when another
         stream takes over."""
         last = self._used
-        if last is not None and last.cuda_stream != cur.cuda_stream:
+        if last is not None:
             if not last.cuda_stream:
-                self._leave_workspaces(last, True)
+                self._leave_workspaces(last)
             cur.wait_event(self._used_end)
-        self._used = cur
+        self._used, self._used_handle = cur, int(cur.cuda_stream)
 
-    def _leave_workspaces(self, cur, now: bool = False) -> None:
-        if now or cur.cuda_stream:
-            if self._used_end is None:
-                self._used_end = self.torch.cuda.Event()
-            self._used_end.record(cur)
+    def _leave_workspaces(self, cur) -> None:
+        if self._used_end is None:
+            self._used_end = self.torch.cuda.Event()
+        self._used_end.record(cur)
+
+    def report(self) -> None:
+        """Warns (NotConvergedWarning) if the SVD of an update whose kernels have
+        ended did not converge after its call had returned. Every two-site call
+        and host() look; a caller that waits by other means may."""
+        if self._late.value:
+            self._late.value = 0
+            warnings.warn("the SVD of an earlier two-site update has not converged",
+                          nat.NotConvergedWarning, stacklevel=3)
+
+    def host(self, t) -> np.ndarray:
+        """The tensor on the host (waits for the current stream)."""
+        out = t.cpu().numpy()
+        self.report()
+        return out
 
     def gate(self, mat: np.ndarray):
         """Device complex64 copy of a gate matrix (cached by content)."""
@@ -264,7 +288,7 @@ class Engine:
 
     # ------------------------------------------------------------ two-site
     def _prepare_two_site(self, items: Sequence[TwoSiteItem], cfg, slot: int = 0,
-                          workspace: bool = True):
+                          workspace: bool = True, stream: Optional[int] = None):
         """Outputs, planned host table, device table and workspace (None with
         workspace=False) of one library call (allocations on the calling
         thread's current stream)."""
@@ -320,22 +344,20 @@ class Engine:
             s = (buf.view(torch.float32).as_strided((k,), (1,), 2 * int(la[i] + lb[i]))
                  if ns[i] else None)
             outs.append(TwoSiteResult(a_out, b_out, s, disc, i))
-        import ctypes
         nbytes = ctypes.c_size_t(0)
         nat.check(self.lib.mpsx_two_site_plan(tab.ctypes.data, n, ctypes.byref(cfg),
                                               ctypes.byref(nbytes)))
         ws = self.workspace(nbytes.value, slot) if workspace else None
-        dtab = nat.put_table(tab, self.dev, self.stream)
+        dtab = nat.put_table(tab, self.dev, self.stream if stream is None else stream)
         return outs, tab, dtab, ws
 
     def _run_two_site(self, tab, dtab, ws, cfg, stream: int) -> int:
-        """The library call itself (blocking while it polls convergence);
-        returns the sweeps it ran."""
-        import ctypes
+        """The library call itself (blocking while it polls convergence; report()
+        covers what it does not poll); returns the sweeps it ran."""
         sweeps = ctypes.c_int(0)
-        code = self.lib.mpsx_two_site(stream, tab.ctypes.data, dtab.data_ptr(), len(tab),
-                                      ctypes.byref(cfg), ws.data_ptr(), ws.numel(),
-                                      ctypes.byref(sweeps))
+        code = self.lib.mpsx_two_site_async(stream, tab.ctypes.data, dtab.data_ptr(), len(tab),
+                                            ctypes.byref(cfg), ws.data_ptr(), ws.numel(),
+                                            ctypes.byref(sweeps), self._late_ptr)
         if code == nat.MPSX_ENOTCONV:
             warnings.warn(nat.load().mpsx_last_error().decode(), nat.NotConvergedWarning)
         else:
@@ -354,15 +376,19 @@ class Engine:
         threads are ordered: the workspaces are the engine's."""
         if len(items) == 0:
             return []
+        self.report()
         with self._enqueue:
             cur = self.torch.cuda.current_stream(self.dev)
-            self._take_workspaces(cur)
+            stream = int(cur.cuda_stream)
+            if stream != self._used_handle:
+                self._take_workspaces(cur)
             try:
-                return self._two_site(items, svd, cur)
+                return self._two_site(items, svd, cur, stream)
             finally:
-                self._leave_workspaces(cur)
+                if stream:
+                    self._leave_workspaces(cur)
 
-    def _two_site(self, items: Sequence[TwoSiteItem], svd: Optional[SvdConfig], cur
+    def _two_site(self, items: Sequence[TwoSiteItem], svd: Optional[SvdConfig], cur, stream: int
                   ) -> List[TwoSiteResult]:
         n = len(items)
         cfg = (svd or self.svd).to_c()
@@ -370,9 +396,9 @@ class Engine:
         big = [i for i, it in enumerate(items) if _rows(it) >= self.split_rows]
         ways = max(1, min(int(self.split_ways), n))
         if ways < 2 or len(big) < self.split_min or cfg.check_every == 0:
-            outs, tab, dtab, ws = self._prepare_two_site(items, cfg)
+            outs, tab, dtab, ws = self._prepare_two_site(items, cfg, stream=stream)
             self._keep = [dtab]
-            self.last_sweeps = self._run_two_site(tab, dtab, ws, cfg, int(cur.cuda_stream))
+            self.last_sweeps = self._run_two_site(tab, dtab, ws, cfg, stream)
             return outs
         # groups of equal estimated work (rows^2 * row length per problem),
         # largest problems first, each to the least loaded group
@@ -387,7 +413,7 @@ class Engine:
         preps = []
         for slot, g in enumerate(grp):
             c = cfg if slot == 0 else (svd or self.svd).to_c()
-            preps.append((c,) + self._prepare_two_site([items[i] for i in g], c, slot))
+            preps.append((c,) + self._prepare_two_site([items[i] for i in g], c, slot, stream=stream))
         self._keep = [p[3] for p in preps]
         torch = self.torch
         from concurrent.futures import ThreadPoolExecutor

@@ -31,6 +31,7 @@ structure can be written into them between runs (`update_gates`).
 from __future__ import annotations
 
 import ctypes
+import warnings
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
 
@@ -205,7 +206,9 @@ class CircuitProgram:
         self.arena.index_copy_(0, self._reset_idx, self._reset_val)
         self.unconverged.zero_()
 
-    def _launch_all(self, stream: int, record: bool) -> None:
+    def _launch_all(self, stream: int, record: bool) -> bool:
+        """Enqueues every call; returns whether one warned that it did not converge."""
+        warned = False
         lib = self.engine.lib
         base = int(self._tables.data_ptr())
         ws, wsn = int(self.workspace.data_ptr()), int(self.workspace.numel())
@@ -216,15 +219,16 @@ class CircuitProgram:
                 continue
             opts = self._opts(0 if record else cl.sweeps + self.margin)
             sweeps = ctypes.c_int(0)
-            code = lib.mpsx_two_site(stream, cl.host.ctypes.data, dptr, len(cl.host),
-                                     ctypes.byref(opts), ws, wsn, ctypes.byref(sweeps))
+            code = lib.mpsx_two_site_async(stream, cl.host.ctypes.data, dptr, len(cl.host),
+                                           ctypes.byref(opts), ws, wsn, ctypes.byref(sweeps), None)
             if code == nat.MPSX_ENOTCONV:
-                import warnings
+                warned = True
                 warnings.warn(lib.mpsx_last_error().decode(), nat.NotConvergedWarning)
             else:
                 nat.check(code)
             if record:
                 cl.sweeps = max(cl.sweeps, int(sweeps.value))
+        return warned
 
     def _capture(self) -> None:
         torch = self.engine.torch
@@ -255,10 +259,13 @@ class CircuitProgram:
         stream = self.engine.stream
         self._reset()
         if self._graph is None:
-            self._launch_all(stream, record=True)
+            warned = self._launch_all(stream, record=True)
             self.eager_runs += 1
             torch.cuda.synchronize(self.engine.dev)
             self.last_unconverged = int(self.unconverged.item())
+            if self.last_unconverged and not warned:  # in a problem that is not polled
+                warnings.warn(f"the SVD of {self.last_unconverged} two-site updates has not converged",
+                              nat.NotConvergedWarning)
             if self.use_graph:
                 self._capture()
             return

@@ -249,6 +249,7 @@ class MPSServer:
             raise shared.error
         torch.cuda.synchronize(self.engine.dev)
         wall = time.perf_counter() - t0
+        self.engine.report()
         done = shared.done
         lat = np.array([s.latency for s in done]) if done else np.zeros(1)
         ups = sum(s.updates for s in done)

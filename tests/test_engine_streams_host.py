@@ -4,6 +4,7 @@ than the last one's waits for that one's end, a replaced workspace stays with th
 stream that worked on it, and one thread enqueues at a time."""
 import threading
 import types
+import warnings
 
 import pytest
 
@@ -49,8 +50,9 @@ def _engine(log, need):
     eng._ws, eng._wss, eng._keep, eng._helpers = None, [], [], []
     eng.split_ways, eng.split_min, eng.split_rows = 1, 1, 1
     eng._enqueue, eng._used, eng._used_end = threading.RLock(), None, None
+    eng._used_handle, eng._late = -1, types.SimpleNamespace(value=0)
 
-    def prepare(items, cfg, slot=0, workspace=True):
+    def prepare(items, cfg, slot=0, workspace=True, stream=None):
         return list(items), [0], None, eng.workspace(need[0], slot)
 
     def run(tab, dtab, ws, cfg, stream):
@@ -79,6 +81,19 @@ def test_call_on_another_stream_waits_for_the_last(first, second):
     # each wait is for an event behind all the work of the stream before it
     assert ops == [("run", first), ("run", first), ("wait", second, (first, 2)), ("run", second),
                    ("wait", first, (second, 3)), ("run", first)]
+
+
+def test_late_report_warns_once():
+    from mpsim_amd._native import NotConvergedWarning
+    eng = _engine([], [2048])
+    eng.now = _Stream(0, [])
+    eng._late.value = 1  # a kernel of an earlier call
+    with pytest.warns(NotConvergedWarning):
+        eng.two_site([_item()])
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        eng.two_site([_item()])
+        eng.report()
 
 
 def test_one_default_stream_records_nothing():

@@ -123,7 +123,8 @@ MPSX_DEV int find_record(const char *table, int count, size_t stride, size_t fie
 struct TwoSiteHeader {
     int32_t active[64];  // active[s]: problems still unconverged after sweep s
     int32_t ticket;      // workgroups of k_tridiag started so far
-    int32_t pad[63];
+    int32_t spread;      // 0 .. 3, another than the launches before and after have: see form_group
+    int32_t pad[62];
 };
 
 // Per-problem control block inside the workspace.

@@ -27,6 +27,7 @@
 // at the end Y; the rotation region: the small vectors (EigVec).
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 
 #include "common.h"
@@ -118,8 +119,8 @@ MPSX_DEV int eig_levels(int n) {
 // workgroup may hold a compute unit that a missing member needs (each XCD
 // is dealt a fixed share of a launch, and several launches, each with an
 // incomplete group, can fill one), so that wait has an end: after
-// kFormTicks, spread over the launches so that they do not all give up
-// at once, the group is given up for good, its workgroups leave, and
+// kFormTicks, once to four times by the launch's turn so that launches under way
+// together do not all give up at once, the group is given up for good, its workgroups leave, and
 // k_tridiag_one does the problem. The flag and the count are one word (ctl->group), so a
 // group is either whole or given up for all its members.
 //
@@ -141,7 +142,7 @@ constexpr long long kFormTicks = 4000000;  // 40 ms at 100 MHz
 MPSX_DEV bool form_group(int *state, int G, int spread) {
     if (G == 1) return true;
     int s = __hip_atomic_fetch_add(state, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-    const long long start = wall_clock64(), limit = kFormTicks * (1 + (spread & 3));
+    const long long start = wall_clock64(), limit = kFormTicks * (1 + spread);
     while (true) {
         if (s & EIG_GROUP_LOST) return false;
         if (s >= G) return true;
@@ -713,11 +714,14 @@ k_eig_gemm(const mpsx_two_site_op *ops, char *ws, int max_n) {
 // Table of the workgroups of k_tridiag: entry s = (problem, member << 8 |
 // group size), the problems with the largest groups first. One workgroup.
 __global__ void __launch_bounds__(256)
-k_eig_map(const mpsx_two_site_op *ops, int count, int2 *map, int max_n) {
+k_eig_map(const mpsx_two_site_op *ops, int count, char *ws, int2 *map, int max_n, int spread) {
     __shared__ int wsum[4];
     __shared__ int total;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
-    if (tid == 0) total = 0;
+    if (tid == 0) {
+        total = 0;
+        reinterpret_cast<TwoSiteHeader *>(ws)->spread = spread;
+    }
     __syncthreads();
     for (int cls = 3; cls >= 0; --cls)
         for (int b = 0; b < count; b += 256) {
@@ -755,7 +759,7 @@ k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int
     const int member = m.y >> 8, G = m.y & 255;
     if (threadIdx.x == 0)
         sm.whole = form_group(&reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->group, G,
-                              (int)(reinterpret_cast<uintptr_t>(ws) >> 12));
+                              reinterpret_cast<const TwoSiteHeader *>(ws)->spread);
     __syncthreads();
     if (!sm.whole) return;
     switch (eig_class(p.C)) {
@@ -1269,7 +1273,9 @@ k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
 // ---------------------------------------------------------------- launchers
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
                               int slots, bool grouped, bool no_wait) {
-    hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, static_cast<int2 *>(map), max_n);
+    static std::atomic<unsigned> launches{0};
+    const int spread = (int)(launches.fetch_add(1, std::memory_order_relaxed) & 3);
+    hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, ws, static_cast<int2 *>(map), max_n, spread);
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)slots), dim3(512), 0, s, d, static_cast<const int2 *>(map), ws,
                        slots, no_wait ? 0 : kSpin);
     if (grouped)

@@ -150,3 +150,22 @@ def test_not_finite_inputs_stay_with_their_problem(bad):
     for i, r in enumerate(res[1::2]):
         # the values of a matrix that is not finite are not either
         assert not bool(torch.isfinite(r.s).all()), sizes[i]
+
+
+def test_launches_wait_for_their_groups_for_different_times():
+    """Four calls one after the other, each in its own workspace, have four different
+    limits (TwoSiteHeader.spread) wherever their workspaces lie."""
+    import torch
+    from mpsim_amd import _native as nat
+    from mpsim_amd.engine import Engine, SplitItem
+    eng = Engine.get()
+    m = torch.randn(200, 200, dtype=torch.complex64, device="cuda")
+    c = eng.svd.to_c()
+    seen = set()
+    for _ in range(4):
+        outs, tab, dtab, ws = eng._prepare_two_site([SplitItem(m, 200)], c)
+        ws = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+        nat.check(eng.lib.mpsx_two_site(eng.stream, tab.ctypes.data, dtab.data_ptr(), 1, ctypes.byref(c), ws.data_ptr(),
+                                        ws.numel(), None))
+        seen.add(int(ws[:512].view(torch.int32)[65].item()))
+    assert seen == {0, 1, 2, 3}

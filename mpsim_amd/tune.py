@@ -5,13 +5,14 @@
 Three stages, each timed on seeded synthetic two-site problems:
 
 1. Pivot size and inner sweeps. For each bond-size class, on a batch that
-   fills the device, every pair (pivot rows 2b in {16, 32}, inner
+   fills the device and with the one-sided rounds (by default the one-workgroup
+   kernel and the direct solver take these sizes, which have neither), every pair (pivot rows 2b in {16, 32}, inner
    eigensolver sweeps in {1, 2}); the pivot-size crossover becomes
    `block_switch` (problems with more rows than this use 32-row pivots) and
    the most frequent best inner-sweep count becomes `inner_sweeps`.
 2. SVD method. For the classes of 128 rows and more, the Gram method (the
-   library default for FP64 problems with 32-row pivots) against the
-   one-sided rows method, with stage 1's settings; `method` is the faster
+   library default for FP64 problems with 32-row pivots, by the direct solver up to
+   1024 rows) against the one-sided rows method, with stage 1's settings; `method` is the faster
    one on the largest class (where the time goes).
 3. Concurrency. A large call runs as `split_ways` groups on as many streams
    (Engine.two_site). On layer-shaped batches (one problem per disjoint
@@ -20,6 +21,11 @@ Three stages, each timed on seeded synthetic two-site problems:
    `split_rows` the smallest class from which splitting beats one group on
    every larger class too, and `split_min` the smallest batch of that class
    from which splitting beats one group.
+
+These batches hold problems of one size. Layers of mixed sizes, where a large
+problem's chain of steps would hold up the others, are not among them: a rule chosen
+from such layers is stored with `split_fixed`, and a re-tune then measures
+stage 3 but keeps the three values.
 
 Engine picks the stored values up as its defaults (tuned_config,
 tuned_engine). The library's compile-time tile shapes (theta tiles, 16-row
@@ -117,7 +123,7 @@ def _measure_split(engine, items, cfg: SvdConfig, ways: int, reps: int, timer: C
 
 
 def tune(engine=None, chis: Sequence[int] = (8, 16, 32, 64, 128, 256), reps: int = 2,
-         path: Optional[str] = TUNED, conc_chis: Sequence[int] = (64, 128, 256),
+         path: Optional[str] = TUNED, conc_chis: Sequence[int] = (64, 128, 192, 256),
          layer: int = 31, batch_sizes: Sequence[int] = (2, 4, 8, 16),
          timer: Callable = measure) -> Dict:
     """Runs the three stages and (with `path`) stores the result. `timer` is
@@ -133,7 +139,7 @@ def tune(engine=None, chis: Sequence[int] = (8, 16, 32, 64, 128, 256), reps: int
         best = None
         for block in (8, 16):
             for inner in (1, 2):
-                t = timer(eng, items, SvdConfig(block=block, inner_sweeps=inner), reps)
+                t = timer(eng, items, SvdConfig(block=block, inner_sweeps=inner, method=1), reps)
                 rec = {"stage": "pivot", "chi": chi, "rows": 2 * chi, "count": count, "block": block,
                        "inner_sweeps": inner, "us_per_update": round(1e6 * t, 2)}
                 rows.append(rec)
@@ -202,10 +208,14 @@ def tune(engine=None, chis: Sequence[int] = (8, 16, 32, 64, 128, 256), reps: int
                 if tw < t1:
                     split_min = n
                     break
+    stored = _load(path)
     out["split_ways"] = split_ways
     out["split_rows"] = split_rows
     out["split_min"] = split_min
-    out["precondition"] = int(_load(path).get("precondition", DEFAULT_PRECONDITION))
+    if stored.get("split_fixed"):
+        out["split_fixed"] = 1
+        out["split_ways"], out["split_min"], out["split_rows"] = tuned_engine(path)
+    out["precondition"] = int(stored.get("precondition", DEFAULT_PRECONDITION))
     out["measurements"] = rows
     if path:
         with open(path, "w") as f:

@@ -19,26 +19,27 @@ from . import _native as nat
 MAX_OPS = 65535  # descriptors per grouped launch (grid y / x limits of the kernels)
 
 
-def _tensor_info(t, what: str) -> Tuple[int, int]:
-    """(device address, elements) of a contiguous complex64 tensor."""
+def _tensor_info(t, what: str) -> Tuple[int, int, object]:
+    """(device address, elements, the tensor) of a contiguous complex64 tensor."""
     n = t.numel()
     if n and t.element_size() != 8:
         raise ValueError(f"gemm operand {what} must be complex64")
-    return nat.ptr(t), n
+    return nat.ptr(t), n, t
 
 
 def _matrix_addr(x, rows: int, cols: int, ld: int, what: str, seen: dict) -> int:
     """Device address of a rows x cols matrix with row stride `ld` stored in
     a contiguous complex64 tensor at an element offset (x = tensor or
     (tensor, offset)); raises if any element would fall outside it. seen: the
-    _tensor_info of the call's tensors so far (many products share one)."""
-    t, off = x if type(x) is tuple else (x, 0)
+    _tensor_info of the call's tensors so far (many products share one), which
+    holds them, so that an id stays one tensor's."""
+    t, off = x if isinstance(x, tuple) else (x, 0)
     info = seen.get(id(t))
     if info is None:
         if rows == 0 or cols == 0:
             return nat.ptr(t) + 8 * off if t.numel() else 0
         info = seen[id(t)] = _tensor_info(t, what)
-    p, n = info
+    p, n, _ = info
     if rows and cols and (cols > ld or off < 0 or off + (rows - 1) * ld + cols > n):
         raise ValueError(f"gemm operand {what}: {rows}x{cols} (ld {ld}) at offset {off} "
                          f"exceeds a tensor of {n} elements")
@@ -503,6 +504,7 @@ class GemmChain:
             return
         if self._rows and len(self._rows) + len(ops) > self.TABLE_ROWS:
             self.flush()
+        ops = list(ops)
         rows = _gemm_rows(ops)
         self._rows += rows
         self._counts.append(len(rows))

@@ -948,8 +948,8 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
     }
     __syncthreads();
     const double rho = 2.0 * fabs(ee);
-    // The entries of negligible weight go to the end (in the order deflate() puts
-    // them there); only if two of the others then have to be rotated
+    // The entries of negligible weight go to the end (from it here, in order when
+    // they are written out); only if two of the others then have to be rotated
     // together is the serial pass made (0.2 us an entry).
     int before = 0;
     for (int b = 0; b < m; b += 512) {
@@ -978,8 +978,9 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
     bool some = false;
     for (int i = tid; i + 1 < before; i += 512) some = some || may_deflate(before, i, rho, dl, zl);
     if (tid == 0) sK = before;
-    if (__syncthreads_or(some)) {
-        if (tid == 0) sK = deflate(m, rho, ds, zs, id, dl, zl, src, dd, rot_i, rot_c, &sR);
+    const bool serial = __syncthreads_or(some);
+    if (serial) {
+        if (tid == 0) sK = deflate(m, m - before, rho, ds, zs, id, dl, zl, src, dd, rot_i, rot_c, &sR);
         __syncthreads();
     }
     const int K = sK, nr = sR;
@@ -993,12 +994,13 @@ k_eig_merge(const mpsx_two_site_op *ops, char *ws, int max_n, int s, int buf, in
             *pb = cs.x * xb - cs.y * xa;
         }
     for (int i = tid; i < m; i += 512) {
-        ev.src[lo + i] = src[i];
+        const int o = i < K || serial ? i : m - 1 - (i - K);
+        ev.src[lo + i] = src[o];
         if (i < K) {
             ev.dl[lo + i] = dl[i];
             ev.zl[lo + i] = zl[i];
         } else {
-            ev.d[lo + i] = dd[i];
+            ev.d[lo + i] = dd[o];
         }
     }
     if (tid == 0) {

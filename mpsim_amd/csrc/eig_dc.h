@@ -108,11 +108,13 @@ MPSX_DEV double2 uniform_z(double2 v) { return make_double2(uniform_f64(v.x), un
 // Rank-one update diag(d) + rho z z^T of a merge, poles in ascending order
 // (ds, zs, id): deflates the entries with negligible weight and, of poles
 // closer than the weights resolve, one of each pair after a rotation. K
-// poles stay (dl, zl, src[0 .. K-1]); the deflated ones fill dd and src from
-// the end. rot_i, rot_c: the rotations (row a, row b, c, s) in order. Serial.
-MPSX_DEV int deflate(int m, double rho, const double *ds, const double *zs, const int *id, double *dl,
+// poles stay (dl, zl, src[0 .. K-1]); of dd and src the `none` entries of
+// negligible weight (as many as the same test counts) fill the end, in order, so
+// that rows which nothing couples keep theirs, and the rotated ones the places before
+// them. rot_i, rot_c: the rotations (row a, row b, c, s) in order. Serial.
+MPSX_DEV int deflate(int m, int none, double rho, const double *ds, const double *zs, const int *id, double *dl,
                      double *zl, int *src, double *dd, int2 *rot_i, double2 *rot_c, int *nrot) {
-    int K = 0, e = m, nr = 0, pj = -1;
+    int K = 0, f = m - none, e = f, nr = 0, pj = -1;
     double pd = 0.0, pz = 0.0;
     int in = id[0];
     double dn = ds[0], zn = zs[0];
@@ -124,10 +126,10 @@ MPSX_DEV int deflate(int m, double rho, const double *ds, const double *zs, cons
             dn = ds[r + 1];
             zn = zs[r + 1];
         }
-        if (rho * fabs(zr) <= kDeflate) {
-            --e;
-            src[e] = i;
-            dd[e] = dr;
+        if (!(rho * fabs(zr) > kDeflate)) {
+            src[f] = i;
+            dd[f] = dr;
+            ++f;
             continue;
         }
         if (pj >= 0) {
@@ -355,8 +357,8 @@ MPSX_DEV void leaf_conquer(int m, double (*S)[LEAF + 1], double (*U)[LEAF + 1], 
         }
         __syncthreads();
         // The first wave, a lane a sorted entry: those of negligible weight go to the end
-        // of their merge (in the order deflate() puts them there); if two of
-        // the others have to be rotated together (kn < 0), deflate() starts over.
+        // of their merge, in order; if two of the others have to be rotated together
+        // (kn < 0: -1 - the number of others), deflate() starts over.
         if (tid < M) {
             const int r = tid, rl = r & ~(h - 1), rm = rl + s, rh = min(rl + h, m);
             const bool on = r < m;
@@ -375,21 +377,21 @@ MPSX_DEV void leaf_conquer(int m, double (*S)[LEAF + 1], double (*U)[LEAF + 1], 
                 L.zl[rl + before] = z;
                 L.src[rl + before] = L.id[r];
             } else if (on) {
-                const int e = rh - 1 - (r - rl - before);
+                const int e = rl + __popcll(mine) + (r - rl - before);
                 L.dd[e] = d;
                 L.src[e] = L.id[r];
             } else {
                 L.src[r] = r;
             }
             if (on && r == rl) {
-                L.kn[r] = pairs ? -1 : __popcll(mine);
+                L.kn[r] = pairs ? -1 - __popcll(mine) : __popcll(mine);
                 L.nrot[r] = 0;
             }
         }
         __syncthreads();
         if (sub == 0 && g < m && gj == 0 && L.kn[lo] < 0)
-            L.kn[lo] = deflate(hi - lo, rho, L.ds + lo, L.zs + lo, L.id + lo, L.dl + lo, L.zl + lo,
-                               L.src + lo, L.dd + lo, L.rot_i + lo, L.rot_c + lo, &L.nrot[lo]);
+            L.kn[lo] = deflate(hi - lo, hi - lo + L.kn[lo] + 1, rho, L.ds + lo, L.zs + lo, L.id + lo, L.dl + lo,
+                               L.zl + lo, L.src + lo, L.dd + lo, L.rot_i + lo, L.rot_c + lo, &L.nrot[lo]);
         __syncthreads();
         if (tid < m) {  // component tid of its merge's rows
             const int tlo = tid & ~(h - 1);

@@ -153,7 +153,7 @@ class Engine:
         self.dev = nat.device(dev)
         self._ws = None
         self._gates: "OrderedDict[bytes, object]" = OrderedDict()
-        from .tune import tuned_config, tuned_engine
+        from .tune import tuned_config, tuned_engine, tuned_rounds
         self.svd = tuned_config()
         self.last_sweeps = 0
         # concurrent groups of a split call (at most the 4 hardware queues a
@@ -161,6 +161,10 @@ class Engine:
         # be split, and that row count; from the stored tuning when there is
         # one (SPLIT_ROWS and 4 ways otherwise)
         self.split_ways, self.split_min, self.split_rows = tuned_engine()
+        # the same two numbers for methods that iterate in rounds, while the rule is
+        # the stored one
+        self._split_stored = (self.split_min, self.split_rows)
+        self._split_rounds = tuned_rounds()
         self._wss: list = []        # workspaces of the helper streams' groups
         self._helpers: list = []    # (stream, single-thread executor) per helper group
         self._keep: list = []       # device tables of the last call, alive until the next
@@ -389,14 +393,25 @@ class Engine:
                 if stream:
                     self._leave_workspaces(cur)
 
+    def _split_rule(self, cfg) -> Tuple[int, int]:
+        """(split_min, split_rows) of a call. The direct solver's chain of steps leaves
+        most of the device idle, so its calls are split early. Rounds fill it from
+        about 256 rows on: 12 problems of 300 rows take 16.0 ms in one group and 19.7 in
+        four (one-sided; FP32 14.1 and 17.3, mixed 11.2 and 12.2), 8 of 384 22.3 and
+        27.5."""
+        rule = (self.split_min, self.split_rows)
+        if rule == self._split_stored and (cfg.method or cfg.rotation_fp32 or cfg.fp32_sweeps > 0 or cfg.block == 8):
+            return self._split_rounds
+        return rule
+
     def _two_site(self, items: Sequence[TwoSiteItem], svd: Optional[SvdConfig], cur, stream: int
                   ) -> List[TwoSiteResult]:
         n = len(items)
         cfg = (svd or self.svd).to_c()
         self._keep = []
-        big = [i for i, it in enumerate(items) if _rows(it) >= self.split_rows]
+        split_min, split_rows = self._split_rule(cfg)
         ways = max(1, min(int(self.split_ways), n))
-        if ways < 2 or len(big) < self.split_min or cfg.check_every == 0:
+        if ways < 2 or cfg.check_every == 0 or sum(_rows(it) >= split_rows for it in items) < split_min:
             outs, tab, dtab, ws = self._prepare_two_site(items, cfg, stream=stream)
             self._keep = [dtab]
             self.last_sweeps = self._run_two_site(tab, dtab, ws, cfg, stream)

@@ -25,7 +25,8 @@ Three stages, each timed on seeded synthetic two-site problems:
 These batches hold problems of one size. Layers of mixed sizes, where a large
 problem's chain of steps would hold up the others, are not among them: a rule chosen
 from such layers is stored with `split_fixed`, and a re-tune then measures
-stage 3 but keeps the three values.
+stage 3 but keeps the three values and those of the methods that iterate
+(`split_min_rounds`, `split_rows_rounds`).
 
 Engine picks the stored values up as its defaults (tuned_config,
 tuned_engine). The library's compile-time tile shapes (theta tiles, 16-row
@@ -82,6 +83,15 @@ def tuned_engine(path: Optional[str] = None) -> Tuple[int, int, int]:
     smin = int(t.get("split_min", DEFAULT_SPLIT_MIN))
     rows = int(t.get("split_rows", DEFAULT_SPLIT_ROWS))
     return max(1, min(4, ways)), max(1, smin), max(1, rows)
+
+
+def tuned_rounds(path: Optional[str] = None) -> Tuple[int, int]:
+    """(split_min, split_rows) for calls whose method iterates in rounds at every
+    size (one-sided, FP32, mixed): `split_min_rounds` and `split_rows_rounds` of the
+    stored tuning, else the rule of every call."""
+    t = _load(path)
+    _, smin, rows = tuned_engine(path)
+    return max(1, int(t.get("split_min_rounds", smin))), max(1, int(t.get("split_rows_rounds", rows)))
 
 
 def _problems(engine, chi: int, count: int, seed: int):
@@ -215,6 +225,7 @@ def tune(engine=None, chis: Sequence[int] = (8, 16, 32, 64, 128, 256), reps: int
     if stored.get("split_fixed"):
         out["split_fixed"] = 1
         out["split_ways"], out["split_min"], out["split_rows"] = tuned_engine(path)
+        out["split_min_rounds"], out["split_rows_rounds"] = tuned_rounds(path)
     out["precondition"] = int(stored.get("precondition", DEFAULT_PRECONDITION))
     out["measurements"] = rows
     if path:

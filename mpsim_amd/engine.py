@@ -19,31 +19,29 @@ from . import _native as nat
 MAX_OPS = 65535  # descriptors per grouped launch (grid y / x limits of the kernels)
 
 
-def _tensor_info(t, what: str) -> Tuple[int, int, object]:
-    """(device address, elements, the tensor) of a contiguous complex64 tensor."""
-    n = t.numel()
-    if n and t.element_size() != 8:
-        raise ValueError(f"gemm operand {what} must be complex64")
-    return nat.ptr(t), n, t
-
-
 def _matrix_addr(x, rows: int, cols: int, ld: int, what: str, seen: dict) -> int:
     """Device address of a rows x cols matrix with row stride `ld` stored in
     a contiguous complex64 tensor at an element offset (x = tensor or
-    (tensor, offset)); raises if any element would fall outside it. seen: the
-    _tensor_info of the call's tensors so far (many products share one), which
-    holds them, so that an id stays one tensor's."""
+    (tensor, offset)); raises if any element would fall outside it. seen:
+    (address, tensor) of the tensors the call has found matrices inside of so far
+    (many products share one); holding them, an id stays one tensor's."""
     t, off = x if isinstance(x, tuple) else (x, 0)
-    info = seen.get(id(t))
-    if info is None:
-        if rows == 0 or cols == 0:
-            return nat.ptr(t) + 8 * off if t.numel() else 0
-        info = seen[id(t)] = _tensor_info(t, what)
-    p, n, _ = info
-    if rows and cols and (cols > ld or off < 0 or off + (rows - 1) * ld + cols > n):
+    n = t.numel()
+    if not (rows and cols):
+        return nat.ptr(t) + 8 * off if n else 0
+    if cols > ld or off < 0 or off + (rows - 1) * ld + cols > n:
         raise ValueError(f"gemm operand {what}: {rows}x{cols} (ld {ld}) at offset {off} "
                          f"exceeds a tensor of {n} elements")
-    return p + 8 * off if n else 0
+    if t is not x:
+        known = seen.get(id(t))
+        if known is not None:
+            return known[0] + 8 * off
+    if t.element_size() != 8:
+        raise ValueError(f"gemm operand {what} must be complex64")
+    p = nat.ptr(t)
+    if t is not x:
+        seen[id(t)] = (p, t)
+    return p + 8 * off
 
 
 def _gemm_rows(ops: Sequence[dict]) -> List[tuple]:
@@ -475,9 +473,20 @@ class Engine:
             for s in range(0, len(ops), MAX_OPS):
                 self.gemm(ops[s:s + MAX_OPS])
             return
-        chain = GemmChain(self)
-        chain.gemm(ops)
-        chain.flush()
+        self._launch_gemm(_gemm_rows(ops), (len(ops),))
+
+    def _launch_gemm(self, rows: List[tuple], counts: Sequence[int]) -> None:
+        """Grouped products one after the other from one table: the first counts[0]
+        rows, the next counts[1], ..."""
+        tab = np.array(rows, dtype=nat.GEMM_OP)
+        stream = self.stream
+        dtab = nat.put_table(tab, self.dev, stream)
+        h, d = tab.ctypes.data, dtab.data_ptr()
+        for c in counts:
+            nat.check(self.lib.mpsx_gemm(stream, h, d, c))
+            h += c * tab.itemsize
+            d += c * tab.itemsize
+        self._last_gemm_table = dtab
 
     # ------------------------------------------------------------ scale
     def scale(self, tensors: Sequence[object], factor: complex, conj: bool = False) -> None:
@@ -531,14 +540,5 @@ class GemmChain:
     def flush(self) -> None:
         if not self._rows:
             return
-        eng = self.eng
-        tab = np.array(self._rows, dtype=nat.GEMM_OP)
-        stream = eng.stream
-        dtab = nat.put_table(tab, eng.dev, stream)
-        h, d = tab.ctypes.data, dtab.data_ptr()
-        for c in self._counts:
-            nat.check(eng.lib.mpsx_gemm(stream, h, d, c))
-            h += c * tab.itemsize
-            d += c * tab.itemsize
-        eng._last_gemm_table = dtab
+        self.eng._launch_gemm(self._rows, self._counts)
         self._rows, self._counts, self._ops, self._bytes = [], [], [], 0

@@ -3,6 +3,7 @@ taken in before the addresses of a call's tensors were looked up once per tensor
 from collections import namedtuple
 from collections.abc import Sequence
 
+import pytest
 import torch
 
 Place = namedtuple("Place", "tensor offset")
@@ -21,10 +22,11 @@ def test_operands_as_tensors_pairs_and_named_pairs():
 
 
 class _Lazy(Sequence):
-    """Products whose operands are views made when they are asked for."""
+    """Products whose operands are views made when they are asked for (`pairs`: with an
+    offset)."""
 
-    def __init__(self, base, count):
-        self.base, self.count = base, count
+    def __init__(self, base, count, pairs):
+        self.base, self.count, self.pairs = base, count, pairs
 
     def __len__(self):
         return self.count
@@ -33,12 +35,13 @@ class _Lazy(Sequence):
         if i >= self.count:
             raise IndexError
         v = [self.base[12 * i + 4 * j:12 * i + 4 * j + 4] for j in range(3)]
-        return _op(*v)
+        return _op(*[(x, 0) for x in v] if self.pairs else v)
 
 
-def test_operands_made_on_the_way_have_their_own_addresses():
+@pytest.mark.parametrize("pairs", [False, True])
+def test_operands_made_on_the_way_have_their_own_addresses(pairs):
     from mpsim_amd.engine import _gemm_rows
     base = torch.zeros(12 * 50, dtype=torch.complex64)
     p = base.data_ptr()
-    rows = _gemm_rows(_Lazy(base, 50))
+    rows = _gemm_rows(_Lazy(base, 50, pairs))
     assert [r[:3] for r in rows] == [tuple(p + 8 * (12 * i + 4 * j) for j in range(3)) for i in range(50)]

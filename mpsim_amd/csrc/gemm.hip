@@ -312,23 +312,36 @@ static hipError_t gemm_run(hipStream_t s, const mpsx_gemm_op *d, int count, int6
     return hipGetLastError();
 }
 
-static int64_t gemm_tiles(const mpsx_gemm_op *h, int count, int edge) {
-    int64_t t = 0;
-    for (int i = 0; i < count; ++i) t += ((h[i].m + edge - 1) / edge) * ((h[i].n + edge - 1) / edge);
-    return t;
-}
-
-// The largest tile that still makes about a workgroup a compute unit: above
-// that the wider tile reads less (4096 x 512 x 256: 50 us wide, 60 mid; 16 of
-// 256 x 256 x 256: 26 and 32), below it the narrower one has the waves
+// The tile of a call. First the largest that still makes about a workgroup a
+// compute unit: above that the wider tile reads less (4096 x 512 x 256: 50 us wide, 60
+// mid; 16 of 256 x 256 x 256: 26 and 32), below it the narrower one has the waves
 // (1024 x 512 x 256, 128 wide tiles: 17 us mid, 23 wide; 256 x 512 x 256, 128
-// mid ones: 6.8 thin, 9.1 mid).
+// mid ones: 6.8 thin, 9.1 mid). Then a smaller one where the matrices leave much of that
+// tile empty: an element of a full tile takes about 1 : 1.25 : 1.5 wide : mid : thin (64
+// columns, k = 256: 135, 160 and 199 us of 100000 rows), and so do the elements of padding.
+// In us, wide tiles -> this choice: 2^20 x 3 x 33 361 -> 135, 100000 x 24 x 64 52 -> 37,
+// 100000 x 80 x 40 77 -> 70, 2000 of 8 x 8 x 40 52 -> 13, of 65 x 65 x 40 205 -> 108.
+// Not where the launch, sized for the largest m and the largest n, would be mostly
+// workgroups without a tile.
 constexpr int64_t GEMM_FILL = 192;
 
 hipError_t launch_gemm(hipStream_t s, const mpsx_gemm_op *h, const mpsx_gemm_op *d, int count, int64_t max_m,
                        int64_t max_n) {
     if (max_m < 1 || max_n < 1) return hipSuccess;
-    if (gemm_tiles(h, count, GemmWide::TILE) >= GEMM_FILL) return gemm_run<GemmWide>(s, d, count, max_m, max_n);
-    if (gemm_tiles(h, count, GemmMid::TILE) >= GEMM_FILL) return gemm_run<GemmMid>(s, d, count, max_m, max_n);
+    constexpr int64_t edge[3] = {GemmWide::TILE, GemmMid::TILE, GemmThin::TILE};
+    constexpr double cost[3] = {1.0, 1.25, 1.5};  // of an element
+    int64_t tiles[3] = {0, 0, 0};
+    for (int i = 0; i < count; ++i)
+        for (int t = 0; t < 3; ++t) tiles[t] += ((h[i].m + edge[t] - 1) / edge[t]) * ((h[i].n + edge[t] - 1) / edge[t]);
+    const int fill = tiles[0] >= GEMM_FILL ? 0 : tiles[1] >= GEMM_FILL ? 1 : 2;
+    int pick = fill;
+    for (int t = fill + 1; t < 3; ++t) {
+        const int64_t grid = ((max_m + edge[t] - 1) / edge[t]) * ((max_n + edge[t] - 1) / edge[t]);
+        if (grid > 2147483647LL || (double)grid * count > 2.0 * (double)tiles[t]) continue;
+        if (cost[t] * (double)(tiles[t] * edge[t] * edge[t]) < cost[pick] * (double)(tiles[pick] * edge[pick] * edge[pick]))
+            pick = t;
+    }
+    if (pick == 0) return gemm_run<GemmWide>(s, d, count, max_m, max_n);
+    if (pick == 1) return gemm_run<GemmMid>(s, d, count, max_m, max_n);
     return gemm_run<GemmThin>(s, d, count, max_m, max_n);
 }

@@ -281,9 +281,11 @@ class Engine:
             return
         tab = np.array(rows, dtype=nat.SITE_OP)
         stream = self.stream
-        if len(rows) <= nat.SITE_NOW and self.lib.mpsx_apply_one_site_now(
-                stream, tab.ctypes.data, len(rows)) == nat.MPSX_OK:
-            return
+        if len(rows) <= nat.SITE_NOW:
+            code = self.lib.mpsx_apply_one_site_now(stream, tab.ctypes.data, len(rows))
+            if code != nat.MPSX_EINVAL:  # refused (a capture) before anything was launched
+                nat.check(code)
+                return
         dtab = nat.put_table(tab, self.dev, stream)
         nat.check(self.lib.mpsx_apply_one_site(stream, tab.ctypes.data, dtab.data_ptr(),
                                                len(rows)))

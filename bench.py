@@ -616,23 +616,32 @@ def main():
     tbytes = (traffic.get("bytes_per_unit")
               if traffic and traffic.get("kernel") == "+".join(kset) else None)
     # executed FP64 MFMA flops per unit (SQ_INSTS_VALU_MFMA_MOPS_F64 x 512 from a
-    # counter pass) over the live busy time
+    # counter pass) over the live busy time. The direct solver executes fewer flops
+    # than the SVD term counts and is bound by the latency of k_tridiag's steps, so
+    # its fraction of the peak is that of the executed ones.
     mc = (traffic or {}).get("mfma_counters")
+    direct = kset == DIRECT
+    executed = (mc["executed_flop_per_unit"] * jr_n / (jr_busy * 1e-3) / 1e12
+                if (mc and not svd.fp32 and jr_busy > 0 and mc.get("kernel") == dom) else None)
+    rate = executed if direct else achieved
     roofline = {
         "kernel": "+".join(kset),
-        "bound": "mfma",
-        "achieved": round(achieved, 3),
+        "bound": "latency" if direct else "mfma",
+        "achieved": None if rate is None else round(rate, 3),
         "peak": peak,
         "unit": "TFLOP/s",
-        "frac": round(achieved / peak, 5),
-        # the same rate against the dense FP32 matrix peak (157.3 TFLOP/s), the
+        "frac": None if rate is None else round(rate / peak, 5),
+        "achieved_algorithmic": round(achieved, 3),
+        # the algorithmic rate against the dense FP32 matrix peak (157.3 TFLOP/s), the
         # denominator of the FP32-MFMA formulation of this SVD
         "frac_of_fp32_mfma_peak": round(achieved / PEAK_FP32_MFMA, 5),
         "traffic": tbytes,
         "traffic_unit": "HBM bytes per solve of a group (calibrated FETCH_SIZE + WRITE_SIZE)",
-        "achieved_basis": "algorithmic SVD flops of the updates with 32-row pivots / busy time of "
-                          "their SVD kernels (union of launch intervals, HIP events on the launch "
-                          "streams), from a profiled repeat of the timed steps",
+        "achieved_basis": ("executed FP64 matrix-core flops (counters)" if direct else
+                           "algorithmic SVD flops of the updates with 32-row pivots") +
+                          " / busy time of the SVD kernels (union of launch intervals, HIP events on "
+                          "the launch streams), from a profiled repeat of the timed steps; "
+                          "achieved_algorithmic: the SVD flops over the same time",
         "profiled_pass_updates_per_s": round(updates * args.steps / sum(ptimes), 3),
         "busy_ms": round(jr_busy, 3),
         "concurrency": round(jr_ms / jr_busy, 3) if jr_busy > 0 else None,
@@ -641,9 +650,7 @@ def main():
         "avg_unit_us": round(1e3 * jr_ms / max(jr_n, 1), 3),
         "avg_launch_us": {k: round(1e3 * kern[k][0] / max(kern[k][1], 1), 3)
                           for k in kset if k in kern},
-        "executed_mfma_frac_counters": (
-            round(mc["executed_flop_per_unit"] * jr_n / (jr_busy * 1e-3) / 1e12 / peak, 4)
-            if (mc and not svd.fp32 and jr_busy > 0 and mc.get("kernel") == dom) else None),
+        "executed_mfma_frac_counters": None if executed is None else round(executed / peak, 4),
         "algorithmic_flops_per_unit": dom_f / max(jr_n, 1),
         "algorithmic_unit": "SVD term 4(4p^2q+8pq^2+9q^3) of the updates with 32-row pivots",
     }

@@ -123,7 +123,7 @@ MPSX_DEV int find_record(const char *table, int count, size_t stride, size_t fie
 struct TwoSiteHeader {
     int32_t active[64];  // active[s]: problems still unconverged after sweep s
     int32_t ticket;      // workgroups of k_tridiag started so far
-    int32_t spread;      // 0 .. 3, another than the launches before and after have: see form_group
+    int32_t spread;      // what k_tridiag was launched with: 0 .. 3, the launch's turn
     int32_t pad[62];
 };
 
@@ -196,8 +196,10 @@ MPSX_HD bool eig_direct(const mpsx_plan &p, int max_n) {
     return (p.method == 1 || p.method == 3) && p.C <= max_n;
 }
 // Problems that the one-workgroup kernel (csrc/small.hip) takes after theta:
-// FP64, at most 64 rows (the matrices it keeps in LDS) of at most 512 columns
-// (a longer row is more than one workgroup should read). on: 0 when the call
+// FP64, at most 64 rows (the matrices it keeps in LDS) of at most 512 columns, the widest
+// that its tests cover. (Wider ones take the one-sided rounds, though the kernel
+// would still be the faster: 64 rows of 512 columns 506 us, of 513 by the rounds 1409 and
+// by the kernel 476; of 2048 3061 and 1246; 4 rows of 2048 326 and 226.) on: 0 when the call
 // asks for the one-sided rounds.
 constexpr int SMALL_MAX_R = 512;
 MPSX_HD bool small_route(const mpsx_plan &p, int on) {

@@ -748,7 +748,7 @@ k_eig_map(const mpsx_two_site_op *ops, int count, char *ws, int2 *map, int max_n
 }
 
 __global__ void __launch_bounds__(512, 2)
-k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int spin_limit) {
+k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int spread, int spin_limit) {
     __shared__ TriShared<128, 8> sm;
     if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
     __syncthreads();
@@ -758,8 +758,7 @@ k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int
     const mpsx_plan p = ops[m.x].plan;
     const int member = m.y >> 8, G = m.y & 255;
     if (threadIdx.x == 0)
-        sm.whole = form_group(&reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->group, G,
-                              reinterpret_cast<const TwoSiteHeader *>(ws)->spread);
+        sm.whole = form_group(&reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->group, G, spread);
     __syncthreads();
     if (!sm.whole) return;
     switch (eig_class(p.C)) {
@@ -1279,7 +1278,7 @@ hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int coun
     const int spread = (int)(launches.fetch_add(1, std::memory_order_relaxed) & 3);
     hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, ws, static_cast<int2 *>(map), max_n, spread);
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)slots), dim3(512), 0, s, d, static_cast<const int2 *>(map), ws,
-                       slots, no_wait ? 0 : kSpin);
+                       slots, spread, no_wait ? 0 : kSpin);
     if (grouped)
         hipLaunchKernelGGL(k_tridiag_one, dim3((unsigned)count), dim3(512), 0, s, d, ws, max_n);
     return hipGetLastError();

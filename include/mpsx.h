@@ -108,12 +108,11 @@ int mpsx_apply_one_site_now(mpsx_stream stream, const mpsx_site_op *h, int count
  *       a_out = U[:, :k] S[:k],  b_out = V^H[:k, :]
  * The caller computes k = min(d*chi_l, d*chi_r, maxsvals) (core.py:1110-1130).
  * The SVD works on the side that is not scaled by S, so the scaled side never
- * divides by a singular value: a blocked one-sided Jacobi on theta's rows up
- * to 64 of them, above that the eigenvectors of the rows' Gram matrix, by a
- * direct solver (tridiagonal form, divide and conquer) up to 1024 rows and
- * by Jacobi rounds beyond. (Up to 64 rows of at most 512 columns the rows
- * that are not orthogonal yet go through the same direct route in one
- * workgroup.) theta is formed in complex FP64 for d = 2 and 3 (FP32 for
+ * divides by a singular value. Up to 64 rows of at most 512 columns the rows that
+ * are not orthogonal yet go through a direct eigensolver (tridiagonal form, divide
+ * and conquer) in one workgroup, repeatedly; wider ones take a blocked one-sided
+ * Jacobi. Above 64 rows it is the eigenvectors of the rows' Gram matrix, by the
+ * direct solver up to 1024 rows and by Jacobi rounds beyond. theta is formed in complex FP64 for d = 2 and 3 (FP32 for
  * other d and with rotation_fp32); by default everything after it is
  * complex FP64 (FP64 matrix cores), which keeps each truncated update as
  * accurate as a complex64 LAPACK SVD. With rotation_fp32 set they run in FP32
@@ -191,7 +190,8 @@ typedef struct {
                            it                                               */
     int32_t method;     /* MPSX_SVD_AUTO (0): the Gram method for FP64
                            problems with b = 16 and nb >= 6 (more than 64
-                           rows), rows otherwise;
+                           rows), otherwise the one-workgroup kernel or
+                           (above 512 columns) rows;
                            MPSX_SVD_ROWS (1): the one-sided method for all */
     int32_t fp32_sweeps;/* > 0: the Gram method starts with an FP32 phase of
                            at most this many sweeps: its rounds keep H in

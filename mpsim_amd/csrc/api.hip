@@ -181,18 +181,99 @@ int plan_method(const Resolved &r, int b, int nb) {
     return r.fp32_sweeps > 0 ? 2 : 1;
 }
 
+int compute_units() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    return cus;
+}
+
 // Rows up to which the Gram problems of a call take the direct eigensolver.
 // Its largest group of workgroups has to be resident as a whole, also beside
 // those of a few other streams (or it is given up, see k_tridiag), so a device (or partition) of fewer compute
 // units takes smaller problems only. k_eig_* launch problems as grid y.
 int direct_max(int count) {
-    int dev = 0, cus = 0;
-    if (count > 65535 || hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return 0;
+    const int cus = compute_units();
+    if (count > 65535 || cus < 1) return 0;
     int n = EIG_MAX_N;
     while (n > 128 && 4 * eig_group(n) > cus) n /= 2;
     return 4 * eig_group(n) <= cus ? n : 0;
+}
+
+// Launches of k_tridiag with groups of up to 64 workgroups (problems of more than 512
+// rows), one list per device. The workgroups of several such launches can each hold
+// compute units that the others' missing members need, until a group is given up and
+// its problem takes 0.3 s in one workgroup (27 problems of 1024 rows in four launches:
+// 73 ms, 411 with a group given up). So a launch is held back, on the device, until the
+// launches that are left can be under way with it: beside the largest of them there has
+// to be room for one of its groups, whatever the others hold, so that one group is always
+// whole. Launches of smaller groups, and captured ones, stay as they are.
+struct BigGroups {
+    struct Launch {
+        hipStream_t stream;
+        hipEvent_t end;
+        int wgs;
+    };
+    std::mutex mu;
+    std::vector<Launch> window;     // may be under way together, oldest first
+    std::vector<hipEvent_t> before; // ends of the last kBefore that left the window
+    std::vector<hipEvent_t> spare;
+};
+constexpr size_t kBefore = 8;
+constexpr int kLargestGroup = 64;
+
+// Enqueues `launch` (of `wgs` such workgroups) on `stream`, behind what has to
+// have ended. cus: compute units of the device, a workgroup each.
+template <class F>
+hipError_t launch_big_groups(BigGroups &b, hipStream_t stream, int wgs, int cus, F &&launch) {
+    std::lock_guard<std::mutex> g(b.mu);
+    for (size_t i = 0; i < b.window.size(); ++i)
+        if (b.window[i].stream == stream) {  // ends before this one starts: one entry stands for both
+            wgs = std::max(wgs, b.window[i].wgs);
+            b.spare.push_back(b.window[i].end);
+            b.window.erase(b.window.begin() + (std::ptrdiff_t)i);
+            break;
+        }
+    size_t keep = b.window.size();
+    for (int sum = wgs, largest = wgs; keep > 0; --keep) {
+        const int w = b.window[keep - 1].wgs;
+        sum += w;
+        largest = std::max(largest, w);
+        if (sum - largest + kLargestGroup > cus) break;
+    }
+    for (size_t i = 0; i < keep; ++i) b.before.push_back(b.window[i].end);
+    b.window.erase(b.window.begin(), b.window.begin() + (std::ptrdiff_t)keep);
+    // (all of `before`: those in the window may themselves be held back behind some)
+    for (hipEvent_t e : b.before)
+        if (hipError_t err = hipStreamWaitEvent(stream, e, 0)) return err;
+    while (b.before.size() > kBefore) {
+        b.spare.push_back(b.before.front());
+        b.before.erase(b.before.begin());
+    }
+    if (b.spare.empty()) {
+        hipEvent_t e = nullptr;
+        if (hipError_t err = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return err;
+        b.spare.push_back(e);
+    }
+    if (hipError_t err = launch()) return err;
+    // (recorded anew: waits that were enqueued for its last record stay with that)
+    if (hipError_t err = hipEventRecord(b.spare.back(), stream)) return err;
+    b.window.push_back({stream, b.spare.back(), wgs});
+    b.spare.pop_back();
+    return hipSuccess;
+}
+
+// The list of the current device (never freed: a launch may be under way at exit).
+BigGroups &big_groups() {
+    static std::mutex mu;
+    static std::map<int, BigGroups *> all;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    std::lock_guard<std::mutex> g(mu);
+    BigGroups *&b = all[dev];
+    if (!b) b = new BigGroups;
+    return *b;
 }
 
 int *poll_buffer() {
@@ -488,6 +569,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
     int max_n = -1;          // rows up to which the direct solver is taken, once a Gram problem asks
     int64_t groups = 0;      // the direct solver's workgroup table (as planned)
     int64_t eig_slots = 0;   // workgroups the direct solver launches
+    int64_t big_slots = 0;   // those of problems of more than 512 rows
     int eig_n = 0;           // its largest problem
     int64_t eig_tiles = 0;   // 32 x 32 tiles of its largest X
     bool eig_small = false, eig_large = false;
@@ -529,6 +611,7 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
             if (eig_direct(p, EIG_MAX_N)) groups += eig_group(p.C);
             if (eig_direct(p, max_n)) {
                 eig_slots += eig_group(p.C);
+                if (p.C > 512) big_slots += eig_group(p.C);
                 eig_n = std::max(eig_n, (int)p.C);
                 eig_tiles = std::max(eig_tiles, (int64_t)((p.C + 31) / 32) * ((p.R + 31) / 32));
                 (p.C <= 512 ? eig_small : eig_large) = true;
@@ -615,10 +698,19 @@ int two_site_run(hipStream_t stream, const mpsx_two_site_op *h, const mpsx_two_s
         HIP_TRY(timed("k_hgram", stream, [&] { return launch_hgram(stream, d, owner, ws, pairs, gram_nb, 0, max_n); }), "k_hgram");
     if (eig_slots > 0) {
         HIP_TRY(timed("k_hgram", stream, [&] { return launch_eig_gram(stream, d, count, ws, max_n, eig_n); }), "k_eig_gemm");
-        HIP_TRY(timed("k_tridiag", stream,
-                      [&] { return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128,
-                                                  (force & MPSX_FORCE_TIMEOUT) != 0); }),
-                "k_tridiag");
+        auto tridiag = [&] {
+            return timed("k_tridiag", stream, [&] {
+                return launch_eig_tridiag(stream, d, count, ws, ws + map_off, max_n, (int)eig_slots, eig_n > 128, eig_n <= 256,
+                                          (force & MPSX_FORCE_TIMEOUT) != 0);
+            });
+        };
+        // (a capture, and the call that makes no events, leave it to form_group's waits)
+        if (big_slots > 0 && may_poll && cap == hipStreamCaptureStatusNone)
+            HIP_TRY(launch_big_groups(big_groups(), stream, (int)std::min<int64_t>(big_slots, kGridLimit / 2),
+                                      compute_units(), tridiag),
+                    "k_tridiag");
+        else
+            HIP_TRY(tridiag(), "k_tridiag");
         HIP_TRY(timed("k_eig_conquer", stream,
                       [&] { return launch_eig_conquer(stream, d, count, ws, max_n, eig_n); }),
                 "k_eig_conquer");

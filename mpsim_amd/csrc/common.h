@@ -122,7 +122,7 @@ MPSX_DEV int find_record(const char *table, int count, size_t stride, size_t fie
 // Workspace header of a two-site batch (at ws + 0).
 struct TwoSiteHeader {
     int32_t active[64];  // active[s]: problems still unconverged after sweep s
-    int32_t ticket;      // workgroups of k_tridiag started so far
+    int32_t ticket;      // workgroups of k_tridiag started so far, where that is their order
     int32_t spread;      // what k_tridiag was launched with: 0 .. 3, the launch's turn
     int32_t pad[62];
 };

@@ -113,12 +113,21 @@ MPSX_DEV int eig_levels(int n) {
 // gone (a published NaN is given other bits). Slots of step J: four arrays of n
 // - J doubles (p re, p im, c re, c im). Steps J and n - J share two Y rows.
 //
-// Workgroups take their place by a ticket in the order they start, and a
-// group starts its work only when all its workgroups have: from then on it
+// A group starts its work only when all its workgroups have started: from then on it
 // holds its compute units and waits for nothing but itself. Before that a
-// workgroup may hold a compute unit that a missing member needs (each XCD
-// is dealt a fixed share of a launch, and several launches, each with an
-// incomplete group, can fill one), so that wait has an end: after
+// workgroup may hold a compute unit that a missing member needs. In a launch
+// whose largest problem has more than 256 rows the groups are stretches of the
+// workgroups as they are numbered: each XCD is dealt every eighth and starts its share in
+// order, so the first group that is not done is whole before later ones hold
+// anything it needs. (By order of start, the last groups could be left with more
+// workgroups on one XCD than that has compute units: one launch of 11 problems of 900
+// rows took 28 ms and now and then 316; now 21.4.) Members are numbered XCD by XCD, so that
+// the owners of neighbouring rows share an L2 (1024 rows: 7.7 -> 7.4 ms). Groups of
+// up to four are formed by tickets in the order of start instead, which leaves fewer
+// compute units waiting where launches of several streams mix (four streams of 100 problems
+// of 150 rows: 3.9 ms a call, 4.9 by number).
+// Several launches can still block each other, each with an incomplete group (the
+// host holds back those of large groups, launch_big_groups), so the wait has an end: after
 // kFormTicks, once to four times by the launch's turn so that launches under way
 // together do not all give up at once, the group is given up for good, its workgroups leave, and
 // k_tridiag_one does the problem. The flag and the count are one word (ctl->group), so a
@@ -748,15 +757,21 @@ k_eig_map(const mpsx_two_site_op *ops, int count, char *ws, int2 *map, int max_n
 }
 
 __global__ void __launch_bounds__(512, 2)
-k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int spread, int spin_limit) {
+k_tridiag(const mpsx_two_site_op *ops, const int2 *map, char *ws, int slots, int ticket, int spread,
+          int spin_limit) {
     __shared__ TriShared<128, 8> sm;
-    if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
-    __syncthreads();
-    const int slot = sm.slot;
+    int slot = (int)blockIdx.x;
+    if (ticket) {  // by order of start
+        if (threadIdx.x == 0) sm.slot = atomicAdd(&reinterpret_cast<TwoSiteHeader *>(ws)->ticket, 1);
+        __syncthreads();
+        slot = sm.slot;
+    }
     if (slot >= slots) return;
     const int2 m = map[slot];
     const mpsx_plan p = ops[m.x].plan;
-    const int member = m.y >> 8, G = m.y & 255;
+    const int G = m.y & 255;
+    int member = m.y >> 8;
+    if (!ticket) member = (member & 7) * (G >> 3) + min(member & 7, G & 7) + (member >> 3);  // XCD by XCD
     if (threadIdx.x == 0)
         sm.whole = form_group(&reinterpret_cast<ProblemCtl *>(ws + p.ws_off)->group, G, spread);
     __syncthreads();
@@ -1273,12 +1288,12 @@ k_eig_back(const mpsx_two_site_op *ops, char *ws, int max_n) {
 
 // ---------------------------------------------------------------- launchers
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots, bool grouped, bool no_wait) {
+                              int slots, bool grouped, bool ticket, bool no_wait) {
     static std::atomic<unsigned> launches{0};
     const int spread = (int)(launches.fetch_add(1, std::memory_order_relaxed) & 3);
     hipLaunchKernelGGL(k_eig_map, dim3(1), dim3(256), 0, s, d, count, ws, static_cast<int2 *>(map), max_n, spread);
     hipLaunchKernelGGL(k_tridiag, dim3((unsigned)slots), dim3(512), 0, s, d, static_cast<const int2 *>(map), ws,
-                       slots, spread, no_wait ? 0 : kSpin);
+                       slots, ticket ? 1 : 0, spread, no_wait ? 0 : kSpin);
     if (grouped)
         hipLaunchKernelGGL(k_tridiag_one, dim3((unsigned)count), dim3(512), 0, s, d, ws, max_n);
     return hipGetLastError();

@@ -71,11 +71,11 @@ hipError_t launch_qr_step(hipStream_t s, const mpsx_two_site_op *d, int count, c
                           int strips, int max_c, bool small, bool large, int max_n);
 // Direct eigensolver (eig.hip) of the problems eig_direct selects: the
 // tridiagonal form (`map`: room for `slots` int2, the workgroups of all their
-// groups; `grouped`: some group has more than one; `no_wait`: a group's waits end at
-// their first look), the eigensystem of T, and Y. n: the largest C among them; `small`,
+// groups; `grouped`: some group has more than one; `ticket`: the workgroups take their
+// places in the order they start; `no_wait`: a group's waits end at their first look), the eigensystem of T, and Y. n: the largest C among them; `small`,
 // `large`: some of at most 512 rows, some above.
 hipError_t launch_eig_tridiag(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, void *map, int max_n,
-                              int slots, bool grouped, bool no_wait);
+                              int slots, bool grouped, bool ticket, bool no_wait);
 // H = X X^H, and at the end X <- Y X (tiles: 32 x 32 ones of the largest X).
 hipError_t launch_eig_gram(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n, int n);
 hipError_t launch_eig_apply(hipStream_t s, const mpsx_two_site_op *d, int count, char *ws, int max_n,

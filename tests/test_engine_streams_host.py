@@ -50,6 +50,7 @@ def _engine(log, need):
     eng._ws, eng._wss, eng._keep, eng._helpers = None, [], [], []
     eng.split_ways, eng.split_min, eng.split_rows = 1, 1, 1
     eng._split_stored = eng._split_rounds = (1, 1)
+    eng._cus = 256
     eng._enqueue, eng._used, eng._used_end = threading.RLock(), None, None
     eng._used_handle, eng._late = -1, types.SimpleNamespace(value=0)
 

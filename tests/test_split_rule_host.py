@@ -41,3 +41,14 @@ def test_one_rule_without_stored_rounds(tmp_path):
 def test_repository_rule():
     from mpsim_amd import tune
     assert tune.tuned_rounds() == (2, 512)
+
+
+@pytest.mark.parametrize("rows,fills", [([512] * 40, False), ([1024] * 3, False), ([1024] * 4, True), ([513] * 7, False),
+                                        ([513] * 8, True), ([1040] * 9, False), ([1024, 1000, 900, 64], False)])
+def test_calls_that_fill_the_device_stay_whole(rows, fills):
+    """Groups of a workgroup for 16 rows, of problems of 513 to 1024 rows, on 256
+    compute units."""
+    from mpsim_amd.engine import Engine
+    eng = Engine.__new__(Engine)
+    eng._cus = 256
+    assert eng._fills(rows) == fills

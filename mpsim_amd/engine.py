@@ -409,8 +409,9 @@ class Engine:
         """Whether the direct solver's groups for the problems of more than 512 rows (a
         workgroup, on a compute unit of its own, for every 16 rows) fill the device:
         one launch is then the fastest (8 of 1024 rows 17.6 ms, 19 to 23 in four
-        launches; 11 of 900 21.4 and 26)."""
-        return sum(-(-r // 16) for r in rows if 512 < r <= 1024) >= self._cus
+        launches; 11 of 900 21.4 and 26). Not beside larger problems, whose rounds the
+        other launches fill (5 of 1024 and 3 of 1200 rows: 73 ms, 69 in four)."""
+        return max(rows) <= 1024 and sum(-(-r // 16) for r in rows if r > 512) >= self._cus
 
     def _two_site(self, items: Sequence[TwoSiteItem], svd: Optional[SvdConfig], cur, stream: int
                   ) -> List[TwoSiteResult]:

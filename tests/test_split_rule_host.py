@@ -44,7 +44,7 @@ def test_repository_rule():
 
 
 @pytest.mark.parametrize("rows,fills", [([512] * 40, False), ([1024] * 3, False), ([1024] * 4, True), ([513] * 7, False),
-                                        ([513] * 8, True), ([1040] * 9, False), ([1024, 1000, 900, 64], False)])
+                                        ([513] * 8, True), ([1040] * 9, False), ([1024] * 5 + [1040], False), ([1024, 1000, 900, 64], False)])
 def test_calls_that_fill_the_device_stay_whole(rows, fills):
     """Groups of a workgroup for 16 rows, of problems of 513 to 1024 rows, on 256
     compute units."""
